@@ -2,7 +2,8 @@
 //
 // Queries (rendering/_raycaster.py:35-36, Raycaster.ray_cast — a stub in the reference):
 //   k_query (closest or any hit): each lane walks its own ray with its own LDS stack (rays may be
-//   incoherent) and takes the next ray of its wave's chunk when its walk ends; rays and hits are
+//   incoherent) and takes the next ray of its wave's chunk when its walk ends; k_query_group: 16 or
+//   64 lanes walk one ray together, for buffers of few rays. Rays and hits are
 //   read/written through (pointer, byte stride) fields, so SoA (stride 4) and the AoS Ray/Hit
 //   records are both accepted.
 // Camera rays:
@@ -109,6 +110,19 @@ __global__ void __launch_bounds__(256) k_query(SceneArgs sc, rt_rays rays, uint3
         [&](bool fin, uint32_t i, const Ray& r, Hit& h) {
             if (fin) finish_query<ANY>(sc, hits, occluded, i, r, h);
         });
+}
+
+// Queries of few rays: one ray per group of G lanes, one wave per workgroup (group_walk).
+template <bool ANY, int G>
+__global__ void __launch_bounds__(64) k_query_group(SceneArgs sc, rt_rays rays, uint32_t n, rt_hits hits,
+                                                    uint8_t* occluded) {
+    __shared__ int32_t stk[kGroupWords];
+    const uint32_t i = refill_slot(blockIdx.x, 0, 1, gridDim.x) * (64u / G) + threadIdx.x / G;
+    const bool want = i < n;
+    const Ray r = query_ray(rays, i, want);
+    Hit h;
+    group_walk<ANY, G>(sc.nodes4, sc.tris, sc.root, r, want, -1, h, stk);
+    if (want && (threadIdx.x & (G - 1)) == 0) finish_query<ANY>(sc, hits, occluded, i, r, h);
 }
 
 __global__ void __launch_bounds__(256) k_generate_rays(rt_camera cam, uint32_t W, uint32_t H,
@@ -945,6 +959,32 @@ uint32_t query_blocks(const void* kern, int variant, uint32_t lane_stack, uint64
     return (uint32_t)((w + 3) / 4);
 }
 
+// Lanes per ray of a query of n rays: 64 or 16 (k_query_group), or 0 for the one-lane walks with
+// refill (k_query). The one-lane walks take as long as their slowest rays whatever n is; groups
+// shorten that chain but cost more per ray (us, closest / any hit of random rays and segments, one
+// lane : 16 : 64 lanes):
+//   triangles   1,000 rays                 16,384 rays                65,536 rays                 131,072 rays
+//   1.3 k       54/53 : 12/9 : 10/7        62/50 : 17/13 : 30/20      62/52 : 44/34 : 91/61       66/55 : 80/57 : 184/115
+//   50 k        107/83 : 26/17 : 18/9      121/89 : 35/23 : 40/28     123/91 : 84/60 : 128/90     132/106 : 142/107 : 244/172
+//   251 k       194/159 : 48/27 : 23/12    238/194 : 70/53 : 58/43    249/220 : 156/105 : 168/116 262/222 : 254/179 : 314/219
+//   1.3 M       573/355 : 99/53 : 42/21    664/469 : 192/116 : 98/68  639/459 : 347/249 : 264/183 649/463 : 533/444 : 477/348
+// so groups serve up to 65,536 rays, twice that in scenes of 250,000 triangles, and whole waves the
+// fewer rays the smaller (shallower) the scene. A caller that bounds the lane stacks, or asks for
+// the binary nodes, gets the walk that has them.
+int query_group(const rt_tuning& tu, uint32_t n, uint32_t n_tris) {
+    if (tu.query != RT_TRAVERSAL_LANE || tu.lane_stack != RT_LANE_STACK_MAX) return 0;
+    if (n > (n_tris >= 250000u ? 131072u : 65536u)) return 0;
+    return n <= std::max(4096u, n_tris / 8u) ? 64 : 16;
+}
+
+template <bool ANY>
+void launch_query_group(int g, const rt_scene* scene, const rt_rays& rays, uint32_t n, const rt_hits& hits,
+                        uint8_t* occluded, hipStream_t s) {
+    const auto k = g == 64 ? k_query_group<ANY, 64> : k_query_group<ANY, 16>;
+    hipLaunchKernelGGL(k, dim3(blocks_for(n, 64u / (uint32_t)g)), dim3(64), 0, s, scene_args(scene), rays, n, hits,
+                       occluded);
+}
+
 }  // namespace
 }  // namespace rt
 
@@ -960,6 +1000,10 @@ extern "C" int rt_trace_closest(const rt_scene* scene, const rt_rays* rays, uint
     rt_tuning tu;
     if ((e = resolve_tuning(tuning, tu, "rt_trace_closest"))) return e;
     if (n == 0) return RT_OK;
+    if (const int g = query_group(tu, n, scene->n_tris)) {
+        launch_query_group<false>(g, scene, *rays, n, *hits, nullptr, (hipStream_t)stream);
+        return check_launch("rt_trace_closest");
+    }
     const size_t lds = 4u * 256u * tu.lane_stack;
     auto k = tu.query == RT_TRAVERSAL_LANE ? k_query<false, RT_TRAVERSAL_LANE>
                                            : k_query<false, RT_TRAVERSAL_BINARY>;
@@ -978,6 +1022,10 @@ extern "C" int rt_trace_any(const rt_scene* scene, const rt_rays* rays, uint32_t
     rt_tuning tu;
     if ((e = resolve_tuning(tuning, tu, "rt_trace_any"))) return e;
     if (n == 0) return RT_OK;
+    if (const int g = query_group(tu, n, scene->n_tris)) {
+        launch_query_group<true>(g, scene, *rays, n, rt_hits{}, occluded, (hipStream_t)stream);
+        return check_launch("rt_trace_any");
+    }
     const size_t lds = 4u * 256u * tu.lane_stack;
     auto k = tu.query == RT_TRAVERSAL_LANE ? k_query<true, RT_TRAVERSAL_LANE>
                                            : k_query<true, RT_TRAVERSAL_BINARY>;

@@ -229,6 +229,139 @@ RT_DEV bool wave_walk(const float4* __restrict__ nodes4, const float4* __restric
     return true;
 }
 
+// ---- one ray per group of lanes ----
+// Each group of G lanes (16 or 64) walks one ray over the 4-wide nodes: a step takes up to G/4
+// entries from the top of the group's LDS stack, lane 4e+c tests child c of entry e against the
+// ray's best t, the entered internal children are pushed (ballot compaction within the group; for
+// closest hits an entry's nearer children above its farther ones, which halves the time) and each
+// entered leaf is tested by its lane; the group's closest candidate (t, then the smaller primitive)
+// is reduced after a step that found one. The closest hit does not depend on the visiting order, so
+// h is the one-lane walk's hit: a box is skipped only where it is entered 2^-18 past the best hit,
+// more than the rounding of an entry distance, which the boxes' padding covers only where the
+// coordinates are not much smaller than the distance. The stack never overflows: above kSwitch entries a step takes one
+// entry, so the walk goes on depth first, whose at most 31 levels push at most 3 each.
+// What bounds a walk of few rays is the chain of dependent steps of its slowest ray (up to 600
+// nodes of one lane): a step costs about the same with 1 entry as with 16, so a group shortens the
+// chain to the depth of the tree plus the nodes / entries left over.
+// `stk`: the wave's kGroupWords words of LDS; `want` is the same in the lanes of a group; h comes
+// back in all of them. Called by all 64 lanes.
+constexpr int kGroupWords = 1024;
+
+// The closest (t, then the smaller primitive; p < 0: none) of a group's lanes, in all of them: row
+// rotations within 16 lanes, then exchanges between the rows.
+template <int G>
+RT_DEV void group_closest(float& t, int32_t& p) {
+    auto merge = [&](float ot, int32_t op) {
+        const bool take = op >= 0 && (p < 0 || ot < t || (ot == t && op < p));
+        t = take ? ot : t;
+        p = take ? op : p;
+    };
+#define RT_ROW_ROR(v, n) __builtin_amdgcn_update_dpp(0, v, 0x120 + (n), 0xF, 0xF, false)
+    merge(__int_as_float(RT_ROW_ROR(__float_as_int(t), 8)), RT_ROW_ROR(p, 8));
+    merge(__int_as_float(RT_ROW_ROR(__float_as_int(t), 4)), RT_ROW_ROR(p, 4));
+    merge(__int_as_float(RT_ROW_ROR(__float_as_int(t), 2)), RT_ROW_ROR(p, 2));
+    merge(__int_as_float(RT_ROW_ROR(__float_as_int(t), 1)), RT_ROW_ROR(p, 1));
+#undef RT_ROW_ROR
+    if (G == 64) {
+        merge(__shfl_xor(t, 16), __shfl_xor(p, 16));
+        merge(__shfl_xor(t, 32), __shfl_xor(p, 32));
+    }
+}
+
+template <bool ANY, int G>
+RT_DEV void group_walk(const float4* __restrict__ nodes4, const float4* __restrict__ tris, int32_t root,
+                       const Ray& r, bool want, int32_t skip_slot, Hit& h, int32_t* stk) {
+    static_assert(G == 16 || G == 64, "lanes per ray");
+    constexpr uint32_t E = G / 4, kCap = kGroupWords * G / 64, kSwitch = kCap - 3 * E - 93;
+    const uint32_t lane = __lane_id(), gl = lane & (G - 1u), c = lane & 3u, entry = gl >> 2;
+    const uint64_t gm = G == 64 ? ~0ull : (((1ull << (G & 63)) - 1ull) << (lane & ~(G - 1u)));
+    h.t = r.tmax;
+    h.u = h.v = 0.0f;
+    h.prim = h.slot = -1;
+    if (root == RT_EMPTY_ROOT) return;
+    float bt = r.tmax;  // the group's best; h is this lane's own until the end
+    int32_t bp = -1;
+    float cull = r.tmax;  // boxes entered past this are skipped
+    if (root < 0) {  // the whole tree is one leaf
+        test_leaf(tris, root, r, want && gl == 0, skip_slot, h);
+    } else {
+        int32_t* st = stk + (lane / G) * kCap;
+        const float idx = safe_inv(r.dx), idy = safe_inv(r.dy), idz = safe_inv(r.dz);
+        const float oxx = r.ox * idx, oyy = r.oy * idy, ozz = r.oz * idz;
+        uint32_t sp = want ? 1u : 0u;
+        if (want && gl == 0) st[0] = root;
+        while (__ballot(sp != 0) != 0) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const uint32_t k = sp > kSwitch ? 1u : sp < E ? sp : E, base = sp - k;
+            const int32_t node = entry < k ? st[base + entry] : RT_EMPTY_ROOT;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            bool push = false, leaf = false;
+            int32_t cref = RT_EMPTY_ROOT;
+            float key = INFINITY;
+            if (node != RT_EMPTY_ROOT) {
+                const float* nf = (const float*)(nodes4 + (size_t)node * 8);
+                const float clx = nf[c], chx = nf[4 + c], cly = nf[8 + c], chy = nf[12 + c], clz = nf[16 + c],
+                            chz = nf[20 + c];
+                cref = __float_as_int(nf[24 + c]);
+                const float x0 = fmaf(clx, idx, -oxx), x1 = fmaf(chx, idx, -oxx);
+                const float y0 = fmaf(cly, idy, -oyy), y1 = fmaf(chy, idy, -oyy);
+                const float z0 = fmaf(clz, idz, -ozz), z1 = fmaf(chz, idz, -ozz);
+                const float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), r.tmin));
+                const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fmaxf(z0, z1)) * kTfarScale;
+                const bool hk = (cref != RT_EMPTY_ROOT) & (tn <= fminf(tf, cull));
+                push = hk & (cref >= 0);
+                leaf = hk & (cref < 0);
+                key = push ? tn : INFINITY;
+            }
+            const uint64_t pm = __ballot(push) & gm;
+            if (ANY) {
+                if (push) st[base + lane_rank(pm)] = cref;
+            } else {
+                // nearer children higher: each entry's farthest (rank 3) first, its nearest (0) last
+                // (key of the entry's other three children by quad permutations; ties in lane order)
+                const float k1 = __int_as_float(dpp_xor1(__float_as_int(key)));
+                const float k2 = __int_as_float(dpp_xor2(__float_as_int(key)));
+                const float k3 = __int_as_float(dpp_xor1(__float_as_int(k2)));
+                const int rank = (k1 < key) + (k2 < key) + (k3 < key);
+                const uint64_t m3 = __ballot(push && rank == 3) & gm, m2 = __ballot(push && rank == 2) & gm,
+                               m1 = __ballot(push && rank == 1) & gm, m0 = pm & ~(m1 | m2 | m3);
+                const uint32_t at2 = (uint32_t)__popcll(m3), at1 = at2 + (uint32_t)__popcll(m2),
+                               at0 = at1 + (uint32_t)__popcll(m1);
+                const uint64_t mine = rank == 0 ? m0 : rank == 1 ? m1 : rank == 2 ? m2 : m3;
+                const uint32_t at = rank == 0 ? at0 : rank == 1 ? at1 : rank == 2 ? at2 : 0u;
+                if (push) st[base + at + lane_rank(mine)] = cref;
+            }
+            sp = base + (uint32_t)__popcll(pm);
+            if (__ballot(leaf)) {
+                bool found = false;
+                if (leaf) found = test_leaf(tris, cref, r, true, skip_slot, h);
+                if (__ballot(found)) {
+                    bt = h.t;
+                    bp = h.prim;
+                    group_closest<G>(bt, bp);
+                    if (ANY && bp >= 0) sp = 0;
+                    if (bp >= 0) cull = fmaf(fabsf(bt), 0x1p-18f, bt);
+                }
+            }
+        }
+    }
+    bt = h.t;
+    bp = h.prim;
+    group_closest<G>(bt, bp);
+    // the lane that holds the winner hands it to its group
+    const uint64_t win = __ballot(bp >= 0 && h.prim == bp && h.t == bt) & gm;
+    const int wl = win ? __ffsll((unsigned long long)win) - 1 : (int)lane;
+    h.t = bt;
+    h.prim = bp;
+    h.u = __shfl(h.u, wl);
+    h.v = __shfl(h.v, wl);
+    h.slot = __shfl(h.slot, wl);
+}
+
 template <bool ANY, int MODE, int PARK, bool NF = false, bool COOP = true, typename Load, typename Finish>
 RT_DEV void refill_walks(const SceneArgs& sc, uint64_t n, uint32_t n_waves, uint32_t wid, int32_t* stk,
                          int stk_stride, int lane_stack, uint32_t* list, float4* pk, Load&& load,
