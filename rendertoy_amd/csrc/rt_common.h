@@ -119,21 +119,31 @@ RT_DEV void refine_hit(const float4* __restrict__ tris, const Ray& r, Hit& h) {
 }
 
 // Tests the triangles of leaf `ref` in slot order against r, updating h (closest hit; ties to the
-// smaller primitive id). Every record of the leaf is fetched before the first test (slots past the
-// leaf's count re-read its first record), so a leaf costs one memory round trip instead of one per
-// triangle. `active` = this lane takes part; `skip_slot` = a slot never reported (a shadow ray's
-// own triangle). Returns whether h changed.
+// smaller primitive id). Every record of the leaf is fetched before the first test, so a leaf costs
+// one memory round trip instead of one per triangle. `active` = this lane takes part; `skip_slot` =
+// a slot never reported (a shadow ray's own triangle). Returns whether h changed.
+// MASK: slots past the leaf's count are not fetched; else they re-read its first record. A load
+// costs the CU's address and tag units one access per lane that takes part, wherever it points, and
+// in the ray-buffer walks those units are the busiest (74% of a 2 M segment query's cycles, against
+// 56% for the vector ALUs): leaves hold 2.9 triangles on average, so a third of the accesses of a
+// full fetch are for nothing. Masked, 2 M segments through 251 k triangles take 1.05 ms instead of
+// 1.18, 1.5 M random rays through 1.3 M 2.49 instead of 2.59, a 3-sphere path frame 3.90 instead of
+// 4.03. The batch refill kernel, bound by its slowest walks, loses 3% to the extra branches.
+template <bool MASK = false>
 RT_DEV bool test_leaf(const float4* __restrict__ tris, int32_t ref, const Ray& r, bool active,
                       int32_t skip_slot, Hit& h) {
     const uint32_t first = leaf_first(ref), count = leaf_count(ref);
     float4 a[kLeafMax], b[kLeafMax], c[kLeafMax];
 #pragma unroll
     for (int k = 0; k < kLeafMax; ++k) {
-        const float4* tr = tris + (size_t)(first + ((uint32_t)k < count ? (uint32_t)k : 0u)) * 3;
-        a[k] = tr[0];
-        b[k] = tr[1];
-        c[k] = tr[2];
+        if (!MASK || (uint32_t)k < count) {
+            const float4* tr = tris + (size_t)(first + ((uint32_t)k < count ? (uint32_t)k : 0u)) * 3;
+            a[k] = tr[0];
+            b[k] = tr[1];
+            c[k] = tr[2];
+        }
     }
+    if (MASK) __builtin_amdgcn_sched_barrier(0);  // the fetches stay ahead of the tests
     bool changed = false;
 #pragma unroll
     for (int k = 0; k < kLeafMax; ++k) {
@@ -184,7 +194,7 @@ enum { kWalkOn = 0, kWalkDone = 1, kWalkOverflow = 2 };
 // At most `steps` iterations (one node or one leaf each) of the binary walk from state w:
 // kWalkDone when the walk has ended (h final), kWalkOverflow when a push would exceed `limit`
 // entries (h invalid), else kWalkOn (w and h hold the walk so far).
-template <bool ANY>
+template <bool ANY, bool MASK = false>
 RT_DEV int bin_steps(const float4* __restrict__ nodes, const float4* __restrict__ tris, const Ray& r,
                      int32_t skip_slot, Hit& h, LaneWalk& w, int32_t* stk, int stride, int limit,
                      int steps) {
@@ -217,7 +227,7 @@ RT_DEV int bin_steps(const float4* __restrict__ nodes, const float4* __restrict_
                 continue;
             }
         } else {
-            if (test_leaf(tris, w.cur, r, true, skip_slot, h) && ANY) return kWalkDone;
+            if (test_leaf<MASK>(tris, w.cur, r, true, skip_slot, h) && ANY) return kWalkDone;
         }
         if (w.sp == 0) return kWalkDone;
         w.cur = stk[(--w.sp) * stride];
@@ -821,7 +831,7 @@ RT_DEV int lane4_children(const float4* __restrict__ nodes4, int32_t cur, const 
 // round for all parked leaves (speculative traversal, Aila & Laine 2009). The closest hit does not
 // depend on the visiting order (a node is skipped only past the best hit so far, which a later leaf
 // can only lower), so the hits are those of the one-node-or-leaf walk. Parking costs ~3 VGPRs.
-template <bool ANY, int PARK = RT_PARK_RENDER, bool NF = false>
+template <bool ANY, int PARK = RT_PARK_RENDER, bool NF = false, bool MASK = false>
 RT_DEV int lane4_steps(const float4* __restrict__ nodes4, const float4* __restrict__ tris, const Ray& r,
                        int32_t skip_slot, Hit& h, LaneWalk& w, int32_t* stk, int stride, int limit,
                        int steps, bool any_rt = false) {
@@ -849,7 +859,7 @@ RT_DEV int lane4_steps(const float4* __restrict__ nodes4, const float4* __restri
             const uint64_t nodes = __ballot(w.cur >= 0 && w.cur != RT_EMPTY_ROOT);
             if (parked != 0 && (nodes == 0 || 4 * __popcll(parked) >= PARK * __popcll(__ballot(true)))) {
                 if (w.leaf != RT_EMPTY_ROOT) {
-                    const bool changed = test_leaf(tris, w.leaf, r, true, skip_slot, h);
+                    const bool changed = test_leaf<MASK>(tris, w.leaf, r, true, skip_slot, h);
                     w.leaf = RT_EMPTY_ROOT;
                     if (changed && (ANY || any_rt)) return kWalkDone;
                 }
@@ -868,7 +878,7 @@ RT_DEV int lane4_steps(const float4* __restrict__ nodes4, const float4* __restri
                     continue;
                 }
             } else {
-                if (test_leaf(tris, w.cur, r, true, skip_slot, h) && (ANY || any_rt)) return kWalkDone;
+                if (test_leaf<MASK>(tris, w.cur, r, true, skip_slot, h) && (ANY || any_rt)) return kWalkDone;
             }
             if (w.sp == 0) return kWalkDone;
             w.cur = stk[(--w.sp) * stride];

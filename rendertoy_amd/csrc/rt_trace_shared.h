@@ -413,9 +413,9 @@ RT_DEV void refill_walks(const SceneArgs& sc, uint64_t n, uint32_t n_waves, uint
                 if (sc.root == RT_EMPTY_ROOT)
                     st = kWalkDone;
                 else if (MODE == RT_TRAVERSAL_BINARY)
-                    st = bin_steps<ANY>(sc.nodes, sc.tris, r, skip, h, w, stk, stk_stride, lane_stack, kRefillSteps);
+                    st = bin_steps<ANY, true>(sc.nodes, sc.tris, r, skip, h, w, stk, stk_stride, lane_stack, kRefillSteps);
                 else
-                    st = lane4_steps<ANY, PARK, NF>(sc.nodes4, sc.tris, r, skip, h, w, stk, stk_stride, lane_stack,
+                    st = lane4_steps<ANY, PARK, NF, true>(sc.nodes4, sc.tris, r, skip, h, w, stk, stk_stride, lane_stack,
                                           kRefillSteps);
             }
             finish(st == kWalkDone, ri, r, h);
