@@ -30,6 +30,10 @@ RT_DEV void st(T* base, uint64_t i, uint32_t stride, T v) {
     if (base) *(T*)((char*)base + i * stride) = v;
 }
 
+__global__ void k_zero_u32(uint32_t* c, uint32_t n) {
+    if (threadIdx.x < n) c[threadIdx.x] = 0;
+}
+
 RT_DEV int32_t mesh_of_prim(const int32_t* __restrict__ offs, uint32_t n_meshes, int32_t prim) {
     // largest m with offs[m] <= prim (empty meshes share offsets: take the last such m)
     uint32_t lo = 0, hi = n_meshes;  // answer in [lo, hi)
@@ -254,6 +258,60 @@ __global__ void __launch_bounds__(64) k_trace_camera_quad(SceneArgs sc, rt_camer
     }
 }
 
+// Pixel of this lane's group of G lanes in a one-wave workgroup: the wave's 64 / G pixels (2x2, or
+// one) lie in 8x8-pixel block (j / waves per block) * 8 + x of XCD x's j-th workgroup, row-major, so
+// the waves of a block are consecutive on one XCD (k_trace_camera_quad's mapping).
+template <int G>
+RT_DEV TilePixel group_pixel(uint32_t W, uint32_t H, uint32_t tiles_x8) {
+    constexpr uint32_t side = G == 16 ? 2 : 1, across = 8 / side, waves = across * across;
+    const uint32_t xcd = blockIdx.x & 7u, j = blockIdx.x >> 3, w = j % waves, blk = (j / waves) * 8u + xcd;
+    const uint32_t g = threadIdx.x / G;
+    TilePixel p;
+    p.col = (blk % tiles_x8) * 8u + (w % across) * side + (g % side);
+    p.row = (blk / tiles_x8) * 8u + (w / across) * side + (g / side);
+    p.valid = p.col < W && p.row < H;
+    return p;
+}
+
+// Workgroups of a group kernel over a W x H image.
+uint32_t group_blocks(int g, uint32_t W, uint32_t H) {
+    const uint32_t blocks8 = ((W + 7u) / 8u) * ((H + 7u) / 8u);
+    return 8u * ((blocks8 + 7u) / 8u) * (uint32_t)g;
+}
+
+// Lanes per pixel of an image of n pixels: 64 or 16 (group_walk), or 0 for the quad-lane packets.
+// Packets share their node fetches, but a frame takes at least as long as its slowest packet's chain
+// of steps, the longer the denser the scene and the fewer the pixels; groups shorten the chain and
+// cost more per pixel (us, mean of three views, quads : 16 : 64 lanes, camera / render):
+//   triangles  64x64                          256x256                       768x512
+//   1.3 k      26/39 : 12/16 : 11/16          20/33 : 26/37 : 74/106        31/54 : 114/163 : 398/575
+//   11.5 k     77/105 : 19/24 : 13/18         42/64 : 32/44 : 76/107        49/80 : 119/167 : 400/559
+//   50 k       197/236 : 32/38 : 18/22        103/129 : 49/60 : 84/119      92/132 : 138/201 : 435/615
+//   251 k      546/627 : 59/70 : 26/32        265/332 : 82/100 : 97/141     221/295 : 175/280 : 472/678
+//   1.3 M      2160/2483 : 168/198 : 64/71    928/1225 : 202/243 : 132/191  720/951 : 340/480 : 556/811
+// The 16-lane groups are faster up to about 900 sqrt(triangles) pixels (1.3 M at 1024x768: 558
+// against 688 us, at 1600x900 831 against 735), whole waves up to 4,096 pixels or, where the tree is
+// deeper, a sixth of the triangles.
+int image_group(uint64_t n, uint32_t n_tris) {
+    if (n * n > 810000ull * n_tris) return 0;
+    return n <= std::max(4096u, std::min(n_tris / 6u, 65536u)) ? 64 : 16;
+}
+
+// Camera closest hit of a small image, G lanes per pixel (image_group).
+template <int G>
+__global__ void __launch_bounds__(64) k_trace_camera_group(SceneArgs sc, rt_camera cam, uint32_t W, uint32_t H,
+                                                           uint32_t tiles_x8, rt_hits hits) {
+    __shared__ int32_t stk[kGroupWords];
+    const TilePixel p = group_pixel<G>(W, H, tiles_x8);
+    const Ray r = camera_ray(cam, W, H, p);
+    Hit h;
+    group_walk<false, G>(sc.nodes4, sc.tris, sc.root, r, p.valid, -1, h, stk);
+    if (p.valid && (threadIdx.x & (G - 1)) == 0) {
+        if (h.prim >= 0) refine_hit(sc.tris, r, h);
+        store_hit(sc, hits, (uint64_t)p.row * W + p.col, h);
+    }
+}
+
 RT_DEV int wrap_i(int i, int n) {
     const int r = i % n;
     return r < 0 ? r + n : r;
@@ -350,13 +408,18 @@ RT_DEV void render_pixel(const SceneArgs& sc, const rt_camera& cam, const rt_ren
                          int32_t* __restrict__ out_prim, uint32_t* __restrict__ stats, float4* pk,
                          int32_t* stk, int stk_stride, int lane_stack, int budget, bool coherent) {
     // PM == RT_TRAVERSAL_QUAD: quad layout (the 4 lanes of a quad hold the same pixel), both rays by
-    // the quad-lane traversal, outputs and counts from lane 0 of each quad
+    // the quad-lane traversal, outputs and counts from lane 0 of each quad; PM == 16 or 64: the same
+    // with groups of that many lanes and group_walk (its LDS stacks at `stk`)
     constexpr bool QL = PM == RT_TRAVERSAL_QUAD;
+    constexpr int G = PM >= 16 ? PM : 0;
+    constexpr uint32_t per_pixel = QL ? 4 : G ? G : 1;  // lanes that hold the same pixel
     const uint32_t W = p.width, H = p.height;
     const Ray r = camera_ray(cam, W, H, px);
     Hit h;
     if constexpr (QL) {
         traverse_quad<false>(sc.nodes4, sc.tris, sc.root, r, px.valid, -1, h);
+    } else if constexpr (G != 0) {
+        group_walk<false, G>(sc.nodes4, sc.tris, sc.root, r, px.valid, -1, h, stk);
     } else {
         trace_primary<PM>(sc, r, px.valid, h, pk, stk, stk_stride, lane_stack, budget, coherent);
     }
@@ -373,6 +436,8 @@ RT_DEV void render_pixel(const SceneArgs& sc, const rt_camera& cam, const rt_ren
     Hit sh;
     if constexpr (QL)
         traverse_quad<true>(sc.nodes4, sc.tris, sc.root, sr, want_shadow, hit ? h.slot : -1, sh);
+    else if constexpr (G != 0)
+        group_walk<true, G>(sc.nodes4, sc.tris, sc.root, sr, want_shadow, hit ? h.slot : -1, sh, stk);
     else
         trace_block<true, SM>(sc, sr, want_shadow, hit ? h.slot : -1, sh, pk, stk, stk_stride, lane_stack,
                               budget);
@@ -380,7 +445,7 @@ RT_DEV void render_pixel(const SceneArgs& sc, const rt_camera& cam, const rt_ren
 
     float alb[3] = {1.0f, 1.0f, 1.0f};
     if (hit) albedo(p, mesh, tu, tv, alb);
-    if (px.valid && (!QL || (threadIdx.x & 3) == 0)) {
+    if (px.valid && (threadIdx.x & (per_pixel - 1)) == 0) {
         const uint64_t pix = (uint64_t)px.row * W + px.col;
         if (hit) {
             const float kk = fmaf(occluded ? 0.0f : 1.0f, ndl, p.ambient);
@@ -396,7 +461,7 @@ RT_DEV void render_pixel(const SceneArgs& sc, const rt_camera& cam, const rt_ren
         if (out_prim) out_prim[pix] = hit ? h.prim : -1;
     }
     if (stats) {
-        const uint64_t one = QL ? kQuadBits : ~0ull;  // one lane per pixel
+        const uint64_t one = QL ? kQuadBits : G == 16 ? 0x0001000100010001ull : G == 64 ? 1ull : ~0ull;  // one lane per pixel
         const uint32_t n_hit = (uint32_t)__popcll(__ballot(hit) & one);
         const uint32_t n_sh = (uint32_t)__popcll(__ballot(want_shadow) & one);
         const uint32_t n_oc = (uint32_t)__popcll(__ballot(occluded) & one);
@@ -484,6 +549,17 @@ __global__ void __launch_bounds__(W1 ? 64 : 256) k_render_quad(SceneArgs sc, rt_
                                                            stats ? bstat : nullptr, nullptr, nullptr, 0, 0, 0, true);
         block_stats_end(stats, bstat);
     }
+}
+
+// Fused render of a small image, G lanes per pixel (image_group); counts as in k_render_quad<true>.
+template <int G>
+__global__ void __launch_bounds__(64) k_render_group(SceneArgs sc, rt_camera cam, rt_render_params p, uint32_t tiles_x8,
+                                                     float* __restrict__ rgb, float* __restrict__ out_t,
+                                                     int32_t* __restrict__ out_prim, uint32_t* __restrict__ stats) {
+    __shared__ int32_t stk[kGroupWords];
+    const TilePixel px = group_pixel<G>(p.width, p.height, tiles_x8);
+    uint32_t* slot = stats ? stats + (blockIdx.x % kCountSlots) * kCountStride : nullptr;
+    render_pixel<G, G>(sc, cam, p, px, rgb, out_t, out_prim, slot, nullptr, stk, 0, 0, 0, true);
 }
 
 // ---- batched render ----
@@ -904,10 +980,6 @@ __global__ void __launch_bounds__(64) k_render_batch_refill(const rt_render_job*
     flush();
 }
 
-__global__ void k_zero_u32(uint32_t* c, uint32_t n) {
-    if (threadIdx.x < n) c[threadIdx.x] = 0;
-}
-
 __global__ void k_zero_words(uint32_t* w, uint32_t n) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) w[i] = 0;
 }
@@ -1069,8 +1141,15 @@ extern "C" int rt_trace_camera(const rt_scene* scene, const rt_camera* cam, uint
     rt_tuning tu;
     if ((e = resolve_tuning(tuning, tu, "rt_trace_camera"))) return e;
     hipStream_t s = (hipStream_t)stream;
-    if (tu.primary == RT_TRAVERSAL_QUAD) {  // 8x8-pixel blocks
-        const TileMap tm8 = make_tile_map(W, H, tu.super_tile, 8);
+    if (tu.primary == RT_TRAVERSAL_QUAD) {
+        const int g = tu.super_tile ? 0 : image_group(n, scene->n_tris);
+        if (g) {
+            const auto k = g == 64 ? k_trace_camera_group<64> : k_trace_camera_group<16>;
+            hipLaunchKernelGGL(k, dim3(group_blocks(g, W, H)), dim3(64), 0, s, scene_args(scene), *cam, W, H,
+                               (W + 7u) / 8u, *hits);
+            return check_launch("rt_trace_camera");
+        }
+        const TileMap tm8 = make_tile_map(W, H, tu.super_tile, 8);  // 8x8-pixel blocks
         hipLaunchKernelGGL(k_trace_camera_quad, dim3(32u * ((tile_map_blocks(tm8) + 7u) / 8u)), dim3(64), 0, s,
                            scene_args(scene), *cam, W, H, tm8, *hits);
         return check_launch("rt_trace_camera");
@@ -1122,8 +1201,14 @@ extern "C" int rt_render(const rt_scene* scene, const rt_camera* cam, const rt_r
         } else {
             uint32_t* part = partial ? (uint32_t*)workspace : nullptr;
             if (part) hipLaunchKernelGGL(k_zero_words, dim3(8), dim3(256), 0, s, part, kCountSlots * kCountStride);
-            hipLaunchKernelGGL(k_render_quad<true>, dim3(32u * ((tx8 * ty8 + 7u) / 8u)), dim3(64), 0, s,
-                               scene_args(scene), *cam, *p, tx8, out->rgb, out->t, out->prim, part);
+            if (const int g = image_group(n, scene->n_tris)) {
+                const auto k = g == 64 ? k_render_group<64> : k_render_group<16>;
+                hipLaunchKernelGGL(k, dim3(group_blocks(g, p->width, p->height)), dim3(64), 0, s, scene_args(scene),
+                                   *cam, *p, tx8, out->rgb, out->t, out->prim, part);
+            } else {
+                hipLaunchKernelGGL(k_render_quad<true>, dim3(32u * ((tx8 * ty8 + 7u) / 8u)), dim3(64), 0, s,
+                                   scene_args(scene), *cam, *p, tx8, out->rgb, out->t, out->prim, part);
+            }
             if (part) hipLaunchKernelGGL(k_sum_counts, dim3(1), dim3(256), 0, s, part, out->stats);
         }
         return check_launch("rt_render");
