@@ -586,22 +586,69 @@ RT_DEV uint32_t job_tiles(const rt_render_job& j, uint32_t unit, uint32_t& statu
     return ((p.width + unit - 1u) / unit) * ((p.height + unit - 1u) / unit);
 }
 
+// The tile queue of k_render_batch_refill in the workspace bytes past the prefix, where the caller
+// gives them: kQueues counters, each on a 256-byte line of its own, then the order of the jobs.
+// Waves of one queue take every kQueues-th grab of tiles. One counter for all waves is the kernel's
+// bound once most tiles miss everything: it is read and written about 70 times a microsecond at
+// most, and 48 images of 128..768 pixels a side are 30,000 grabs of 4 tiles.
+constexpr uint32_t kQueues = 64, kQueueStride = 64;  // words
+
+struct BatchQueue {
+    uint32_t* counters;  // NULL: the one counter ws[0], jobs in table order
+    uint32_t* order;     // job of the p-th prefix entry
+};
+
+// A grab is the launch's unit of work at its end: a wave can hold one of its densest tiles (256 pixels
+// of 4 tiles take up to 1.5 ms). Smaller grabs cost more job changes, whose drains leave lanes idle:
+// with 1 : 2 : 4 tiles, 122,000 tiles in all take 1.44 : 1.24 : 1.55 ms, 30,000 tiles 0.64 : 0.84 :
+// 1.38 (0.55 : 0.76 : 1.14 over 3 scenes instead of 12).
+constexpr uint32_t kGrabsPerWave = 16;
+
+inline uint64_t batch_queue_offset(uint32_t n_jobs) { return (4ull * (kBatchPrefixWord + (uint64_t)n_jobs + 1) + 255) & ~255ull; }
+inline uint64_t batch_queue_bytes(uint32_t n_jobs) { return 4ull * (kQueues * kQueueStride + n_jobs); }
+
 // One block of 1024 threads: per-job tile counts, exclusive prefix (n_jobs <= 4096, at most 4 jobs
-// per thread), work counter and status cleared, every job's stats zeroed.
+// per thread), work counters and status cleared, every job's stats zeroed. With a queue, the jobs
+// are taken by the sizes of their scenes, largest first (a bitonic sort; jobs of equal sizes in
+// table order): the tiles of a dense scene take longest, and the launch ends with its last tile.
 __global__ void __launch_bounds__(1024) k_batch_prepare(const rt_render_job* __restrict__ jobs,
                                                          uint32_t n_jobs, uint32_t unit,
-                                                         uint32_t* __restrict__ ws) {
+                                                         uint32_t* __restrict__ ws, BatchQueue q) {
     __shared__ uint32_t part[1024];
     __shared__ uint32_t status;
+    __shared__ uint64_t keys[RT_BATCH_MAX_JOBS];
     const uint32_t t = threadIdx.x;
     if (t == 0) status = 0;
+    if (q.counters) {
+        uint32_t m = 1;
+        while (m < n_jobs) m <<= 1;
+        for (uint32_t j = t; j < m; j += 1024u)
+            keys[j] = j < n_jobs ? (uint64_t)(~jobs[j].scene.n_tris) << 32 | j : ~0ull;
+        for (uint32_t k = 2; k <= m; k <<= 1) {
+            for (uint32_t d = k >> 1; d > 0; d >>= 1) {
+                __syncthreads();
+                for (uint32_t i = t; i < m; i += 1024u) {
+                    const uint32_t x = i ^ d;
+                    if (x <= i) continue;
+                    const uint64_t a = keys[i], b = keys[x];
+                    if ((a > b) == ((i & k) == 0)) {
+                        keys[i] = b;
+                        keys[x] = a;
+                    }
+                }
+            }
+        }
+        if (t < kQueues) q.counters[t * kQueueStride] = 0;
+    }
     __syncthreads();
     uint32_t cnt[4], sum = 0, bad = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const uint32_t j = t * 4 + k;
+        const uint32_t p = t * 4 + k;
         cnt[k] = 0;
-        if (j < n_jobs) {
+        if (p < n_jobs) {
+            const uint32_t j = q.counters ? (uint32_t)keys[p] : p;
+            if (q.counters) q.order[p] = j;
             cnt[k] = job_tiles(jobs[j], unit, bad);
             uint32_t* st = as_global(jobs[j].out.stats);
             if (st) {
@@ -745,9 +792,9 @@ __global__ void __launch_bounds__(64) k_render_batch(const rt_render_job* __rest
 #endif
 constexpr int kRefillPasses = RT_REFILL_PASSES;  // refills per round while culled rays free lanes
 
-__global__ void __launch_bounds__(64) k_render_batch_refill(const rt_render_job* __restrict__ jobs,
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_render_batch_refill(const rt_render_job* __restrict__ jobs,
                                                              uint32_t n_jobs, uint32_t* __restrict__ ws,
-                                                             uint32_t grab, int lane_stack) {
+                                                             uint32_t grab, int lane_stack, BatchQueue queue) {
     extern __shared__ uint32_t smem[];
     __shared__ float4 pk[kPacketLds];
     uint32_t* pref = smem;
@@ -756,11 +803,17 @@ __global__ void __launch_bounds__(64) k_render_batch_refill(const rt_render_job*
     for (uint32_t j = lane; j <= n_jobs; j += 64) pref[j] = ws[kBatchPrefixWord + j];
     __syncthreads();
     const uint32_t total = pref[n_jobs];
+    if (queue.counters) {  // at least kGrabsPerWave grabs per wave where the caller's grab allows it
+        const uint32_t most = (total + gridDim.x * kGrabsPerWave - 1u) / (gridDim.x * kGrabsPerWave);
+        grab = grab < most ? grab : most;
+    }
 
     // wave-uniform: the tile being handed out, its next pixel, the end of the grabbed tiles, and
     // the job the lanes work on (with its scene, camera, parameters and counts)
     uint32_t tile = 0, tile_px = 64, pool_end = 0, job = 0xFFFFFFFFu, tile_job = 0;
     bool exhausted = false;
+    // XCD x (workgroups go to the 8 XCDs round robin) starts on queues x, x + 8, ...
+    uint32_t q = blockIdx.x % kQueues;
     SceneArgs sc{};
     rt_camera cam{};
     rt_render_params p{};
@@ -807,8 +860,24 @@ __global__ void __launch_bounds__(64) k_render_batch_refill(const rt_render_job*
             if (tile_px == 64u) {
                 if (++tile >= pool_end) {
                     uint32_t u0 = 0;
-                    if (lane == 0) u0 = atomicAdd(&ws[0], grab);
-                    u0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)u0);
+                    if (queue.counters) {
+                        // the next grab of the wave's queue; once that is empty, of the next one that
+                        // is not (the counters only grow, so every wave finds all of them empty)
+                        for (;;) {
+                            if (lane == 0) u0 = atomicAdd(&queue.counters[q * kQueueStride], 1u);
+                            u0 = ((uint32_t)__builtin_amdgcn_readfirstlane((int)u0) * kQueues + q) * grab;
+                            if (u0 < total) break;
+                            const uint32_t at = __hip_atomic_load(&queue.counters[lane * kQueueStride],
+                                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            const uint64_t open = __ballot((at * kQueues + lane) * grab < total);
+                            if (open == 0) break;
+                            const uint64_t after = open & ~((2ull << q) - 1ull);
+                            q = (uint32_t)__ffsll((unsigned long long)(after ? after : open)) - 1u;
+                        }
+                    } else {
+                        if (lane == 0) u0 = atomicAdd(&ws[0], grab);
+                        u0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)u0);
+                    }
                     if (u0 >= total) {
                         exhausted = true;
                     } else {
@@ -829,7 +898,7 @@ __global__ void __launch_bounds__(64) k_render_batch_refill(const rt_render_job*
             if (!exhausted && tile_job != job && n_idle == 64u) {  // drained: move to the tile's job
                 flush();
                 job = tile_job;
-                const rt_render_job& jb = jobs[job];
+                const rt_render_job& jb = jobs[queue.counters ? queue.order[job] : job];
                 sc = job_scene(jb);
                 cam = jb.cam;
                 p = job_params(jb);
@@ -1250,9 +1319,16 @@ int check_batch_args(const rt_render_job* jobs_dev, uint32_t n_jobs, const rt_ba
 // The two launches of a batch (prepare + persistent kernel) on `ws`, a workspace of
 // rt_render_batch_workspace_bytes(n_jobs) bytes whose every word the prepare kernel rewrites.
 int launch_batch(const rt_render_job* jobs_dev, uint32_t n_jobs, const rt_batch_config* cfg,
-                 uint32_t* ws, hipStream_t s, const char* what) {
+                 uint32_t* ws, uint64_t ws_bytes, hipStream_t s, const char* what) {
     const bool quad = cfg->primary == RT_TRAVERSAL_QUAD;
-    hipLaunchKernelGGL(k_batch_prepare, dim3(1), dim3(1024), 0, s, jobs_dev, n_jobs, quad ? 4u : 8u, ws);
+    const bool refill = cfg->primary == RT_TRAVERSAL_LANE && cfg->shadow == RT_TRAVERSAL_LANE;
+    BatchQueue queue{nullptr, nullptr};
+    const uint64_t at = batch_queue_offset(n_jobs);
+    if (refill && ws_bytes >= at + batch_queue_bytes(n_jobs)) {
+        queue.counters = ws + at / 4;
+        queue.order = queue.counters + kQueues * kQueueStride;
+    }
+    hipLaunchKernelGGL(k_batch_prepare, dim3(1), dim3(1024), 0, s, jobs_dev, n_jobs, quad ? 4u : 8u, ws, queue);
     const bool lds_stack = !quad && (cfg->primary != RT_TRAVERSAL_PACKET || cfg->shadow != RT_TRAVERSAL_PACKET);
     const size_t lds = 4u * ((n_jobs + 1 + 3) & ~3u) + (lds_stack ? 4u * 64u * kLaneStack : 0u);
     const uint32_t grid = (uint32_t)device_cu_count() * cfg->waves_per_cu;
@@ -1262,9 +1338,9 @@ int launch_batch(const rt_render_job* jobs_dev, uint32_t n_jobs, const rt_batch_
         {k_render_batch<1, 0>, k_render_batch<1, 1>, k_render_batch<1, 2>},
         {k_render_batch<2, 0>, k_render_batch<2, 1>, k_render_batch<2, 2>},
         {k_render_batch<3, 0>, k_render_batch<3, 1>, k_render_batch<3, 2>}};
-    if (cfg->primary == RT_TRAVERSAL_LANE && cfg->shadow == RT_TRAVERSAL_LANE) {
+    if (refill) {
         hipLaunchKernelGGL(k_render_batch_refill, dim3(grid), dim3(64), lds, s, jobs_dev, n_jobs, ws,
-                           cfg->tiles_per_grab, (int)cfg->lane_stack);
+                           cfg->tiles_per_grab, (int)cfg->lane_stack, queue);
         return check_launch(what);
     }
     const K kern = quad ? k_render_batch<RT_TRAVERSAL_QUAD, RT_TRAVERSAL_QUAD> : kerns[cfg->primary][cfg->shadow];
@@ -1284,7 +1360,7 @@ extern "C" int rt_render_batch(const rt_render_job* jobs_dev, uint32_t n_jobs, c
     if (!workspace || ws_bytes < rt_render_batch_workspace_bytes(n_jobs))
         return set_error(RT_EINVAL, "rt_render_batch: workspace too small");
     if ((uintptr_t)workspace & 15) return set_error(RT_EINVAL, "rt_render_batch: workspace must be 16-byte aligned");
-    return launch_batch(jobs_dev, n_jobs, cfg, (uint32_t*)workspace, (hipStream_t)stream, "rt_render_batch");
+    return launch_batch(jobs_dev, n_jobs, cfg, (uint32_t*)workspace, ws_bytes, (hipStream_t)stream, "rt_render_batch");
 }
 
 // ---- allocation-free batched render ----
@@ -1323,5 +1399,5 @@ extern "C" int rt_render_batch_static(const rt_render_job* jobs_dev, uint32_t n_
     if (n_jobs == 0) return RT_OK;
     uint32_t* ws = nullptr;
     if ((e = scratch_address(&ws, "rt_render_batch_static"))) return e;
-    return launch_batch(jobs_dev, n_jobs, cfg, ws, (hipStream_t)stream, "rt_render_batch_static");
+    return launch_batch(jobs_dev, n_jobs, cfg, ws, 4ull * kStaticBatchWords, (hipStream_t)stream, "rt_render_batch_static");
 }
