@@ -163,16 +163,19 @@ template <int PM>
 __global__ void __launch_bounds__(256) k_paths_primary(SceneArgs sc, rt_camera cam, PathArgs a,
                                                         uint32_t tiles_x, int lane_stack, int budget,
                                                         bool coherent) {
-    // PM == RT_TRAVERSAL_QUAD: quad layout, one wave per workgroup (wave j of XCD x takes the 4x4
+    // PM == RT_TRAVERSAL_QUAD: quad layout, one 4x4 quarter per workgroup (workgroup j of XCD x takes
     // quarter w = j & 3 of 8x8 block (j >> 2) * 8 + x, row-major, at ((w & 1) * 4, (w >> 1) * 4),
-    // lanes 4q..4q+3 its pixel (q & 3, q >> 2)); else a 256-thread block covers 16x16 pixels
+    // lanes 4q..4q+3 its pixel (q & 3, q >> 2)), with one wave for each of up to 4 samples at a time
+    // (one wave taking its pixels' 4 samples in turn made the frame wait for four slow packets in a
+    // row: 960x540 of 3 spheres of 251k triangles 1.33 ms, now 1.05); else a 256-thread block covers
+    // 16x16 pixels
     constexpr bool QL = PM == RT_TRAVERSAL_QUAD;
     __shared__ int32_t stk[(uses_lds(PM) && !QL) ? kLaneStack * 256 : 1];
     __shared__ float4 pk[QL ? 1 : 4][kPacketLds];
-    // QUAD: the bounce entries of up to 4 samples of the wave's 16 pixels, appended with one queue
-    // reservation (one same-address atomic per wave and sample took ~2 ms of a framed 4-spp frame)
+    // QUAD: the bounce entries of up to 4 samples of the workgroup's 16 pixels, appended with one
+    // queue reservation (one same-address atomic per sample took ~2 ms of a framed 4-spp frame)
     __shared__ float4 stage[QL ? 64 * 3 : 1];
-    uint32_t staged = 0;
+    __shared__ uint32_t s_count, s_base;
     const uint32_t lane = threadIdx.x & 63;
     uint32_t wave, blk;
     if constexpr (QL) {
@@ -191,7 +194,14 @@ __global__ void __launch_bounds__(256) k_paths_primary(SceneArgs sc, rt_camera c
     const bool lead = !QL || (lane & 3) == 0;  // the lane that writes for its pixel
     const bool valid = col < a.W && row < a.H;
     const uint32_t pixel = valid ? row * a.W + col : 0u;
-    for (uint32_t s = 0; s < a.spp; ++s) {
+    const uint32_t n_waves = QL ? blockDim.x >> 6 : 1u, swave = QL ? threadIdx.x >> 6 : 0u;
+    for (uint32_t s0 = 0; s0 < a.spp; s0 += n_waves) {
+        const uint32_t s = s0 + swave;
+        if (QL) {
+            if (threadIdx.x == 0) s_count = 0;
+            __syncthreads();
+        }
+        const bool live = valid && s < a.spp;
         const uint4 rnd = philox4x32_10(make_uint4(pixel, s, 0u, 0u), a.key0, a.key1);
         const float fx = (float)col + unit_float(rnd.x), fy = (float)row + unit_float(rnd.y);
         const float nx = fx / (float)a.W * 2.0f - 1.0f, ny = 1.0f - fy / (float)a.H * 2.0f;
@@ -213,41 +223,37 @@ __global__ void __launch_bounds__(256) k_paths_primary(SceneArgs sc, rt_camera c
             // leaf records in pairs: 94 VGPRs and 5 waves per SIMD instead of 111 and 4; the 4-spp
             // frames of the 2M-triangle cluster take 2.5% less time this way (the camera and render
             // kernels gain nothing from pairs on the C2 frame and lose 4% on C1, so they keep 4)
-            traverse_quad<false, 2>(sc.nodes4, sc.tris, sc.root, r, valid, -1, h);
+            traverse_quad<false, 2>(sc.nodes4, sc.tris, sc.root, r, live, -1, h);
         } else {
             trace_primary<PM>(sc, r, valid, h, pk[wave], stk + threadIdx.x, 256, lane_stack, budget,
                               coherent);
         }
-        const bool hit = valid && h.prim >= 0;
+        const bool hit = live && h.prim >= 0;
         if (hit) refine_hit(sc.tris, r, h);
         const uint32_t id = pixel * a.spp + s;
-        if (valid && lead) a.samples[id] = hit ? 0.0f : a.sky;
+        if (live && lead) a.samples[id] = hit ? 0.0f : a.sky;
         if (a.bounces > 0) {
             if constexpr (QL) {
                 const bool go = hit && lead;
                 float4 e0, e1, e2;
                 bounce_entry(sc, a, r, h, go, id, 1u, 1.0f, e0, e1, e2);
                 const uint64_t mask = __ballot(go);
+                uint32_t at = 0;
+                if (mask != 0 && lane == 0) at = atomicAdd(&s_count, (uint32_t)__popcll(mask));  // LDS
+                at = (uint32_t)__shfl((int)at, 0);
                 if (go) {
-                    const uint32_t j = (staged + mask_rank(mask)) * 3u;
+                    const uint32_t j = (at + mask_rank(mask)) * 3u;
                     stage[j] = e0;
                     stage[j + 1] = e1;
                     stage[j + 2] = e2;
                 }
-                staged += (uint32_t)__popcll(mask);
-                if ((s & 3u) == 3u || s + 1u == a.spp) {
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    uint32_t b = 0;
-                    if (staged && lane == 0) b = atomicAdd(&a.counts[1], staged);
-                    b = (uint32_t)__shfl((int)b, 0);
-                    for (uint32_t x = lane; x < staged * 3u; x += 64u) a.q[0][(size_t)b * 3 + x] = stage[x];
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    staged = 0;
-                }
+                __syncthreads();
+                const uint32_t staged = s_count;
+                if (threadIdx.x == 0 && staged) s_base = atomicAdd(&a.counts[1], staged);
+                __syncthreads();
+                for (uint32_t x = threadIdx.x; x < staged * 3u; x += blockDim.x)
+                    a.q[0][(size_t)s_base * 3 + x] = stage[x];
+                __syncthreads();  // before the next samples' count and entries
             } else {
                 emit_bounce(sc, a, r, h, hit && lead, id, 1u, 1.0f, a.q[0], &a.counts[1]);
             }
@@ -428,16 +434,18 @@ extern "C" int rt_trace_paths(const rt_scene* scene, const rt_camera* cam, const
                               k_paths_primary<3>};
     if (tu.primary == RT_TRAVERSAL_QUAD) {
         const uint32_t tx8 = (p->width + 7) / 8, ty8 = (p->height + 7) / 8;
-        hipLaunchKernelGGL(k_paths_primary<RT_TRAVERSAL_QUAD>, dim3(32u * ((tx8 * ty8 + 7u) / 8u)), dim3(64), 0, s,
-                           sc, *cam, a, tx8, (int)tu.lane_stack, (int)tu.packet_budget, coherent);
+        hipLaunchKernelGGL(k_paths_primary<RT_TRAVERSAL_QUAD>, dim3(32u * ((tx8 * ty8 + 7u) / 8u)),
+                           dim3(64u * std::min(p->spp, 4u)), 0, s, sc, *cam, a, tx8, (int)tu.lane_stack, (int)tu.packet_budget, coherent);
     } else {
         hipLaunchKernelGGL(prim[tu.primary], dim3(tiles_x * tiles_y), dim3(256), 0, s, sc, *cam, a,
                            tiles_x, (int)tu.lane_stack, (int)tu.packet_budget, coherent);
     }
+    // the emission's waves each take one same-address atomic (~14 ns): 4 workgroups per CU, 4,096 waves,
+    // emit 1 M bounces in 86 us, 16 per CU in 200
     const uint32_t grid = (uint32_t)device_cu_count() * 16u;
     for (uint32_t k = 1; k <= p->bounces; ++k) {
         hipLaunchKernelGGL(k_paths_bounce, dim3(grid), dim3(64), 0, s, sc, a, k, (int)tu.lane_stack);
-        hipLaunchKernelGGL(k_paths_emit, dim3(grid), dim3(256), 0, s, sc, a, k);
+        hipLaunchKernelGGL(k_paths_emit, dim3(grid / 4u), dim3(256), 0, s, sc, a, k);
     }
     const uint64_t px = (uint64_t)p->width * p->height;
     const uint32_t rb = (uint32_t)((std::max<uint64_t>(px, RT_PATHS_MAX_BOUNCES + 1) + 255) / 256);
