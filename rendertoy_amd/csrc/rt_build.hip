@@ -11,16 +11,12 @@
 //                  per-tile histogram -> per-digit row scan -> scatter, the scatter ranking keys
 //                  with wave64 ballot/mbcnt multi-split so equal digits keep input order and
 //                  writing each tile digit by digit from LDS.
-//   5. hierarchy   Karras 2012 binary radix tree over the extended keys (code, slot).
-//   6. emit        permute tri/shade records into slot order.
-//   7. refit       nodes whose leaf range lies inside one 1024-leaf block: bottom-up in that
-//                  block's workgroup (the second thread to reach a node unions its children's
-//                  boxes and continues upward, LDS counters). The ~0.6% spanning blocks: each
-//                  child box is the union of its slot range, from per-block prefix/suffix unions
-//                  and a sparse table over blocks (min/max are exact, so this equals the
-//                  bottom-up union), one thread per node with no waiting.
-//   8. wide        4-wide records from the binary ones.
-// PLOC (rt_tuning.builder) replaces 5-7 with locally ordered clustering over the same order.
+//   5. emit        permute tri/shade records into slot order.
+//   6. tree        Karras 2012 binary radix tree over the extended keys (code, slot), with its boxes:
+//                  bottom-up in LDS inside blocks of 1024 slots, then one wave per node that spans
+//                  blocks (min/max are exact, so range unions equal the bottom-up boxes).
+//   7. wide        4-wide records from the binary ones.
+// PLOC (rt_tuning.builder) replaces 5-6 with locally ordered clustering over the same order.
 // Every result is an integer or an exact FP32 min/max/sub, so the output is byte-identical to the
 // CPU restatement under the same inputs.
 #include <algorithm>
@@ -34,6 +30,30 @@ namespace rt {
 namespace {
 
 constexpr int kReduceBlocks = 512;
+
+// LBVH tree: slots per workgroup of the local pass, and the most top boundaries of one block
+constexpr int kTreeBlock = 1024;
+constexpr int kTopMax = 132;
+constexpr int kTopThreads = 512;
+
+// A top boundary: its position, its diff, the code of slot p, and the ends of its node's slots
+// [lo, hi1) where they lie in the boundary's block, else -1.
+struct alignas(16) TopEntry {
+    int32_t p, lo, hi1, diff;
+    uint32_t key;
+    int32_t pad[3];
+};
+
+// Global arrays of the top boundaries. By position P: pre[2 P] the box of [block start, P), suf[2 P]
+// that of [P, block end), child[4 P] and child[4 P + 2] the left and right child where it is a segment.
+struct TopArrays {
+    TopEntry* list;    // kTopMax per block
+    uint32_t* count;   // per block
+    float4* pre;
+    float4* suf;
+    float4* child;
+    float4* block;     // 2 per block: box of all its slots
+};
 
 struct Workspace {
     float4* cent;      // n
@@ -49,11 +69,6 @@ struct Workspace {
     float* partial;    // kReduceBlocks * 8
     float* cbounds;    // 8
     int32_t* parent;   // (n-1) internal then n leaves
-    int32_t* rangej;   // n-1: the other end j of internal node i's leaf range [min(i,j), max(i,j)]
-    int32_t* split;    // n-1: split position g of internal node i (children ranges [lo,g], [g+1,hi])
-    float4* nodebox;   // 2(n-1)
-    int32_t* top_list; // n-1: internal nodes whose leaf range spans several refit blocks
-    uint32_t* top_count;
     // PLOC builder
     int32_t* cid[2];   // n: cluster refs by position (internal id, or ~prim), ping-pong
     float4* cbox[2];   // 2n: cluster boxes by position, ping-pong
@@ -68,27 +83,12 @@ struct Workspace {
     uint32_t* part;    // 2 * chunks: per-chunk counts, then exclusive offsets
     int32_t* state;    // 8: PlocState per iteration parity
     uint32_t* depth;   // 1: internal ancestors of the deepest triangle of the PLOC tree
-    float4* pre;       // 2n: union of the leaf boxes from the start of the slot's refit block to it
-    float4* suf;       // 2n: union from the slot to the end of its refit block
-    float4* sparse;    // 2 * nb * levels: unions of 2^k consecutive refit blocks
+    TopArrays top;     // boundaries whose nodes span several tree blocks
     uint32_t* slot_order;  // n: primitive of each slot
     uint64_t bytes;
 };
 
 inline uint64_t align256(uint64_t x) { return (x + 255) & ~uint64_t(255); }
-
-// Refit blocks: bottom-up refit inside each range of kRefitBlock leaves runs in one workgroup
-// (k_refit_local, which also scans the block's leaf boxes into prefix/suffix unions); the nodes
-// whose range spans several blocks ("top" nodes) are refit afterwards from those range unions
-// (k_block_sparse, k_refit_top).
-constexpr int kRefitBlock = 1024;
-
-// levels of the sparse table over nb blocks: level k holds unions of 2^k consecutive blocks
-inline uint32_t sparse_levels(uint64_t nb) {
-    uint32_t l = 1;
-    while ((1ull << l) <= nb) ++l;
-    return l;
-}
 
 Workspace carve(char* base, uint64_t n) {
     Workspace w{};
@@ -113,11 +113,6 @@ Workspace carve(char* base, uint64_t n) {
     w.partial = (float*)take(4 * 8 * kReduceBlocks);
     w.cbounds = (float*)take(4 * 8);
     w.parent = (int32_t*)take(4 * (ni + n));
-    w.rangej = (int32_t*)take(4 * ni);
-    w.split = (int32_t*)take(4 * ni);
-    w.nodebox = (float4*)take(32 * ni);
-    w.top_list = (int32_t*)take(4 * ni);
-    w.top_count = (uint32_t*)take(4);
     const uint64_t nchunk = (n + 1023) / 1024 + 1;
     for (int k = 0; k < 2; ++k) {
         w.cid[k] = (int32_t*)take(4 * n);
@@ -134,12 +129,13 @@ Workspace carve(char* base, uint64_t n) {
     w.part = (uint32_t*)take(8 * nchunk);
     w.state = (int32_t*)take(4 * 8);
     w.depth = (uint32_t*)take(4);
-    w.pre = (float4*)take(32 * n);
-    w.suf = (float4*)take(32 * n);
-    {
-        const uint64_t nb = (n + kRefitBlock - 1) / kRefitBlock;
-        w.sparse = (float4*)take(32 * nb * sparse_levels(nb));
-    }
+    const uint64_t nb = (n + kTreeBlock - 1) / kTreeBlock;
+    w.top.list = (TopEntry*)take(sizeof(TopEntry) * kTopMax * nb);
+    w.top.count = (uint32_t*)take(4 * nb);
+    w.top.pre = (float4*)take(32 * n);
+    w.top.suf = (float4*)take(32 * n);
+    w.top.child = (float4*)take(64 * n);
+    w.top.block = (float4*)take(32 * nb);
     w.slot_order = (uint32_t*)take(4 * n);
     w.bytes = off;
     return w;
@@ -356,60 +352,6 @@ __global__ void __launch_bounds__(256) k_morton(const float4* __restrict__ cent,
     vals[i] = i;
 }
 
-// ---- hierarchy ----
-
-
-RT_DEV int delta(const uint32_t* __restrict__ k, int64_t n, int64_t i, int64_t j) {
-    if (j < 0 || j >= n) return -1;
-    const uint32_t a = k[i], b = k[j];
-    if (a != b) return __clz(a ^ b);
-    return 32 + __clz((uint32_t)i ^ (uint32_t)j);
-}
-
-__global__ void __launch_bounds__(256) k_hierarchy(const uint32_t* __restrict__ keys, uint32_t n,
-                                                    float4* __restrict__ nodes,
-                                                    int32_t* __restrict__ parent,
-                                                    int32_t* __restrict__ rangej,
-                                                    int32_t* __restrict__ split,
-                                                    uint32_t* __restrict__ top_count,
-                                                    int32_t* __restrict__ top_list) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)n - 1) return;
-    const int d = (delta(keys, n, i, i + 1) - delta(keys, n, i, i - 1)) >= 0 ? 1 : -1;
-    const int dmin = delta(keys, n, i, i - d);
-    int64_t lmax = 2;
-    while (delta(keys, n, i, i + lmax * d) > dmin) lmax *= 2;
-    int64_t l = 0;
-    for (int64_t t = lmax / 2; t >= 1; t /= 2)
-        if (delta(keys, n, i, i + (l + t) * d) > dmin) l += t;
-    const int64_t j = i + l * d;
-    const int dnode = delta(keys, n, i, j);
-    int64_t s = 0, t = l;
-    for (;;) {
-        t = (t + 1) / 2;
-        if (delta(keys, n, i, i + (s + t) * d) > dnode) s += t;
-        if (t <= 1) break;
-    }
-    const int64_t gamma = i + s * d + (d < 0 ? -1 : 0);
-    const int64_t lo = i < j ? i : j, hi = i < j ? j : i;
-    // binary radix tree (used by the refit): children gamma / gamma+1, leaves when their range is
-    // a single slot
-    const int32_t left = (lo == gamma) ? ~(int32_t)gamma : (int32_t)gamma;
-    const int32_t right = (hi == gamma + 1) ? ~(int32_t)(gamma + 1) : (int32_t)(gamma + 1);
-    // traversal refs: a child whose range holds <= kLeafMax slots becomes one leaf of that range
-    const int64_t nl = gamma - lo + 1, nr = hi - gamma;
-    const int32_t tl = nl <= kLeafMax ? leaf_ref((uint32_t)lo, (uint32_t)nl) : (int32_t)gamma;
-    const int32_t tr = nr <= kLeafMax ? leaf_ref((uint32_t)(gamma + 1), (uint32_t)nr) : (int32_t)(gamma + 1);
-    nodes[(uint64_t)i * 4 + 3] = make_float4(__int_as_float(tl), __int_as_float(tr), 0.0f, 0.0f);
-    const uint64_t ni = (uint64_t)n - 1;
-    parent[left >= 0 ? (uint64_t)left : ni + (uint64_t)(~left)] = (int32_t)i;
-    parent[right >= 0 ? (uint64_t)right : ni + (uint64_t)(~right)] = (int32_t)i;
-    rangej[i] = (int32_t)j;
-    split[i] = (int32_t)gamma;
-    if (i == 0) parent[0] = -1;
-    if (lo / kRefitBlock != hi / kRefitBlock) top_list[atomicAdd(top_count, 1u)] = (int32_t)i;
-}
-
 // One thread per float4 of the outputs: thread x copies shade float4 x (record x/4) and, for
 // x < 3n, tris float4 x (record x/3), so each store instruction writes consecutive 16 B pieces
 // and each record's source is read as consecutive pieces by neighbouring lanes.
@@ -428,321 +370,267 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order
     }
 }
 
-// ---- refit ----
-// Internal node i covers the sorted leaves [min(i,j), max(i,j)] (j = rangej[i]). With blocks of
-// kRefitBlock consecutive leaves, a node whose range lies in one block is "local": its whole
-// subtree is refit by that block's workgroup, which synchronises only through LDS. The few nodes
-// whose ranges span blocks ("top" nodes) are refit afterwards with device-scope counters.
+// ---- tree ----
+// The binary radix tree over the extended keys (code, slot). Boundary P lies between slots P - 1
+// and P; diff(P) is the common prefix of the two (-1 at 0 and n). Each boundary inside the range is
+// the split of one internal node, whose slots reach to the nearest boundaries on either side with a
+// smaller diff; that pair never ties except at the root. A node [lo, hi] is the right child of
+// boundary lo if diff(lo) > diff(hi + 1), else the left child of boundary hi + 1, and its id is lo or
+// hi accordingly (the root's is 0).
+//
+// k_tree_local: one workgroup per kTreeBlock slots builds every node that lies inside them in one
+// pass, bottom-up in LDS: a node stores its box under its id, the second child to arrive at a
+// boundary (LDS counter, workgroup acq_rel) makes the parent and goes on. Left over are the "top"
+// boundaries, whose nodes span blocks: the strict prefix and suffix minima of diff, so at most 2 x 64,
+// and the block's lower edge. They cut the block into segments, the largest subtrees inside it.
+// k_tree_top: one wave per top boundary finds the ends that lie in other blocks by a 64-ary search and
+// unites its children's boxes from segments, block suffixes and prefixes at top boundaries and whole
+// blocks. No node waits on another workgroup.
+//
+// What bounds it: LDS round trips per level of a walk (10 to 17 levels), and 64 B per node of stores
+// in pieces of 16 B; 37 KB of LDS and one slot per thread put two
+// workgroups on a CU.
+// At 1.31 M triangles 72 us for the local pass and 25 for the top; separate kernels for the hierarchy
+// (binary searches in memory, 93 us), a refit over its arrays (142), a sparse table of block unions
+// (17) and the top refit (10) took 262. At 11,560 triangles 25 us against 61.
+struct Box {
+    float lo[3], hi[3];
+};
 
-// Children of internal node i in the binary radix tree: internal ids, or ~slot for single leaves.
-RT_DEV void binary_children(const int32_t* __restrict__ rangej, const int32_t* __restrict__ split,
-                            int32_t i, int32_t& l, int32_t& r) {
-    const int32_t j = rangej[i], g = split[i];
-    const int32_t lo = i < j ? i : j, hi = i < j ? j : i;
-    l = lo == g ? ~g : g;
-    r = hi == g + 1 ? ~(g + 1) : g + 1;
+// length of the common prefix of the extended keys (a, i) and (b, j)
+RT_DEV int key_prefix(uint32_t a, uint32_t b, int64_t i, int64_t j) {
+    return a != b ? __clz(a ^ b) : 32 + __clz((uint32_t)i ^ (uint32_t)j);
 }
 
-RT_DEV void leaf_box(const float4* __restrict__ leafbox, const uint32_t* __restrict__ order,
-                     int32_t ref, float* lo, float* hi) {
-    const uint64_t p = order[~ref];
-    const float4 a = leafbox[2 * p], b = leafbox[2 * p + 1];
-    lo[0] = a.x; lo[1] = a.y; lo[2] = a.z;
-    hi[0] = b.x; hi[1] = b.y; hi[2] = b.z;
+// common prefix of slots p - 1 and p; -1 at the scene's ends
+RT_DEV int diff_at(const uint32_t* __restrict__ keys, int64_t n, int64_t p) {
+    return p <= 0 || p >= n ? -1 : key_prefix(keys[p - 1], keys[p], p - 1, p);
 }
 
-// Writes the child boxes into node record `node`, its own box (union) to nodebox, and returns it.
-RT_DEV void store_node(float4* __restrict__ nodes, float4* __restrict__ nodebox,
-                       float* __restrict__ bounds, int32_t node, const float* l_lo, const float* l_hi,
-                       const float* r_lo, const float* r_hi, float* u_lo, float* u_hi) {
-    float4* nd = nodes + (uint64_t)node * 4;
-    nd[0] = make_float4(l_lo[0], l_hi[0], l_lo[1], l_hi[1]);
-    nd[1] = make_float4(r_lo[0], r_hi[0], r_lo[1], r_hi[1]);
-    nd[2] = make_float4(l_lo[2], l_hi[2], r_lo[2], r_hi[2]);
-    for (int c = 0; c < 3; ++c) {
-        u_lo[c] = fminf(l_lo[c], r_lo[c]);
-        u_hi[c] = fmaxf(l_hi[c], r_hi[c]);
-    }
-    nodebox[2 * (uint64_t)node] = make_float4(u_lo[0], u_lo[1], u_lo[2], 0.0f);
-    nodebox[2 * (uint64_t)node + 1] = make_float4(u_hi[0], u_hi[1], u_hi[2], 0.0f);
-    if (node == 0) {
-        bounds[0] = u_lo[0]; bounds[1] = u_lo[1]; bounds[2] = u_lo[2]; bounds[3] = 0.0f;
-        bounds[4] = u_hi[0]; bounds[5] = u_hi[1]; bounds[6] = u_hi[2]; bounds[7] = 0.0f;
-    }
+RT_DEV Box empty_box() {
+    return {{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
 }
 
-// Range unions for the top refit, per refit block: the prefix and suffix unions of its leaf boxes
-// in slot order and the block's total, level 0 of the sparse table. A workgroup scan over the
-// block's slots, kRefitBlock / 256 per thread (thread t holds slots s0 .. s0 + kPer - 1 in lo/hi,
-// empty boxes past n); tlo/thi are 256-entry LDS rows. Called by all threads of the workgroup.
-constexpr int kPer = kRefitBlock / 256;
-RT_DEV void block_unions(const float (&lo)[kPer][3], const float (&hi)[kPer][3], uint64_t s0, uint32_t n,
-                         float4* __restrict__ pre, float4* __restrict__ suf,
-                         float4* __restrict__ sparse, float (*tlo)[256], float (*thi)[256]) {
-    const uint32_t t = threadIdx.x;
-    // exclusive prefix union of the thread totals, then inclusive per slot
-    float tl[3], th[3];
+RT_DEV Box unite(const Box& a, const Box& b) {
+    Box u;
     for (int c = 0; c < 3; ++c) {
-        tl[c] = INFINITY;
-        th[c] = -INFINITY;
-        for (int k = 0; k < kPer; ++k) {
-            tl[c] = fminf(tl[c], lo[k][c]);
-            th[c] = fmaxf(th[c], hi[k][c]);
-        }
-        tlo[c][t] = tl[c];
-        thi[c][t] = th[c];
+        u.lo[c] = fminf(a.lo[c], b.lo[c]);
+        u.hi[c] = fmaxf(a.hi[c], b.hi[c]);
     }
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {  // inclusive scan of the totals
-        float xl[3], xh[3];
-        for (int c = 0; c < 3; ++c) {
-            xl[c] = t >= (uint32_t)off ? tlo[c][t - off] : INFINITY;
-            xh[c] = t >= (uint32_t)off ? thi[c][t - off] : -INFINITY;
-        }
-        __syncthreads();
-        for (int c = 0; c < 3; ++c) {
-            tlo[c][t] = fminf(tlo[c][t], xl[c]);
-            thi[c][t] = fmaxf(thi[c][t], xh[c]);
-        }
-        __syncthreads();
-    }
-    float rl[3], rh[3];
-    for (int c = 0; c < 3; ++c) {
-        rl[c] = t > 0 ? tlo[c][t - 1] : INFINITY;
-        rh[c] = t > 0 ? thi[c][t - 1] : -INFINITY;
-    }
-    if (t == 255) {
-        sparse[2 * (uint64_t)blockIdx.x] = make_float4(tlo[0][255], tlo[1][255], tlo[2][255], 0.0f);
-        sparse[2 * (uint64_t)blockIdx.x + 1] = make_float4(thi[0][255], thi[1][255], thi[2][255], 0.0f);
-    }
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        for (int c = 0; c < 3; ++c) {
-            rl[c] = fminf(rl[c], lo[k][c]);
-            rh[c] = fmaxf(rh[c], hi[k][c]);
-        }
-        if (s0 + k < n) {
-            pre[2 * (s0 + k)] = make_float4(rl[0], rl[1], rl[2], 0.0f);
-            pre[2 * (s0 + k) + 1] = make_float4(rh[0], rh[1], rh[2], 0.0f);
-        }
-    }
-    __syncthreads();
-    // suffix: the same over the reversed thread order
-    for (int c = 0; c < 3; ++c) {
-        tlo[c][t] = tl[c];
-        thi[c][t] = th[c];
-    }
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        float xl[3], xh[3];
-        for (int c = 0; c < 3; ++c) {
-            xl[c] = t + off < 256u ? tlo[c][t + off] : INFINITY;
-            xh[c] = t + off < 256u ? thi[c][t + off] : -INFINITY;
-        }
-        __syncthreads();
-        for (int c = 0; c < 3; ++c) {
-            tlo[c][t] = fminf(tlo[c][t], xl[c]);
-            thi[c][t] = fmaxf(thi[c][t], xh[c]);
-        }
-        __syncthreads();
-    }
-    for (int c = 0; c < 3; ++c) {
-        rl[c] = t < 255 ? tlo[c][t + 1] : INFINITY;
-        rh[c] = t < 255 ? thi[c][t + 1] : -INFINITY;
-    }
-#pragma unroll
-    for (int k = kPer - 1; k >= 0; --k) {
-        for (int c = 0; c < 3; ++c) {
-            rl[c] = fminf(rl[c], lo[k][c]);
-            rh[c] = fmaxf(rh[c], hi[k][c]);
-        }
-        if (s0 + k < n) {
-            suf[2 * (s0 + k)] = make_float4(rl[0], rl[1], rl[2], 0.0f);
-            suf[2 * (s0 + k) + 1] = make_float4(rh[0], rh[1], rh[2], 0.0f);
-        }
-    }
+    return u;
 }
 
+RT_DEV Box load_box(const float4* __restrict__ p) {
+    const float4 a = p[0], b = p[1];
+    return {{a.x, a.y, a.z}, {b.x, b.y, b.z}};
+}
 
-// Phase 1: block b walks up from each of its leaves through the local nodes (those whose leaf range
-// lies inside the block; a node's id is an end of its range, so local nodes have ids in the block
-// too). The block first copies what the walks read into LDS: the rangej / split / parent entries of
-// its node ids and the boxes of its leaves (gathered through `order`). The first thread to reach a
-// node stops; the second (LDS counter, workgroup acq_rel) unions the children's boxes from LDS and
-// writes the node. Before the walks, the block scans its leaf boxes into range unions.
-__global__ void __launch_bounds__(256) k_refit_local(const uint32_t* __restrict__ order, uint32_t n,
-                                                      const float4* __restrict__ leafbox,
-                                                      const int32_t* __restrict__ parent,
-                                                      const int32_t* __restrict__ rangej,
-                                                      const int32_t* __restrict__ split,
-                                                      float4* __restrict__ nodes,
-                                                      float4* __restrict__ nodebox,
-                                                      float* __restrict__ bounds,
-                                                      float4* __restrict__ pre,
-                                                      float4* __restrict__ suf,
-                                                      float4* __restrict__ sparse) {
-    __shared__ uint32_t lflag[kRefitBlock];
-    __shared__ float tlo[3][256], thi[3][256];
-    __shared__ float lbox[kRefitBlock][6];   // boxes of the block's internal nodes
-    __shared__ float lleaf[kRefitBlock][6];  // boxes of the block's leaves (slots)
-    __shared__ int32_t lj[kRefitBlock], lsplit[kRefitBlock], lpar[kRefitBlock];
-    const int64_t blo = (int64_t)blockIdx.x * kRefitBlock;
-    const int64_t bhi = std::min<int64_t>(blo + kRefitBlock, n);  // exclusive
-    const int64_t ni = (int64_t)n - 1;
-    for (int k = threadIdx.x; k < kRefitBlock; k += blockDim.x) {
-        lflag[k] = 0;
-        if (blo + k < ni) {
-            lj[k] = rangej[blo + k];
-            lsplit[k] = split[blo + k];
-            lpar[k] = parent[blo + k];
-        }
-        if (blo + k < bhi) {
-            const uint64_t p = order[blo + k];
-            const float4 a = leafbox[2 * p], b = leafbox[2 * p + 1];
-            lleaf[k][0] = a.x; lleaf[k][1] = a.y; lleaf[k][2] = a.z;
-            lleaf[k][3] = b.x; lleaf[k][4] = b.y; lleaf[k][5] = b.z;
-        }
+RT_DEV void store_box(float4* __restrict__ p, const Box& b) {
+    p[0] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f);
+    p[1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.0f);
+}
+
+// Record of node `id` with slots [lo, hi1) split at boundary p; a child of at most kLeafMax slots
+// becomes one leaf of them.
+RT_DEV void store_tree_node(float4* __restrict__ nodes, uint32_t id, uint32_t lo, uint32_t p, uint32_t hi1,
+                            const Box& l, const Box& r) {
+    const uint32_t nl = p - lo, nr = hi1 - p;
+    const int32_t tl = nl <= (uint32_t)kLeafMax ? leaf_ref(lo, nl) : (int32_t)(p - 1);
+    const int32_t tr = nr <= (uint32_t)kLeafMax ? leaf_ref(p, nr) : (int32_t)p;
+    float4* nd = nodes + (uint64_t)id * 4;
+    nd[0] = make_float4(l.lo[0], l.hi[0], l.lo[1], l.hi[1]);
+    nd[1] = make_float4(r.lo[0], r.hi[0], r.lo[1], r.hi[1]);
+    nd[2] = make_float4(l.lo[2], l.hi[2], r.lo[2], r.hi[2]);
+    nd[3] = make_float4(__int_as_float(tl), __int_as_float(tr), 0.0f, 0.0f);
+}
+
+RT_DEV void store_bounds(float* __restrict__ bounds, const Box& b) {
+    for (int c = 0; c < 3; ++c) {
+        bounds[c] = b.lo[c];
+        bounds[4 + c] = b.hi[c];
     }
+    bounds[3] = bounds[7] = 0.0f;
+}
+
+__global__ void __launch_bounds__(kTreeBlock) k_tree_local(const uint32_t* __restrict__ keys,
+                                                             const uint32_t* __restrict__ order, uint32_t n,
+                                                             const float4* __restrict__ leafbox,
+                                                             float4* __restrict__ nodes,
+                                                             float* __restrict__ bounds, TopArrays top) {
+    __shared__ float box[6][kTreeBlock];  // by local node id: the box of a node whose parent is pending
+    __shared__ int32_t other[kTreeBlock];  // and the end of its slots that is not its id
+    __shared__ uint32_t arrived[kTreeBlock];
+    __shared__ int32_t diff[kTreeBlock + 1];
+    __shared__ int32_t seg[kTopMax + 2];
+    __shared__ int32_t nseg;
+    const int64_t blo = (int64_t)blockIdx.x * kTreeBlock;
+    const int cnt = (int)(n - blo < kTreeBlock ? n - blo : kTreeBlock);
+    const int tid = threadIdx.x;
+    Box b = empty_box();
+    if (tid < cnt) {
+        const uint32_t prim = order[blo + tid];
+        diff[tid] = diff_at(keys, n, blo + tid);
+        if (tid == 0) diff[cnt] = diff_at(keys, n, blo + cnt);
+        b = load_box(leafbox + 2 * (uint64_t)prim);
+    }
+    arrived[tid] = 0;
     __syncthreads();
-    {  // the block's range unions, from the leaf boxes already in LDS
-        float lo[kPer][3], hi[kPer][3];
-        const uint32_t l0 = threadIdx.x * kPer;
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const bool in = blo + l0 + k < bhi;
-            for (int c = 0; c < 3; ++c) {
-                lo[k][c] = in ? lleaf[l0 + k][c] : INFINITY;
-                hi[k][c] = in ? lleaf[l0 + k][3 + c] : -INFINITY;
+    auto put = [&](int e, const Box& b) {
+        for (int c = 0; c < 3; ++c) {
+            box[c][e] = b.lo[c];
+            box[3 + c][e] = b.hi[c];
+        }
+    };
+    auto get = [&](int e) {
+        Box b;
+        for (int c = 0; c < 3; ++c) {
+            b.lo[c] = box[c][e];
+            b.hi[c] = box[3 + c][e];
+        }
+        return b;
+    };
+    if (tid < cnt) {
+        Box l = b, r = b;
+        int lo = tid, hi = tid, split = tid;
+        for (;;) {
+            const int dl = diff[lo], dr = diff[hi + 1];
+            const bool right = dl > dr, root = dl < 0 && dr < 0;
+            const int e = right ? lo : hi;
+            if (lo < hi)
+                store_tree_node(nodes, root ? 0u : (uint32_t)(blo + e), (uint32_t)(blo + lo),
+                                (uint32_t)(blo + split), (uint32_t)(blo + hi + 1), l, r);
+            if (root) {
+                store_bounds(bounds, b);
+                break;
             }
-        }
-        block_unions(lo, hi, (uint64_t)blo + l0, n, pre, suf, sparse, tlo, thi);
-    }
-    for (int64_t s = blo + threadIdx.x; s < bhi; s += blockDim.x) {
-        int32_t node = parent[ni + s];
-        while (node >= blo && node < bhi && node < ni) {
-            const int32_t li = (int32_t)(node - blo);
-            const int64_t j = lj[li];
-            const int64_t lo = std::min<int64_t>(node, j), hi = std::max<int64_t>(node, j);
-            if (lo < blo || hi >= bhi) break;  // a top node: phase 2
-            const uint32_t prev = __hip_atomic_fetch_add(&lflag[li], 1u, __ATOMIC_ACQ_REL,
+            put(e, b);
+            other[e] = right ? hi : lo;
+            const int p = right ? lo : hi + 1;
+            if (p == 0 || p == cnt) break;  // the boundary to another block
+            const uint32_t prev = __hip_atomic_fetch_add(&arrived[p], 1u, __ATOMIC_ACQ_REL,
                                                          __HIP_MEMORY_SCOPE_WORKGROUP);
             if (prev == 0) break;
-            const int32_t g = lsplit[li];
-            const int32_t l = lo == g ? ~g : g, r = hi == g + 1 ? ~(g + 1) : g + 1;
-            const float* lb = l < 0 ? lleaf[~l - blo] : lbox[l - blo];
-            const float* rb = r < 0 ? lleaf[~r - blo] : lbox[r - blo];
-            float l_lo[3], l_hi[3], r_lo[3], r_hi[3], u_lo[3], u_hi[3];
-            for (int c = 0; c < 3; ++c) {
-                l_lo[c] = lb[c];
-                l_hi[c] = lb[3 + c];
-                r_lo[c] = rb[c];
-                r_hi[c] = rb[3 + c];
+            const int q = right ? lo - 1 : hi + 1;  // the sibling's id
+            const Box o = get(q);
+            if (right) {
+                l = o;
+                r = b;
+                lo = other[q];
+            } else {
+                l = b;
+                r = o;
+                hi = other[q];
             }
-            store_node(nodes, nodebox, bounds, node, l_lo, l_hi, r_lo, r_hi, u_lo, u_hi);
+            split = p;
+            b = unite(l, r);
+        }
+    }
+    if (gridDim.x == 1) return;
+    __syncthreads();
+    // the segments' starts: 0 and the boundaries at which fewer than two children arrived
+    if (tid < 64) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int k = 0; k < kTreeBlock / 64; ++k) {
+            const int p = k * 64 + tid;
+            const bool is = p == 0 || (p < cnt && arrived[p] < 2u);
+            const uint64_t mask = __ballot(is);
+            const uint32_t at = m + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+            if (is && at < (uint32_t)kTopMax) seg[at] = p;  // always true: at most 129
+            m += (uint32_t)__popcll(mask);
+        }
+        if (tid == 0) {
+            nseg = (int32_t)(m < (uint32_t)kTopMax ? m : (uint32_t)kTopMax);
+            seg[nseg] = cnt;
+        }
+    }
+    __syncthreads();
+    const int m = nseg;
+    const int first = blo == 0 ? 1 : 0;  // boundary 0 of the scene is no node's split
+    if (tid == 0) top.count[blockIdx.x] = (uint32_t)(m - first);
+    if (tid >= m) return;
+    auto seg_id = [&](int j) { return diff[seg[j]] > diff[seg[j + 1]] ? seg[j] : seg[j + 1] - 1; };
+    const int j = tid, p = seg[j], d = diff[p];
+    const Box own = get(seg_id(j));
+    if (d > diff[seg[j + 1]])
+        store_box(top.child + 4 * (uint64_t)(blo + p) + 2, own);
+    else
+        store_box(top.child + 4 * (uint64_t)(blo + seg[j + 1]), own);
+    Box pre = empty_box(), suf = empty_box();
+    for (int i = 0; i < j; ++i) pre = unite(pre, get(seg_id(i)));
+    for (int i = j; i < m; ++i) suf = unite(suf, get(seg_id(i)));
+    store_box(top.pre + 2 * (uint64_t)(blo + p), pre);
+    store_box(top.suf + 2 * (uint64_t)(blo + p), suf);
+    if (j == 0) store_box(top.block + 2 * (uint64_t)blockIdx.x, suf);
+    if (j < first) return;
+    TopEntry t{(int32_t)(blo + p), -1, -1, d, keys[blo + p], {}};
+    for (int i = j - 1; i >= 0 && t.lo < 0; --i)
+        if (diff[seg[i]] < d) t.lo = (int32_t)(blo + seg[i]);
+    for (int i = j + 1; i <= m && t.hi1 < 0; ++i)
+        if (diff[seg[i]] < d) t.hi1 = (int32_t)(blo + seg[i]);
+    top.list[(uint64_t)blockIdx.x * kTopMax + (j - first)] = t;
+}
+
+// The first x in [a, b] for which pred(x) holds, with pred(b) true and pred monotone, by all 64 lanes:
+// each round tests 64 evenly spaced positions.
+template <typename Pred>
+RT_DEV int64_t wave_first(int64_t a, int64_t b, int lane, Pred pred) {
+    while (a < b) {
+        const int64_t step = (b - a + 63) / 64;
+        const int64_t x = a + lane * step;
+        const uint64_t yes = __ballot(x >= b || pred(x));
+        const int f = yes ? __ffsll((unsigned long long)yes) - 1 : 64;
+        const int64_t hit = a + f * step;
+        if (f > 0) a = a + (f - 1) * step + 1;
+        if (f < 64 && hit < b) b = hit;
+    }
+    return a;
+}
+
+// Box of slots [lo, hi1), which span several blocks: the suffix of lo's block, the prefix of hi1's and
+// the whole blocks between, spread over the lanes. (min and max are exact, so the order is free.)
+RT_DEV Box wave_range_box(const TopArrays& top, int64_t lo, int64_t hi1, uint32_t n, uint32_t nb, int lane) {
+    const int64_t b0 = (lo + kTreeBlock - 1) / kTreeBlock;
+    const int64_t b1 = hi1 == (int64_t)n ? (int64_t)nb : hi1 / kTreeBlock;
+    Box b = empty_box();
+    if (lo % kTreeBlock) b = unite(b, load_box(top.suf + 2 * (uint64_t)lo));
+    if (hi1 != (int64_t)n && hi1 % kTreeBlock) b = unite(b, load_box(top.pre + 2 * (uint64_t)hi1));
+    if (b0 < b1) {
+        for (int64_t k = b0 + lane; k < b1; k += 64) b = unite(b, load_box(top.block + 2 * (uint64_t)k));
+        for (int x = 1; x < 64; x <<= 1)
             for (int c = 0; c < 3; ++c) {
-                lbox[li][c] = u_lo[c];
-                lbox[li][3 + c] = u_hi[c];
+                b.lo[c] = fminf(b.lo[c], __shfl_xor(b.lo[c], x));
+                b.hi[c] = fmaxf(b.hi[c], __shfl_xor(b.hi[c], x));
             }
-            node = lpar[li];
-        }
     }
+    return b;
 }
 
-RT_DEV bool is_local(const int32_t* __restrict__ rangej, int32_t ref) {
-    if (ref < 0) return true;
-    const int32_t j = rangej[ref];
-    const int32_t lo = ref < j ? ref : j, hi = ref < j ? j : ref;
-    return lo / kRefitBlock == hi / kRefitBlock;
-}
-
-RT_DEV void node_box(const float4* __restrict__ leafbox, const uint32_t* __restrict__ order,
-                     const float4* nodebox, int32_t ref, float* lo, float* hi) {
-    if (ref < 0) {
-        leaf_box(leafbox, order, ref, lo, hi);
-    } else {
-        const float4 a = nodebox[2 * (uint64_t)ref], b = nodebox[2 * (uint64_t)ref + 1];
-        lo[0] = a.x; lo[1] = a.y; lo[2] = a.z;
-        hi[0] = b.x; hi[1] = b.y; hi[2] = b.z;
-    }
-}
-
-// Sparse table levels 1.. in one workgroup: level k, block b = union of levels k-1 at b and
-// b + 2^(k-1) (the workgroup's barrier orders the levels' global stores and loads).
-__global__ void __launch_bounds__(1024) k_block_sparse(float4* __restrict__ sparse, uint32_t nb,
-                                                        uint32_t levels) {
-    for (uint32_t k = 1; k < levels; ++k) {
-        const uint32_t half = 1u << (k - 1), cnt = nb - (2u * half) + 1u;
-        const float4* src = sparse + 2 * (uint64_t)(k - 1) * nb;
-        float4* dst = sparse + 2 * (uint64_t)k * nb;
-        for (uint32_t b = threadIdx.x; b < cnt; b += blockDim.x) {
-            const float4 a0 = src[2 * (uint64_t)b], a1 = src[2 * (uint64_t)b + 1];
-            const float4 b0 = src[2 * (uint64_t)(b + half)], b1 = src[2 * (uint64_t)(b + half) + 1];
-            dst[2 * (uint64_t)b] = make_float4(fminf(a0.x, b0.x), fminf(a0.y, b0.y), fminf(a0.z, b0.z), 0.0f);
-            dst[2 * (uint64_t)b + 1] = make_float4(fmaxf(a1.x, b1.x), fmaxf(a1.y, b1.y), fmaxf(a1.z, b1.z), 0.0f);
+__global__ void __launch_bounds__(kTopThreads) k_tree_top(const uint32_t* __restrict__ keys, uint32_t n,
+                                                  float4* __restrict__ nodes, float* __restrict__ bounds,
+                                                  TopArrays top) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t nb = gridDim.x, cnt = top.count[blockIdx.x];
+    for (uint32_t i = threadIdx.x >> 6; i < cnt; i += blockDim.x >> 6) {
+        const TopEntry t = top.list[(uint64_t)blockIdx.x * kTopMax + i];
+        const int64_t p = t.p, edge = (int64_t)blockIdx.x * kTreeBlock;
+        int64_t lo = t.lo, hi1 = t.hi1;
+        // slots of the node are those that share its d leading bits
+        const auto prefix = [&](int64_t x) { return key_prefix(keys[x], t.key, x, p); };
+        if (lo < 0) lo = wave_first(0, edge - 1, lane, [&](int64_t x) { return prefix(x) >= t.diff; });
+        if (hi1 < 0) hi1 = wave_first(edge + kTreeBlock, n, lane, [&](int64_t x) { return prefix(x) < t.diff; });
+        const bool root = lo == 0 && hi1 == (int64_t)n;
+        const bool right = diff_at(keys, n, lo) > diff_at(keys, n, hi1);
+        const bool l_in = lo / kTreeBlock == (p - 1) / kTreeBlock;
+        const bool r_in = p / kTreeBlock == (hi1 - 1) / kTreeBlock;
+        const Box l = l_in ? load_box(top.child + 4 * (uint64_t)p) : wave_range_box(top, lo, p, n, nb, lane);
+        const Box r = r_in ? load_box(top.child + 4 * (uint64_t)p + 2) : wave_range_box(top, p, hi1, n, nb, lane);
+        if (lane == 0) {
+            store_tree_node(nodes, root ? 0u : (uint32_t)(right ? lo : hi1 - 1), (uint32_t)lo, (uint32_t)p,
+                            (uint32_t)hi1, l, r);
+            if (root) store_bounds(bounds, unite(l, r));
         }
-        __syncthreads();
-    }
-}
-
-// Union of the leaf boxes of slots [lo, hi], which span at least two refit blocks: the suffix of
-// lo's block, the prefix of hi's block and the blocks between (two overlapping sparse-table
-// entries; min/max are exact, so overlap and order do not change the result).
-RT_DEV void range_box(const float4* __restrict__ pre, const float4* __restrict__ suf,
-                      const float4* __restrict__ sparse, uint32_t nb, int32_t lo, int32_t hi,
-                      float* blo, float* bhi) {
-    const float4 s0 = suf[2 * (uint64_t)lo], s1 = suf[2 * (uint64_t)lo + 1];
-    const float4 p0 = pre[2 * (uint64_t)hi], p1 = pre[2 * (uint64_t)hi + 1];
-    blo[0] = fminf(s0.x, p0.x); blo[1] = fminf(s0.y, p0.y); blo[2] = fminf(s0.z, p0.z);
-    bhi[0] = fmaxf(s1.x, p1.x); bhi[1] = fmaxf(s1.y, p1.y); bhi[2] = fmaxf(s1.z, p1.z);
-    const int32_t b0 = lo / kRefitBlock + 1, b1 = hi / kRefitBlock - 1;
-    if (b0 <= b1) {
-        const uint32_t len = (uint32_t)(b1 - b0 + 1);
-        const uint32_t k = 31u - __builtin_clz(len);
-        const float4* lv = sparse + 2 * (uint64_t)k * nb;
-        const uint64_t x = (uint64_t)b0, y = (uint64_t)(b1 - (int32_t)(1u << k) + 1);
-        const float4 a0 = lv[2 * x], a1 = lv[2 * x + 1], c0 = lv[2 * y], c1 = lv[2 * y + 1];
-        blo[0] = fminf(blo[0], fminf(a0.x, c0.x));
-        blo[1] = fminf(blo[1], fminf(a0.y, c0.y));
-        blo[2] = fminf(blo[2], fminf(a0.z, c0.z));
-        bhi[0] = fmaxf(bhi[0], fmaxf(a1.x, c1.x));
-        bhi[1] = fmaxf(bhi[1], fmaxf(a1.y, c1.y));
-        bhi[2] = fmaxf(bhi[2], fmaxf(a1.z, c1.z));
-    }
-}
-
-// Phase 3, one thread per top node (the list written by k_hierarchy): each child's box is its
-// range union (a top child), or the box phase 1 computed (a local child or a leaf). No node waits on
-// another.
-__global__ void __launch_bounds__(256) k_refit_top(const uint32_t* __restrict__ order, uint32_t n,
-                                                    const float4* __restrict__ leafbox,
-                                                    const int32_t* __restrict__ rangej,
-                                                    const int32_t* __restrict__ split,
-                                                    float4* __restrict__ nodes, float4* nodebox,
-                                                    float* __restrict__ bounds,
-                                                    const int32_t* __restrict__ top_list,
-                                                    const uint32_t* __restrict__ top_count,
-                                                    const float4* __restrict__ pre,
-                                                    const float4* __restrict__ suf,
-                                                    const float4* __restrict__ sparse, uint32_t nb) {
-    const uint32_t cnt = *top_count;
-    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < cnt; t += gridDim.x * blockDim.x) {
-        const int32_t node = top_list[t];
-        int32_t l, r;
-        binary_children(rangej, split, node, l, r);
-        float l_lo[3], l_hi[3], r_lo[3], r_hi[3], u_lo[3], u_hi[3];
-        if (is_local(rangej, l)) {
-            node_box(leafbox, order, nodebox, l, l_lo, l_hi);
-        } else {
-            const int32_t j = rangej[l];
-            range_box(pre, suf, sparse, nb, l < j ? l : j, l < j ? j : l, l_lo, l_hi);
-        }
-        if (is_local(rangej, r)) {
-            node_box(leafbox, order, nodebox, r, r_lo, r_hi);
-        } else {
-            const int32_t j = rangej[r];
-            range_box(pre, suf, sparse, nb, r < j ? r : j, r < j ? j : r, r_lo, r_hi);
-        }
-        store_node(nodes, nodebox, bounds, node, l_lo, l_hi, r_lo, r_hi, u_lo, u_hi);
     }
 }
 
@@ -1625,22 +1513,14 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
         sc->root = n <= (uint32_t)kLeafMax ? leaf_ref(0, n) : 0;
         vi = w.slot_order;
     } else {
-    // 5. hierarchy, 6. emit, 7. refit (LBVH, or a PLOC tree found too deep)
-    if (n > 1) {
-        hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, s, w.top_count);
-        hipLaunchKernelGGL(k_hierarchy, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, ki, n, nodes,
-                           w.parent, w.rangej, w.split, w.top_count, w.top_list);
-    }
+    // 5. emit, 6. tree (LBVH, or a PLOC tree found too deep)
     hipLaunchKernelGGL(k_emit, dim3(blocks_for(4 * (uint64_t)n, 256)), dim3(256), 0, s, vi, n, w.tri_u, w.shade_u,
                        (float4*)sc->tris, (float4*)sc->shade);
     if (n > 1) {
-        const uint32_t nb = blocks_for(n, kRefitBlock);
-        hipLaunchKernelGGL(k_refit_local, dim3(nb), dim3(256), 0, s, vi, n, w.leafbox, w.parent,
-                           w.rangej, w.split, nodes, w.nodebox, sc->bounds, w.pre, w.suf, w.sparse);
-        hipLaunchKernelGGL(k_block_sparse, dim3(1), dim3(1024), 0, s, w.sparse, nb, sparse_levels(nb));
-        hipLaunchKernelGGL(k_refit_top, dim3(std::min<uint32_t>(blocks_for(n, 256), 1024)), dim3(256), 0, s,
-                           vi, n, w.leafbox, w.rangej, w.split, nodes, w.nodebox, sc->bounds, w.top_list,
-                           w.top_count, w.pre, w.suf, w.sparse, nb);
+        const uint32_t nb = blocks_for(n, kTreeBlock);
+        hipLaunchKernelGGL(k_tree_local, dim3(nb), dim3(kTreeBlock), 0, s, ki, vi, n, w.leafbox, nodes,
+                           sc->bounds, w.top);
+        if (nb > 1) hipLaunchKernelGGL(k_tree_top, dim3(nb), dim3(kTopThreads), 0, s, ki, n, nodes, sc->bounds, w.top);
         hipLaunchKernelGGL(k_wide, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n,
                            (const float4*)nodes, (float4*)sc->nodes4);
         sc->root = n <= (uint32_t)kLeafMax ? leaf_ref(0, n) : 0;

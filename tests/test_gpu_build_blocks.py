@@ -1,0 +1,28 @@
+"""LBVH builds around the tree's block of 1,024 slots, byte for byte against the twin: spread triangles,
+equal codes (every split by slot number), and codes in a few crowded cells."""
+import numpy as np
+import pytest
+
+from helpers import gpu_from_meshes, twin_from_meshes
+from test_gpu_parity import assert_build_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def _mesh(n, kind):
+    rng = np.random.default_rng(n)
+    at = rng.uniform(-1, 1, (n, 1, 3))
+    if kind == "equal":
+        at[:] = 0.25
+    elif kind == "crowded":
+        at = np.sign(at) * 2.0 ** -np.floor(rng.exponential(4.0, (n, 1, 1)))
+    size = 0.0 if kind == "equal" else 1e-3
+    pos = at + size * rng.uniform(-1, 1, (n, 3, 3)) + (0.0 if size else np.eye(3))
+    return {"pos": pos.reshape(-1, 3).astype(np.float32), "idx": np.arange(3 * n, dtype=np.int32).reshape(-1, 3)}
+
+
+@pytest.mark.parametrize("kind", ["spread", "equal", "crowded"])
+@pytest.mark.parametrize("n", [2, 5, 1023, 1024, 1025, 2047, 2048, 2049, 65 * 1024 + 1, 70 * 1024])
+def test_block_edges(ren, n, kind):
+    meshes = [_mesh(n, kind)]
+    assert_build_equal(gpu_from_meshes(meshes), twin_from_meshes(meshes))
