@@ -64,88 +64,96 @@ __global__ void __launch_bounds__(kSortThreads) k_sort_rowscan(uint32_t* __restr
     }
     if (threadIdx.x == kSortThreads - 1) totals[blockIdx.x] = s[kSortThreads - 1];
 }
-// Stable scatter of one tile of kSortTile items. Items are visited in rounds of 256 (item order =
-// (round, thread)); each round is ranked by wave64 multi-split (8 ballots give the lanes sharing
-// this lane's digit) and written into LDS grouped by digit, so the tile ends up in LDS in
-// (digit, input order). The tile is then written out with consecutive threads taking consecutive
-// items: each digit's run of the tile lands in one contiguous span of the output.
+// Rank of each valid lane's digit among the wave's items so far, and the wave's counts advanced: `count`
+// is this wave's own row of LDS, cleared before its first round.
+template <int kBits>
+RT_DEV uint32_t wave_digit_rank(uint32_t d, bool valid, int lane, uint32_t* count) {
+    uint64_t peers = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < kBits; ++b) {
+        const bool bit = (d >> b) & 1u;
+        const uint64_t mb = __ballot(bit);
+        peers &= bit ? mb : ~mb;
+    }
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(peers >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
+    const uint32_t before = __hip_atomic_load(&count[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    if (valid && rank == 0)
+        __hip_atomic_store(&count[d], before + (uint32_t)__popcll(peers), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WAVEFRONT);
+    return before + rank;
+}
+
+// Stable scatter of one tile of kSortTile items, wave w holding items [w, w + 1) * 64 * kSortItems.
+// Each wave ranks its items alone, 64 at a time: 8 ballots give the lanes that share a lane's digit, and
+// the wave's own count of the digit in LDS goes on from the items before (a wave's LDS accesses stay
+// in order, so this takes no barrier; one round of all waves at a time, with three barriers each, took
+// 17.2 us a pass at 1.31 M pairs and 11.8 at 11,560, this takes 11.5 and 6.1). After one scan over digits and waves the tile goes to LDS in (digit, input order) and is
+// written out with consecutive threads taking consecutive items: each digit's run of the tile lands in
+// one contiguous span of the output.
 __global__ void __launch_bounds__(kSortThreads) k_sort_scatter(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin, uint32_t n, int shift,
     const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals, uint32_t nblk,
     uint32_t* __restrict__ kout,
     uint32_t* __restrict__ vout) {
     constexpr int kWaves = kSortThreads / 64;
-    __shared__ uint32_t base[kRadix];    // output position of this tile's first item of digit d
-    __shared__ uint32_t lstart[kRadix];  // LDS position of this tile's first item of digit d
-    __shared__ uint32_t run[kRadix];
-    __shared__ uint32_t wcount[kWaves][kRadix];
+    __shared__ uint32_t wcount[kWaves][kRadix];  // a wave's count of digit d, then its LDS position
+    __shared__ uint32_t base[kRadix];            // output position minus LDS position of digit d
+    __shared__ uint64_t wsum[kWaves];
     __shared__ uint32_t sk[kSortTile];
     __shared__ uint32_t sv[kSortTile];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t blk = blockIdx.x;
-    // the row scan left exclusive per-tile prefixes: this tile's count of digit tid is the step
-    // to the next tile's prefix (to the digit total for the last tile)
-    const uint32_t h0 = hist[(uint64_t)tid * nblk + blk];
-    const uint32_t cnt = (blk + 1 < nblk ? hist[(uint64_t)tid * nblk + blk + 1] : totals[tid]) - h0;
-    run[tid] = totals[tid];
-    lstart[tid] = cnt;
-    __syncthreads();
-    for (int off = 1; off < kRadix; off <<= 1) {  // inclusive scans of the totals and tile counts
-        const uint32_t x = tid >= off ? run[tid - off] : 0u;
-        const uint32_t y = tid >= off ? lstart[tid - off] : 0u;
-        __syncthreads();
-        run[tid] += x;
-        lstart[tid] += y;
-        __syncthreads();
-    }
-    base[tid] = run[tid] - totals[tid] + h0;
-    lstart[tid] -= cnt;
-    run[tid] = 0;
-    for (int w = 0; w < kWaves; ++w) wcount[w][tid] = 0;
-    __syncthreads();
     const uint64_t tile = (uint64_t)blk * kSortTile;
     const uint32_t m = (uint32_t)(n - tile < (uint64_t)kSortTile ? n - tile : (uint64_t)kSortTile);
-    for (int r = 0; r < kSortItems; ++r) {
-        const uint64_t i = tile + (uint64_t)r * kSortThreads + tid;
-        const bool valid = i < n;
-        const uint32_t key = valid ? kin[i] : 0u;
-        const uint32_t val = valid ? vin[i] : 0u;
-        const uint32_t d = (key >> shift) & (kRadix - 1);
-        uint64_t peers = __ballot(valid);
+    const uint32_t first = wave * (64 * kSortItems) + lane;
+    uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
 #pragma unroll
-        for (int b = 0; b < kRadixBits; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t mb = __ballot(bit);
-            peers &= bit ? mb : ~mb;
-        }
-        const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
-            (uint32_t)(peers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
-        const int leader = __ffsll((unsigned long long)peers) - 1;
-        if (valid && lane == leader) wcount[wave][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (valid) {
-            uint32_t off = lstart[d] + run[d] + rank;
-            for (int w = 0; w < wave; ++w) off += wcount[w][d];
-            if (off < (uint32_t)kSortTile) {  // always true for a consistent histogram
-                sk[off] = key;
-                sv[off] = val;
-            }
-        }
-        __syncthreads();
-        uint32_t add = 0;
-        for (int w = 0; w < kWaves; ++w) {
-            add += wcount[w][tid];
-            wcount[w][tid] = 0;
-        }
-        run[tid] += add;
-        __syncthreads();
+    for (int r = 0; r < kSortItems; ++r) {
+        const uint32_t i = first + r * 64;
+        key[r] = i < m ? kin[tile + i] : 0u;
+        val[r] = i < m ? vin[tile + i] : 0u;
     }
+    const uint32_t total = totals[tid], before = hist[(uint64_t)tid * nblk + blk];
+    for (int w = 0; w < kWaves; ++w) wcount[w][tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r)
+        rank[r] = wave_digit_rank<kRadixBits>((key[r] >> shift) & (kRadix - 1), first + r * 64 < m, lane, wcount[wave]);
+    __syncthreads();
+    uint32_t cnt = 0;
+    for (int w = 0; w < kWaves; ++w) cnt += wcount[w][tid];
+    // exclusive scans over the digits of the totals (high half) and the tile's counts (low half)
+    uint64_t incl = ((uint64_t)total << 32) | cnt;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint64_t x = __shfl_up((unsigned long long)incl, off);
+        if (lane >= off) incl += x;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) incl += wsum[w];
+    uint32_t at = (uint32_t)incl - cnt;  // the digit's first LDS position
+    base[tid] = (uint32_t)(incl >> 32) - total + before - at;
+    for (int w = 0; w < kWaves; ++w) {
+        const uint32_t c = wcount[w][tid];
+        wcount[w][tid] = at;
+        at += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r) {
+        if (first + r * 64 < m) {
+            const uint32_t off = wcount[wave][(key[r] >> shift) & (kRadix - 1)] + rank[r];
+            sk[off] = key[r];
+            sv[off] = val[r];
+        }
+    }
+    __syncthreads();
     for (uint32_t j = tid; j < m; j += kSortThreads) {
-        const uint32_t key = sk[j];
-        const uint32_t d = (key >> shift) & (kRadix - 1);
-        const uint32_t off = base[d] + (j - lstart[d]);
+        const uint32_t k = sk[j];
+        const uint32_t off = base[(k >> shift) & (kRadix - 1)] + j;
         if (off < n) {  // always true for a consistent histogram; keeps writes in bounds
-            kout[off] = key;
+            kout[off] = k;
             vout[off] = sv[j];
         }
     }
