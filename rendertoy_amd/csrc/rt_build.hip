@@ -5,7 +5,7 @@
 //   1. gather      per mesh: read MeshVertex P/N/C (rendering/_modeling.py:22-28) through the
 //                  optional int32 index list, write unsorted tri/shade records, padded leaf box,
 //                  AABB centroid.
-//   2. bounds      two-stage min/max reduction of the centroids.
+//   2. bounds      min/max of the centroids per workgroup of the gather, folded by the next kernel.
 //   3. morton      30-bit Morton code of each centroid quantised to 1024^3 over those bounds.
 //   4. sort        stable LSD radix sort of (code, primitive) in 4 passes of 8 bits (rt_sort.h):
 //                  per-tile histogram -> per-digit row scan -> scatter, the scatter ranking keys
@@ -28,8 +28,6 @@
 
 namespace rt {
 namespace {
-
-constexpr int kReduceBlocks = 512;
 
 // LBVH tree: slots per workgroup of the local pass, and the most top boundaries of one block
 constexpr int kTreeBlock = 1024;
@@ -66,7 +64,7 @@ struct Workspace {
     uint32_t* vals1;
     uint32_t* hist;    // kRadix * nblk
     uint32_t* totals;  // kRadix
-    float* partial;    // kReduceBlocks * 8
+    float4* partial;   // 2 per workgroup of the gather: bounds of its centroids (the space of cbox[0])
     float* cbounds;    // 8
     int32_t* parent;   // (n-1) internal then n leaves
     // PLOC builder
@@ -110,7 +108,6 @@ Workspace carve(char* base, uint64_t n) {
     w.vals1 = (uint32_t*)take(4 * n);
     w.hist = (uint32_t*)take(4 * kRadix * (nblk ? nblk : 1));
     w.totals = (uint32_t*)take(4 * kRadix);
-    w.partial = (float*)take(4 * 8 * kReduceBlocks);
     w.cbounds = (float*)take(4 * 8);
     w.parent = (int32_t*)take(4 * (ni + n));
     const uint64_t nchunk = (n + 1023) / 1024 + 1;
@@ -118,6 +115,7 @@ Workspace carve(char* base, uint64_t n) {
         w.cid[k] = (int32_t*)take(4 * n);
         w.cbox[k] = (float4*)take(32 * n);
     }
+    w.partial = w.cbox[0];  // every workgroup of the gather has a triangle, so there are at most n
     w.nn = (int32_t*)take(4 * n);
     w.nleft = (int32_t*)take(4 * ni);
     w.nright = (int32_t*)take(4 * ni);
@@ -156,6 +154,58 @@ RT_DEV float3 load_f3(const char* base, uint64_t i, uint32_t stride, uint32_t of
     return make_float3(p[0], p[1], p[2]);
 }
 
+struct Box {
+    float lo[3], hi[3];
+};
+
+RT_DEV Box empty_box() {
+    return {{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
+}
+
+RT_DEV Box unite(const Box& a, const Box& b) {
+    Box u;
+    for (int c = 0; c < 3; ++c) {
+        u.lo[c] = fminf(a.lo[c], b.lo[c]);
+        u.hi[c] = fmaxf(a.hi[c], b.hi[c]);
+    }
+    return u;
+}
+
+RT_DEV Box load_box(const float4* __restrict__ p) {
+    const float4 a = p[0], b = p[1];
+    return {{a.x, a.y, a.z}, {b.x, b.y, b.z}};
+}
+
+RT_DEV void store_box(float4* __restrict__ p, const Box& b) {
+    p[0] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f);
+    p[1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.0f);
+}
+
+// Union over the wave's lanes, in every lane.
+RT_DEV Box wave_unite(Box b) {
+    for (int x = 1; x < 64; x <<= 1)
+        for (int c = 0; c < 3; ++c) {
+            b.lo[c] = fminf(b.lo[c], __shfl_xor(b.lo[c], x));
+            b.hi[c] = fmaxf(b.hi[c], __shfl_xor(b.hi[c], x));
+        }
+    return b;
+}
+
+// Union of parts[2 i] for i < count over a workgroup of T threads, in every thread; `lds` holds two
+// float4s per wave.
+template <int T>
+RT_DEV Box block_unite(const float4* __restrict__ parts, uint32_t count, float4* lds) {
+    Box b = empty_box();
+#pragma unroll 4
+    for (uint32_t i = threadIdx.x; i < count; i += T) b = unite(b, load_box(parts + 2 * (uint64_t)i));
+    b = wave_unite(b);
+    if ((threadIdx.x & 63) == 0) store_box(lds + 2 * (threadIdx.x >> 6), b);
+    __syncthreads();
+    b = load_box(lds);
+    for (int w = 1; w < T / 64; ++w) b = unite(b, load_box(lds + 2 * w));
+    return b;
+}
+
 // Copies `per` float4s of each of the block's `rows` records from LDS (record r at
 // stage[r * pitch]) to out[0 .. rows*per), one float4 per thread and instruction.
 RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t rows, uint32_t per,
@@ -169,22 +219,26 @@ RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t
 // One thread per triangle: positions (canonical zeros), the centroid, the padded leaf box, the
 // intersection record (p0, e1, e2, primitive id) and the shading record (three normals, three
 // uvs, mesh id). The block's records go out through LDS as consecutive float4s.
-__global__ void __launch_bounds__(256) k_gather(rt_mesh_desc m, uint32_t mesh_id,
+__global__ void __launch_bounds__(256) k_gather(rt_mesh_desc m, uint32_t mesh_id, uint32_t n_meshes,
                                                  uint32_t prim_base, float4* __restrict__ cent,
                                                  float4* __restrict__ leafbox,
                                                  float4* __restrict__ tri_u,
                                                  float4* __restrict__ shade_u,
-                                                 int32_t* __restrict__ mesh_offsets) {
+                                                 int32_t* __restrict__ mesh_offsets,
+                                                 float4* __restrict__ partial) {
     constexpr uint32_t kPitch = 5;  // float4s per staged record (4 used)
     __shared__ float4 stage[256 * kPitch];
+    __shared__ float4 wpart[4][2];
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) mesh_offsets[mesh_id] = (int32_t)prim_base;
+    if (t == 0 && mesh_id + 1 == n_meshes) mesh_offsets[n_meshes] = (int32_t)(prim_base + m.n_tris);
     const uint32_t t0 = blockIdx.x * blockDim.x;
     if (t0 >= m.n_tris) return;  // whole block (only the launch for an empty mesh)
     const uint32_t rows = m.n_tris - t0 < blockDim.x ? m.n_tris - t0 : blockDim.x;
     const uint64_t pb = (uint64_t)prim_base + t0;  // the block's first primitive
     const bool mine = t < m.n_tris;
     float4 box[2], tri[3], shd[4];
+    Box cb = empty_box();
     if (mine) {
         const char* vb = (const char*)m.vertices;
         uint32_t i0 = 3 * t, i1 = 3 * t + 1, i2 = 3 * t + 2;
@@ -208,7 +262,9 @@ __global__ void __launch_bounds__(256) k_gather(rt_mesh_desc m, uint32_t mesh_id
         const float lox = fminf(fminf(p0.x, p1.x), p2.x), hix = fmaxf(fmaxf(p0.x, p1.x), p2.x);
         const float loy = fminf(fminf(p0.y, p1.y), p2.y), hiy = fmaxf(fmaxf(p0.y, p1.y), p2.y);
         const float loz = fminf(fminf(p0.z, p1.z), p2.z), hiz = fmaxf(fmaxf(p0.z, p1.z), p2.z);
-        cent[p] = make_float4((lox + hix) * 0.5f, (loy + hiy) * 0.5f, (loz + hiz) * 0.5f, 0.0f);
+        const float cx = (lox + hix) * 0.5f, cy = (loy + hiy) * 0.5f, cz = (loz + hiz) * 0.5f;
+        cent[p] = make_float4(cx, cy, cz, 0.0f);
+        cb = unite(cb, {{cx, cy, cz}, {cx, cy, cz}});
         const float px = pad_of(lox, hix), py = pad_of(loy, hiy), pz = pad_of(loz, hiz);
         box[0] = make_float4(lox - px, loy - py, loz - pz, 0.0f);
         box[1] = make_float4(hix + px, hiy + py, hiz + pz, 0.0f);
@@ -246,9 +302,15 @@ __global__ void __launch_bounds__(256) k_gather(rt_mesh_desc m, uint32_t mesh_id
         shd[2] = make_float4(n2.z, uv0.x, uv0.y, uv1.x);
         shd[3] = make_float4(uv1.y, uv2.x, uv2.y, __int_as_float((int32_t)mesh_id));
     }
+    cb = wave_unite(cb);
+    if ((threadIdx.x & 63) == 0) store_box(wpart[threadIdx.x >> 6], cb);
     float4* st = stage + threadIdx.x * kPitch;
     if (mine) { st[0] = shd[0]; st[1] = shd[1]; st[2] = shd[2]; st[3] = shd[3]; }
     __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) cb = unite(cb, load_box(wpart[w]));
+        store_box(partial + 2 * (uint64_t)blockIdx.x, cb);
+    }
     store_staged(shade_u + 4 * pb, stage, rows, 4, kPitch);
     __syncthreads();
     if (mine) { st[0] = tri[0]; st[1] = tri[1]; st[2] = tri[2]; }
@@ -262,65 +324,6 @@ __global__ void __launch_bounds__(256) k_gather(rt_mesh_desc m, uint32_t mesh_id
 
 __global__ void k_mesh_offsets_tail(int32_t* mesh_offsets, uint32_t n_meshes, uint32_t n) {
     if (threadIdx.x == 0 && blockIdx.x == 0) mesh_offsets[n_meshes] = (int32_t)n;
-}
-
-// Stage 1: each block reduces a grid-stride share of the centroids to (min.xyz, max.xyz).
-__global__ void __launch_bounds__(256) k_bounds_partial(const float4* __restrict__ cent,
-                                                         uint32_t n, float* __restrict__ partial) {
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const float4 c = cent[i];
-        lo[0] = fminf(lo[0], c.x); lo[1] = fminf(lo[1], c.y); lo[2] = fminf(lo[2], c.z);
-        hi[0] = fmaxf(hi[0], c.x); hi[1] = fmaxf(hi[1], c.y); hi[2] = fmaxf(hi[2], c.z);
-    }
-    __shared__ float s[6][256];
-    for (int c = 0; c < 3; ++c) {
-        s[c][threadIdx.x] = lo[c];
-        s[3 + c][threadIdx.x] = hi[c];
-    }
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            for (int c = 0; c < 3; ++c) {
-                s[c][threadIdx.x] = fminf(s[c][threadIdx.x], s[c][threadIdx.x + w]);
-                s[3 + c][threadIdx.x] = fmaxf(s[3 + c][threadIdx.x], s[3 + c][threadIdx.x + w]);
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x < 6) partial[blockIdx.x * 8 + threadIdx.x] = s[threadIdx.x][0];
-}
-
-// Stage 2: one block folds the partials into (lo.xyz, scale.xyz) for the quantiser.
-__global__ void __launch_bounds__(256) k_bounds_final(const float* __restrict__ partial,
-                                                       int nparts, float* __restrict__ cb) {
-    __shared__ float s[6][256];
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int i = threadIdx.x; i < nparts; i += blockDim.x)
-        for (int c = 0; c < 3; ++c) {
-            lo[c] = fminf(lo[c], partial[i * 8 + c]);
-            hi[c] = fmaxf(hi[c], partial[i * 8 + 3 + c]);
-        }
-    for (int c = 0; c < 3; ++c) {
-        s[c][threadIdx.x] = lo[c];
-        s[3 + c][threadIdx.x] = hi[c];
-    }
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            for (int c = 0; c < 3; ++c) {
-                s[c][threadIdx.x] = fminf(s[c][threadIdx.x], s[c][threadIdx.x + w]);
-                s[3 + c][threadIdx.x] = fmaxf(s[3 + c][threadIdx.x], s[3 + c][threadIdx.x + w]);
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x < 3) {
-        const float l = s[threadIdx.x][0], h = s[3 + threadIdx.x][0];
-        const float ext = h - l;
-        cb[threadIdx.x] = l;
-        cb[4 + threadIdx.x] = ext > 0.0f ? 1024.0f / ext : 0.0f;
-    }
 }
 
 RT_DEV uint32_t expand10(uint32_t v) {
@@ -338,6 +341,28 @@ RT_DEV uint32_t quantize10(float c, float lo, float scale) {
     return (uint32_t)q;
 }
 
+RT_DEV float quantize_scale(float lo, float hi) {
+    const float ext = hi - lo;
+    return ext > 0.0f ? 1024.0f / ext : 0.0f;
+}
+
+RT_DEV uint32_t morton30(float x, float y, float z, const float* lo, const float* scale) {
+    return (expand10(quantize10(x, lo[0], scale[0])) << 2) | (expand10(quantize10(y, lo[1], scale[1])) << 1) |
+           expand10(quantize10(z, lo[2], scale[2]));
+}
+
+// One block folds the gather's bounds of 256 centroids each into (lo.xyz, scale.xyz) for the quantiser.
+__global__ void __launch_bounds__(1024) k_bounds_final(const float4* __restrict__ partial, uint32_t nparts,
+                                                       float* __restrict__ cb) {
+    __shared__ float4 lds[2 * 1024 / 64];
+    const Box b = block_unite<1024>(partial, nparts, lds);
+    if (threadIdx.x == 0)
+        for (int a = 0; a < 3; ++a) {
+            cb[a] = b.lo[a];
+            cb[4 + a] = quantize_scale(b.lo[a], b.hi[a]);
+        }
+}
+
 __global__ void __launch_bounds__(256) k_morton(const float4* __restrict__ cent, uint32_t n,
                                                  const float* __restrict__ cb,
                                                  uint32_t* __restrict__ keys,
@@ -345,25 +370,129 @@ __global__ void __launch_bounds__(256) k_morton(const float4* __restrict__ cent,
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float4 c = cent[i];
-    const uint32_t qx = quantize10(c.x, cb[0], cb[4]);
-    const uint32_t qy = quantize10(c.y, cb[1], cb[5]);
-    const uint32_t qz = quantize10(c.z, cb[2], cb[6]);
-    keys[i] = (expand10(qx) << 2) | (expand10(qy) << 1) | expand10(qz);
+    keys[i] = morton30(c.x, c.y, c.z, cb, cb + 4);
     vals[i] = i;
+}
+
+// Order of a scene of at most kSmallMax triangles in two launches. k_order_chunks: a workgroup folds
+// the gather's bounds for itself, and codes and sorts its kOrderChunk triangles by counting
+// smaller keys. k_order_merge: a pair's place is its place in its chunk plus, for every other chunk,
+// a binary search in LDS; each of 4 waves takes a quarter of the chunks for the same 64 pairs.
+// Equal codes keep their order: they count as smaller in chunks before the pair's own.
+// The general path's 14 launches of codes and radix passes run up to 6 workgroups each at 11,560
+// triangles and take 58 us of kernel time, these two take 13; one workgroup that held all pairs and made
+// the four radix passes in LDS took 44, bound by the ballots of its 16 waves. The limit is the LDS that
+// holds all codes: at 32,000 triangles these take 30 us, the general path 59 at 33,620.
+constexpr uint32_t kOrderChunk = 256;
+constexpr uint32_t kSmallMax = 32 * 1024;
+
+__global__ void __launch_bounds__(kOrderChunk) k_order_chunks(const float4* __restrict__ cent, uint32_t n,
+                                                              const float4* __restrict__ partial,
+                                                              uint32_t nparts, uint32_t* __restrict__ keys,
+                                                              uint32_t* __restrict__ vals) {
+    constexpr int kWaves = kOrderChunk / 64;
+    __shared__ float4 lds[2 * kWaves];
+    __shared__ uint4 sk[kOrderChunk / 4];
+    const uint32_t tid = threadIdx.x;
+    const int wave = tid >> 6;
+    const Box b = block_unite<kOrderChunk>(partial, nparts, lds);
+    float scale[3];
+    for (int a = 0; a < 3; ++a) scale[a] = quantize_scale(b.lo[a], b.hi[a]);
+    const uint32_t i = blockIdx.x * kOrderChunk + tid;
+    uint32_t key = 0xFFFFFFFFu;  // past the end: above every code
+    if (i < n) {
+        const float4 c = cent[i];
+        key = morton30(c.x, c.y, c.z, b.lo, scale);
+    }
+    ((uint32_t*)sk)[tid] = key;
+    __syncthreads();
+    uint32_t rank = 0;
+    // four keys a step; equal ones count before this thread's own
+#pragma unroll 8
+    for (int j = 0; j < 16 * wave; ++j) {
+        const uint4 q = sk[j];
+        rank += (uint32_t)(q.x <= key) + (uint32_t)(q.y <= key) + (uint32_t)(q.z <= key) + (uint32_t)(q.w <= key);
+    }
+#pragma unroll 8
+    for (int j = 16 * wave; j < 16 * (wave + 1); ++j) {
+        const uint4 q = sk[j];
+        const uint32_t j0 = 4 * (uint32_t)j;
+        rank += (uint32_t)(q.x < key + (j0 < tid)) + (uint32_t)(q.y < key + (j0 + 1 < tid)) +
+                (uint32_t)(q.z < key + (j0 + 2 < tid)) + (uint32_t)(q.w < key + (j0 + 3 < tid));
+    }
+#pragma unroll 8
+    for (int j = 16 * (wave + 1); j < 16 * kWaves; ++j) {
+        const uint4 q = sk[j];
+        rank += (uint32_t)(q.x < key) + (uint32_t)(q.y < key) + (uint32_t)(q.z < key) + (uint32_t)(q.w < key);
+    }
+    if (i < n) {
+        keys[i - tid + rank] = key;
+        vals[i - tid + rank] = i;
+    }
+}
+
+template <uint32_t kMax>
+__global__ void __launch_bounds__(256) k_order_merge(const uint32_t* __restrict__ kin,
+                                                     const uint32_t* __restrict__ vin, uint32_t n,
+                                                     uint32_t* __restrict__ keys,
+                                                     uint32_t* __restrict__ order) {
+    __shared__ uint32_t sk[kMax];
+    __shared__ uint32_t part[4][64];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t chunks = (n + kOrderChunk - 1) / kOrderChunk;
+    for (uint32_t i0 = tid; i0 < chunks * kOrderChunk; i0 += 32 * 256) {  // 32 loads in flight
+        uint32_t v[32];
+#pragma unroll
+        for (int q = 0; q < 32; ++q) v[q] = i0 + q * 256 < n ? kin[i0 + q * 256] : 0xFFFFFFFFu;
+#pragma unroll
+        for (int q = 0; q < 32; ++q) sk[i0 + q * 256] = v[q];  // kMax is a multiple of the 8,192 of a round
+    }
+    const uint32_t i = blockIdx.x * 64 + lane;
+    const uint32_t val = wave == 0 && i < n ? vin[i] : 0u;
+    __syncthreads();
+    const uint32_t own = blockIdx.x * 64 / kOrderChunk;
+    const uint32_t key = sk[i];  // blocks cover whole chunks at most
+    uint32_t rank = 0;
+    for (uint32_t c0 = wave; c0 < chunks; c0 += 16) {  // four searches at a time hide each other's LDS latency
+        uint32_t at[4] = {0, 0, 0, 0}, k[4];
+        const uint32_t* a[4];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint32_t c = c0 + 4 * q;
+            k[q] = c >= chunks || c == own ? 0u : c < own ? key + 1 : key;  // count codes below k (30 bits)
+            a[q] = sk + (c < chunks ? c : 0u) * kOrderChunk;
+        }
+#pragma unroll
+        for (uint32_t step = kOrderChunk / 2; step; step >>= 1)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) at[q] += a[q][at[q] + step - 1] < k[q] ? step : 0u;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) rank += at[q] + (a[q][at[q]] < k[q] ? 1u : 0u);
+    }
+    part[wave][lane] = rank;
+    __syncthreads();
+    if (wave == 0 && i < n) {
+        const uint32_t at = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane] + i % kOrderChunk;
+        keys[at] = key;
+        order[at] = val;
+    }
 }
 
 // One thread per float4 of the outputs: thread x copies shade float4 x (record x/4) and, for
 // x < 3n, tris float4 x (record x/3), so each store instruction writes consecutive 16 B pieces
-// and each record's source is read as consecutive pieces by neighbouring lanes.
+// and each record's source is read as consecutive pieces by neighbouring lanes. Also the slot of each
+// primitive.
 __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order, uint32_t n,
                                               const float4* __restrict__ tri_u,
                                               const float4* __restrict__ shade_u,
                                               float4* __restrict__ tris,
-                                              float4* __restrict__ shade) {
+                                              float4* __restrict__ shade,
+                                              uint32_t* __restrict__ prim_slot) {
     const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= 4 * (uint64_t)n) return;
     const uint64_t ps = order[x >> 2];
     shade[x] = shade_u[4 * ps + (x & 3)];
+    if ((x & 3) == 0) prim_slot[ps] = (uint32_t)(x >> 2);
     if (x < 3 * (uint64_t)n) {
         const uint64_t s = x / 3;
         tris[x] = tri_u[3 * (uint64_t)order[s] + (x - 3 * s)];
@@ -393,10 +522,6 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order
 // At 1.31 M triangles 72 us for the local pass and 25 for the top; separate kernels for the hierarchy
 // (binary searches in memory, 93 us), a refit over its arrays (142), a sparse table of block unions
 // (17) and the top refit (10) took 262. At 11,560 triangles 25 us against 61.
-struct Box {
-    float lo[3], hi[3];
-};
-
 // length of the common prefix of the extended keys (a, i) and (b, j)
 RT_DEV int key_prefix(uint32_t a, uint32_t b, int64_t i, int64_t j) {
     return a != b ? __clz(a ^ b) : 32 + __clz((uint32_t)i ^ (uint32_t)j);
@@ -405,29 +530,6 @@ RT_DEV int key_prefix(uint32_t a, uint32_t b, int64_t i, int64_t j) {
 // common prefix of slots p - 1 and p; -1 at the scene's ends
 RT_DEV int diff_at(const uint32_t* __restrict__ keys, int64_t n, int64_t p) {
     return p <= 0 || p >= n ? -1 : key_prefix(keys[p - 1], keys[p], p - 1, p);
-}
-
-RT_DEV Box empty_box() {
-    return {{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
-}
-
-RT_DEV Box unite(const Box& a, const Box& b) {
-    Box u;
-    for (int c = 0; c < 3; ++c) {
-        u.lo[c] = fminf(a.lo[c], b.lo[c]);
-        u.hi[c] = fmaxf(a.hi[c], b.hi[c]);
-    }
-    return u;
-}
-
-RT_DEV Box load_box(const float4* __restrict__ p) {
-    const float4 a = p[0], b = p[1];
-    return {{a.x, a.y, a.z}, {b.x, b.y, b.z}};
-}
-
-RT_DEV void store_box(float4* __restrict__ p, const Box& b) {
-    p[0] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f);
-    p[1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.0f);
 }
 
 // Record of node `id` with slots [lo, hi1) split at boundary p; a child of at most kLeafMax slots
@@ -598,11 +700,7 @@ RT_DEV Box wave_range_box(const TopArrays& top, int64_t lo, int64_t hi1, uint32_
     if (hi1 != (int64_t)n && hi1 % kTreeBlock) b = unite(b, load_box(top.pre + 2 * (uint64_t)hi1));
     if (b0 < b1) {
         for (int64_t k = b0 + lane; k < b1; k += 64) b = unite(b, load_box(top.block + 2 * (uint64_t)k));
-        for (int x = 1; x < 64; x <<= 1)
-            for (int c = 0; c < 3; ++c) {
-                b.lo[c] = fminf(b.lo[c], __shfl_xor(b.lo[c], x));
-                b.hi[c] = fmaxf(b.hi[c], __shfl_xor(b.hi[c], x));
-            }
+        b = wave_unite(b);
     }
     return b;
 }
@@ -1348,13 +1446,6 @@ __global__ void k_export_empty(float4* __restrict__ out, uint32_t* __restrict__ 
     }
 }
 
-// prim_slot[order[s]] = s: the triangle-record slot of each global primitive id
-__global__ void __launch_bounds__(256) k_prim_slot(const uint32_t* __restrict__ order, uint32_t n,
-                                                        uint32_t* __restrict__ inv) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n) inv[order[s]] = s;
-}
-
 // BVH_Triangle records (64 B as 4 float4: v0, v1, v2, (index, mesh, 0, 0)) of mesh m, written at
 // the slot of each triangle; vertex indices are clamped to n_vertices - 1 as the build does.
 __global__ void __launch_bounds__(256) k_export_tris(rt_mesh_desc d, uint32_t m, uint32_t base,
@@ -1444,27 +1535,32 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
     Workspace w = carve((char*)workspace, n);
 
     // 1. gather (one launch per mesh; the descriptor travels as a kernel argument)
-    uint32_t base = 0;
+    uint32_t base = 0, nparts = 0;
     for (uint32_t m = 0; m < n_meshes; ++m) {
         const rt_mesh_desc& d = meshes[m];
         hipLaunchKernelGGL(k_gather, dim3(d.n_tris ? blocks_for(d.n_tris, 256) : 1), dim3(256), 0, s,
-                           d, m, base, w.cent, w.leafbox, w.tri_u, w.shade_u, sc->mesh_offsets);
+                           d, m, n_meshes, base, w.cent, w.leafbox, w.tri_u, w.shade_u, sc->mesh_offsets,
+                           w.partial + 2 * (uint64_t)nparts);
         base += d.n_tris;
+        nparts += blocks_for(d.n_tris, 256);
     }
-    hipLaunchKernelGGL(k_mesh_offsets_tail, dim3(1), dim3(1), 0, s, sc->mesh_offsets, n_meshes, n);
-    // 2. centroid bounds
-    const int nparts = (int)std::min<uint32_t>(kReduceBlocks, blocks_for(n, 256));
-    hipLaunchKernelGGL(k_bounds_partial, dim3(nparts), dim3(256), 0, s, w.cent, n, w.partial);
-    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(256), 0, s, w.partial, nparts, w.cbounds);
-    // 3. Morton codes
-    hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, 256)), dim3(256), 0, s, w.cent, n, w.cbounds,
-                       w.keys0, w.vals0);
-    // 4. radix sort, 4 passes over the 30-bit keys
-    uint32_t *ki = w.keys0, *vi = w.vals0;
-    sort_pairs(ki, vi, w.keys1, w.vals1, n, 30, w.hist, w.totals, s);
-    // after 4 passes the sorted arrays are back in keys0/vals0
-    float4* nodes = (float4*)sc->nodes;
+    // 2. - 4. centroid bounds, Morton codes and their sort, into the caller's arrays where it wants them
+    // (PLOC writes the order of its own slots there)
     bool ploc = n > 1 && tu.builder == RT_BUILD_PLOC;
+    uint32_t* ki = keys_out ? keys_out : w.keys0;
+    uint32_t* vi = order_out && !ploc ? order_out : w.vals0;
+    if (n <= kSmallMax) {
+        hipLaunchKernelGGL(k_order_chunks, dim3(blocks_for(n, kOrderChunk)), dim3(kOrderChunk), 0, s, w.cent, n,
+                           w.partial, nparts, w.keys1, w.vals1);
+        hipLaunchKernelGGL(n <= kSmallMax / 2 ? k_order_merge<kSmallMax / 2> : k_order_merge<kSmallMax>,
+                           dim3(blocks_for(n, 64)), dim3(256), 0, s, w.keys1, w.vals1, n, ki, vi);
+    } else {
+        hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(1024), 0, s, w.partial, nparts, w.cbounds);
+        hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, 256)), dim3(256), 0, s, w.cent, n, w.cbounds,
+                           w.keys0, w.vals0);
+        sort_pairs(w.keys0, w.vals0, w.keys1, w.vals1, ki, vi, n, 30, w.hist, w.totals, s);
+    }
+    float4* nodes = (float4*)sc->nodes;
     const uint32_t nchunk = blocks_for(n, kPlocChunk);
     if (ploc) {
         // 5. PLOC hierarchy (node boxes as it merges, scene bounds at the root), 6. leaf slots and
@@ -1495,27 +1591,29 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
         if (!e) e = check_hip(hipStreamSynchronize(s), "rt_scene_build(PLOC depth)");
         if (e) return e;
         ploc = deep == 0;
+        if (!ploc && order_out)
+            hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, order_out, n);
     }
     if (ploc) {
+        uint32_t* slot_order = order_out ? order_out : w.slot_order;
         hipLaunchKernelGGL(k_ploc_leafroots, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, vi, w.parent,
                            w.nsize, w.nleft, w.nright, w.pos_of, w.scan);
         hipLaunchKernelGGL(k_scan_chunks, dim3(nchunk), dim3(256), 0, s, n, w.scan, w.part);
         hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, nchunk, w.part);
         hipLaunchKernelGGL(k_scan_apply, dim3(nchunk), dim3(256), 0, s, n, w.scan, w.part);
         hipLaunchKernelGGL(k_ploc_slots, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, vi, w.parent,
-                           w.nsize, w.nleft, w.nright, w.pos_of, w.scan, w.slot_order, w.slot_of, w.fslot);
+                           w.nsize, w.nleft, w.nright, w.pos_of, w.scan, slot_order, w.slot_of, w.fslot);
         hipLaunchKernelGGL(k_ploc_refs, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n, w.nleft,
                            w.nright, w.nsize, w.slot_of, w.fslot, nodes);
-        hipLaunchKernelGGL(k_emit, dim3(blocks_for(4 * (uint64_t)n, 256)), dim3(256), 0, s, w.slot_order, n, w.tri_u,
-                           w.shade_u, (float4*)sc->tris, (float4*)sc->shade);
+        hipLaunchKernelGGL(k_emit, dim3(blocks_for(4 * (uint64_t)n, 256)), dim3(256), 0, s, slot_order, n, w.tri_u,
+                           w.shade_u, (float4*)sc->tris, (float4*)sc->shade, (uint32_t*)sc->prim_slot);
         hipLaunchKernelGGL(k_wide, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n,
                            (const float4*)nodes, (float4*)sc->nodes4);
         sc->root = n <= (uint32_t)kLeafMax ? leaf_ref(0, n) : 0;
-        vi = w.slot_order;
     } else {
     // 5. emit, 6. tree (LBVH, or a PLOC tree found too deep)
     hipLaunchKernelGGL(k_emit, dim3(blocks_for(4 * (uint64_t)n, 256)), dim3(256), 0, s, vi, n, w.tri_u, w.shade_u,
-                       (float4*)sc->tris, (float4*)sc->shade);
+                       (float4*)sc->tris, (float4*)sc->shade, (uint32_t*)sc->prim_slot);
     if (n > 1) {
         const uint32_t nb = blocks_for(n, kTreeBlock);
         hipLaunchKernelGGL(k_tree_local, dim3(nb), dim3(kTreeBlock), 0, s, ki, vi, n, w.leafbox, nodes,
@@ -1529,12 +1627,6 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
         sc->root = ~0;
     }
     }
-    hipLaunchKernelGGL(k_prim_slot, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, n,
-                       (uint32_t*)sc->prim_slot);
-    if (keys_out)
-        hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, ki, keys_out, n);
-    if (order_out)
-        hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, order_out, n);
     return check_launch("rt_scene_build");
 }
 

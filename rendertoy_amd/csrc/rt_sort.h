@@ -1,11 +1,9 @@
 // rt_sort.h — stable LSD radix sort of (uint32 key, uint32 value) pairs on the device, used by the
-// scene build (Morton codes) and by the per-vertex normals (vertex ids). Each pass of 8 bits is a
-// per-tile histogram -> per-digit row scan -> scatter; the scatter block scans the 256 digit totals
-// itself, ranks keys with wave64 ballot/mbcnt multi-split so equal digits keep input order, groups
-// its tile by digit in LDS and writes each digit's run of the tile contiguously.
+// scene build (Morton codes). Each pass of 8 bits is a per-tile histogram -> per-digit row scan ->
+// scatter; the scatter block scans the 256 digit totals itself, ranks keys with wave64 ballot/mbcnt
+// multi-split so equal digits keep input order, groups its tile by digit in LDS and writes each
+// digit's run of the tile contiguously.
 #pragma once
-
-#include <utility>
 
 #include "rt_common.h"
 
@@ -165,19 +163,21 @@ inline uint64_t sort_hist_bytes(uint64_t n) {
     return 4ull * kRadix * (nblk ? nblk : 1);
 }
 
-// Sorts n pairs by the low `bits` bits of the keys in ceil(bits / 8) passes, ping-ponging between
-// (ki, vi) and (ko, vo); on return ki/vi point at the sorted arrays. hist: sort_hist_bytes(n),
-// totals: kRadix words.
-inline void sort_pairs(uint32_t*& ki, uint32_t*& vi, uint32_t* ko, uint32_t* vo, uint32_t n, int bits,
-                       uint32_t* hist, uint32_t* totals, hipStream_t s) {
+// Sorts n pairs (k0, v0) by the low `bits` bits of the keys in an even number of passes, ceil(bits / 8),
+// ping-ponging over (k1, v1); the last pass writes (kout, vout), which may be (k0, v0). hist:
+// sort_hist_bytes(n), totals: kRadix words.
+inline void sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint32_t* kout, uint32_t* vout,
+                       uint32_t n, int bits, uint32_t* hist, uint32_t* totals, hipStream_t s) {
     const uint32_t nblk = (uint32_t)((n + kSortTile - 1) / kSortTile);
     for (int shift = 0; shift < bits; shift += kRadixBits) {
+        const bool odd = (shift / kRadixBits) & 1, last = shift + kRadixBits >= bits;
+        const uint32_t *ki = odd ? k1 : k0, *vi = odd ? v1 : v0;
+        uint32_t* ko = last ? kout : odd ? k0 : k1;
+        uint32_t* vo = last ? vout : odd ? v0 : v1;
         hipLaunchKernelGGL(k_sort_hist, dim3(nblk), dim3(kSortThreads), 0, s, ki, n, shift, hist, nblk);
         hipLaunchKernelGGL(k_sort_rowscan, dim3(kRadix), dim3(kSortThreads), 0, s, hist, nblk, totals);
         hipLaunchKernelGGL(k_sort_scatter, dim3(nblk), dim3(kSortThreads), 0, s, ki, vi, n, shift, hist,
                            totals, nblk, ko, vo);
-        std::swap(ki, ko);
-        std::swap(vi, vo);
     }
 }
 

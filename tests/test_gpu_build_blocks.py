@@ -26,3 +26,11 @@ def _mesh(n, kind):
 def test_block_edges(ren, n, kind):
     meshes = [_mesh(n, kind)]
     assert_build_equal(gpu_from_meshes(meshes), twin_from_meshes(meshes))
+
+
+@pytest.mark.parametrize("kind", ["spread", "equal", "crowded"])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 16384, 16385, 32767, 32768, 32769, 40961])
+def test_small_order(ren, n, kind):
+    """Order by chunks of 256 and merge by search (up to 32,768 triangles), and by radix passes from there."""
+    meshes = [_mesh(n, kind)]
+    assert_build_equal(gpu_from_meshes(meshes), twin_from_meshes(meshes))
