@@ -519,7 +519,7 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order
 // What bounds it: LDS round trips per level of a walk (10 to 17 levels), and 64 B per node of stores
 // in pieces of 16 B; 37 KB of LDS and one slot per thread put two
 // workgroups on a CU.
-// At 1.31 M triangles 72 us for the local pass and 25 for the top; separate kernels for the hierarchy
+// At 1.31 M triangles 67 us for the local pass and 25 for the top; separate kernels for the hierarchy
 // (binary searches in memory, 93 us), a refit over its arrays (142), a sparse table of block unions
 // (17) and the top refit (10) took 262. At 11,560 triangles 25 us against 61.
 // length of the common prefix of the extended keys (a, i) and (b, j)
@@ -563,7 +563,9 @@ __global__ void __launch_bounds__(kTreeBlock) k_tree_local(const uint32_t* __res
     __shared__ int32_t other[kTreeBlock];  // and the end of its slots that is not its id
     __shared__ uint32_t arrived[kTreeBlock];
     __shared__ int32_t diff[kTreeBlock + 1];
-    __shared__ int32_t seg[kTopMax + 2];
+    __shared__ int32_t seg[kTopMax + 2];   // segment starts, then the block's end
+    __shared__ int32_t sdiff[kTopMax + 2];  // diff there
+    __shared__ float sbox[kTopMax + 2][6];
     __shared__ int32_t nseg;
     const int64_t blo = (int64_t)blockIdx.x * kTreeBlock;
     const int cnt = (int)(n - blo < kTreeBlock ? n - blo : kTreeBlock);
@@ -651,27 +653,41 @@ __global__ void __launch_bounds__(kTreeBlock) k_tree_local(const uint32_t* __res
     const int m = nseg;
     const int first = blo == 0 ? 1 : 0;  // boundary 0 of the scene is no node's split
     if (tid == 0) top.count[blockIdx.x] = (uint32_t)(m - first);
-    if (tid >= m) return;
-    auto seg_id = [&](int j) { return diff[seg[j]] > diff[seg[j + 1]] ? seg[j] : seg[j + 1] - 1; };
-    const int j = tid, p = seg[j], d = diff[p];
-    const Box own = get(seg_id(j));
-    if (d > diff[seg[j + 1]])
-        store_box(top.child + 4 * (uint64_t)(blo + p) + 2, own);
-    else
-        store_box(top.child + 4 * (uint64_t)(blo + seg[j + 1]), own);
+    const int j = tid, p = j <= m ? seg[j] : 0, d = diff[p];
+    const bool is = j < m;
+    Box own = empty_box();
+    if (j <= m) sdiff[j] = d;
+    if (is) {
+        const int end = seg[j + 1], de = diff[end];
+        own = get(d > de ? p : end - 1);
+        store_box(top.child + 4 * (uint64_t)(d > de ? blo + p : blo + end) + (d > de ? 2 : 0), own);
+        for (int c = 0; c < 3; ++c) {
+            sbox[j][c] = own.lo[c];
+            sbox[j][3 + c] = own.hi[c];
+        }
+    }
+    __syncthreads();
+    if (!is) return;
     Box pre = empty_box(), suf = empty_box();
-    for (int i = 0; i < j; ++i) pre = unite(pre, get(seg_id(i)));
-    for (int i = j; i < m; ++i) suf = unite(suf, get(seg_id(i)));
+    TopEntry t{(int32_t)(blo + p), -1, -1, d, keys[blo + p], {}};
+#pragma unroll 2
+    for (int i = 0; i < m; ++i) {
+        const Box b = {{sbox[i][0], sbox[i][1], sbox[i][2]}, {sbox[i][3], sbox[i][4], sbox[i][5]}};
+        if (i < j)
+            pre = unite(pre, b);
+        else
+            suf = unite(suf, b);
+        const bool less = sdiff[i] < d;
+        if (i < j && less) t.lo = seg[i];  // the last one before j
+        if (i > j && less && t.hi1 < 0) t.hi1 = seg[i];
+    }
+    if (t.hi1 < 0 && sdiff[m] < d) t.hi1 = cnt;
+    if (t.lo >= 0) t.lo += (int32_t)blo;
+    if (t.hi1 >= 0) t.hi1 += (int32_t)blo;
     store_box(top.pre + 2 * (uint64_t)(blo + p), pre);
     store_box(top.suf + 2 * (uint64_t)(blo + p), suf);
     if (j == 0) store_box(top.block + 2 * (uint64_t)blockIdx.x, suf);
-    if (j < first) return;
-    TopEntry t{(int32_t)(blo + p), -1, -1, d, keys[blo + p], {}};
-    for (int i = j - 1; i >= 0 && t.lo < 0; --i)
-        if (diff[seg[i]] < d) t.lo = (int32_t)(blo + seg[i]);
-    for (int i = j + 1; i <= m && t.hi1 < 0; ++i)
-        if (diff[seg[i]] < d) t.hi1 = (int32_t)(blo + seg[i]);
-    top.list[(uint64_t)blockIdx.x * kTopMax + (j - first)] = t;
+    if (j >= first) top.list[(uint64_t)blockIdx.x * kTopMax + (j - first)] = t;
 }
 
 // The first x in [a, b] for which pred(x) holds, with pred(b) true and pred monotone, by all 64 lanes:
