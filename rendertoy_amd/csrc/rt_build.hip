@@ -78,8 +78,8 @@ struct Workspace {
     uint32_t* slot_of; // n: slot of each primitive
     uint32_t* fslot;   // n-1: first slot of each internal node inside a leaf
     uint32_t* scan;    // n: leaf-root sizes at their first Morton position, then their first slot
-    uint32_t* part;    // 2 * chunks: per-chunk counts, then exclusive offsets
-    int32_t* state;    // 8: PlocState per iteration parity
+    uint32_t* part;    // per tile or chunk: counts, then the slot scan's offsets
+    int32_t* state;    // 8: cluster count, nodes created and buffer per iteration parity
     uint32_t* depth;   // 1: internal ancestors of the deepest triangle of the PLOC tree
     TopArrays top;     // boundaries whose nodes span several tree blocks
     uint32_t* slot_order;  // n: primitive of each slot
@@ -110,7 +110,6 @@ Workspace carve(char* base, uint64_t n) {
     w.totals = (uint32_t*)take(4 * kRadix);
     w.cbounds = (float*)take(4 * 8);
     w.parent = (int32_t*)take(4 * (ni + n));
-    const uint64_t nchunk = (n + 1023) / 1024 + 1;
     for (int k = 0; k < 2; ++k) {
         w.cid[k] = (int32_t*)take(4 * n);
         w.cbox[k] = (float4*)take(32 * n);
@@ -124,7 +123,7 @@ Workspace carve(char* base, uint64_t n) {
     w.slot_of = (uint32_t*)take(4 * n);
     w.fslot = (uint32_t*)take(4 * ni);
     w.scan = (uint32_t*)take(4 * n);
-    w.part = (uint32_t*)take(8 * nchunk);
+    w.part = (uint32_t*)take(4 * ((n + 255) / 256));
     w.state = (int32_t*)take(4 * 8);
     w.depth = (uint32_t*)take(4);
     const uint64_t nb = (n + kTreeBlock - 1) / kTreeBlock;
@@ -776,21 +775,19 @@ __global__ void __launch_bounds__(256) k_ploc_depth(uint32_t n, const int32_t* _
 // merge into a new node kept at the lower position, the higher one drops out, survivors keep their
 // order. An iteration with no mutual pair (possible only with NaN boxes) merges positions 0 and 1.
 // The k-th node created (over iterations, in position order) gets id n-2-k: the root is 0 and
-// children have larger ids than their parents. Large iterations run as four grid launches
-// (neighbours; per-chunk counts; chunk offsets and the next cluster count; compaction); once at
-// most kPlocTail clusters remain, one workgroup finishes in a single launch. Subtrees of at most
+// children have larger ids than their parents. Large iterations run as two grid launches
+// (the pairs and their counts per tile; compaction), which took 297 us of a build of 151,380 triangles
+// where four (neighbours, counts, offsets, compaction) took 598; once at most kPlocTail clusters remain,
+// one workgroup finishes in a single launch. Subtrees of at most
 // kLeafMax triangles whose parent is larger become leaves: leaf roots take consecutive slot ranges
 // in the order of their smallest Morton position, their triangles left to right.
 constexpr int kPlocRadius = 16;
 constexpr int kPlocTile = 256;        // clusters per neighbour-search tile (one per thread)
-constexpr int kPlocChunk = 1024;      // clusters per count / compaction chunk (4 per thread)
+constexpr int kPlocChunk = 1024;      // values per chunk of the slot scan (4 per thread)
 constexpr int kPlocGrid = 1024;       // blocks of the grid-stride iteration kernels
 constexpr int32_t kPlocTail = 4096;   // cluster count handed to the one-workgroup tail
 
-// state[4 * parity]: clusters m, nodes created, forced merge, buffer parity of the clusters
-struct PlocState {
-    int32_t m, created, forced, buf;
-};
+// state[4 * parity]: clusters m, nodes created, buffer parity of the clusters
 
 RT_DEV float union_area(const float4& alo, const float4& ahi, const float4& blo, const float4& bhi) {
     const float dx = fmaxf(ahi.x, bhi.x) - fminf(alo.x, blo.x);
@@ -818,7 +815,6 @@ __global__ void __launch_bounds__(256) k_ploc_init(const uint32_t* __restrict__ 
         state[0] = (int32_t)n;
         state[1] = 0;
         state[2] = 0;
-        state[3] = 0;
     }
 }
 
@@ -844,35 +840,56 @@ RT_DEV int32_t ploc_nn(int32_t i, int32_t m, BoxAt box) {
     return bj;
 }
 
-__global__ void __launch_bounds__(kPlocTile) k_ploc_nn(int it, const int32_t* __restrict__ state,
-                                                        const float4* __restrict__ cbox0,
-                                                        const float4* __restrict__ cbox1,
-                                                        int32_t* __restrict__ nn) {
+// First kernel of an iteration: the mutual pairs of a tile of kPlocTile positions. The neighbours of the
+// kPlocRadius positions on either side are searched again here, so that a pair is known without another
+// launch. mate[i] is the position i merges with, or -1; part[tile] = positions kept | merges << 16.
+// 33 union boxes per position make it VALU work: 2.4 us for 150,000 positions, behind a launch's latency.
+constexpr int kPlocLoad = kPlocTile + 4 * kPlocRadius;  // boxes a tile's searches read, one per thread
+
+__global__ void __launch_bounds__(kPlocLoad) k_ploc_pairs(int it, const int32_t* __restrict__ state,
+                                                          const float4* __restrict__ cbox0,
+                                                          const float4* __restrict__ cbox1,
+                                                          int32_t* __restrict__ mate,
+                                                          uint32_t* __restrict__ part) {
     const int32_t m = state[4 * (it & 1)];
     if (m <= kPlocTail) return;
     const float4* __restrict__ B = (it & 1) ? cbox1 : cbox0;
-    __shared__ float4 wlo[kPlocTile + 2 * kPlocRadius], whi[kPlocTile + 2 * kPlocRadius];
-    for (int32_t base = blockIdx.x * kPlocTile; base < m; base += gridDim.x * kPlocTile) {
-        const int32_t wb = base - kPlocRadius;
-        for (int k = threadIdx.x; k < kPlocTile + 2 * kPlocRadius; k += kPlocTile) {
-            const int32_t g = wb + k;
-            if (g >= 0 && g < m) {
-                wlo[k] = B[2 * (uint64_t)g];
-                whi[k] = B[2 * (uint64_t)g + 1];
-            }
+    __shared__ float4 wlo[kPlocLoad], whi[kPlocLoad];
+    __shared__ int32_t nn[kPlocTile + 2 * kPlocRadius];
+    __shared__ uint32_t wcount[kPlocTile / 64];
+    const int32_t t = threadIdx.x, ntile = (m + kPlocTile - 1) / kPlocTile;
+    for (int32_t tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        const int32_t nb = tile * kPlocTile - kPlocRadius, wb = nb - kPlocRadius;
+        if (wb + t >= 0 && wb + t < m) {
+            wlo[t] = B[2 * (uint64_t)(wb + t)];
+            whi[t] = B[2 * (uint64_t)(wb + t) + 1];
         }
         __syncthreads();
-        const int32_t i = base + (int32_t)threadIdx.x;
-        if (i < m)
-            nn[i] = ploc_nn(i, m, [&](int32_t j, float4& lo, float4& hi) {
+        if (t < kPlocTile + 2 * kPlocRadius && nb + t >= 0 && nb + t < m)
+            nn[t] = ploc_nn(nb + t, m, [&](int32_t j, float4& lo, float4& hi) {
                 lo = wlo[j - wb];
                 hi = whi[j - wb];
             });
         __syncthreads();
+        if (t < kPlocTile) {
+            const int32_t i = tile * kPlocTile + t;
+            bool keep = false, merge = false;
+            if (i < m) {
+                const int32_t j = nn[i - nb];
+                const bool mutual = nn[j - nb] == i;
+                keep = !mutual || i < j;
+                merge = mutual && i < j;
+                mate[i] = mutual ? j : -1;
+            }
+            const uint32_t c = (uint32_t)__popcll(__ballot(keep)) | ((uint32_t)__popcll(__ballot(merge)) << 16);
+            if ((t & 63) == 0) wcount[t >> 6] = c;
+        }
+        __syncthreads();
+        if (t == 0) part[tile] = wcount[0] + wcount[1] + wcount[2] + wcount[3];
     }
 }
 
-// keep / merge flags of position i (forced: the iteration's fallback merge of 0 and 1)
+// keep / merge flags of position i from the neighbours nn (forced: the fallback merge of 0 and 1)
 RT_DEV void ploc_flags(const int32_t* __restrict__ nn, int32_t i, bool forced, uint32_t& keep,
                        uint32_t& merge) {
     if (forced) {
@@ -905,85 +922,15 @@ RT_DEV uint64_t block_exclusive_scan(uint64_t v, uint64_t* lds, uint64_t& total)
     return incl - v;
 }
 
-// per chunk of kPlocChunk positions: number kept and number merged
-__global__ void __launch_bounds__(256) k_ploc_count(int it, const int32_t* __restrict__ state,
-                                                     const int32_t* __restrict__ nn,
-                                                     uint32_t* __restrict__ part) {
-    const int32_t m = state[4 * (it & 1)];
-    if (m <= kPlocTail) return;
-    __shared__ uint64_t lds[256];
-    const int32_t nchunk = (m + kPlocChunk - 1) / kPlocChunk;
-    for (int32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
-        uint64_t v = 0;
-        for (int q = 0; q < 4; ++q) {
-            const int32_t i = c * kPlocChunk + (int32_t)threadIdx.x * 4 + q;
-            if (i < m) {
-                uint32_t keep, merge;
-                ploc_flags(nn, i, false, keep, merge);
-                v += (uint64_t)keep | ((uint64_t)merge << 32);
-            }
-        }
-        uint64_t total;
-        block_exclusive_scan<256>(v, lds, total);
-        if (threadIdx.x == 0) {
-            part[2 * (uint64_t)c] = (uint32_t)total;
-            part[2 * (uint64_t)c + 1] = (uint32_t)(total >> 32);
-        }
-    }
-}
-
-// one workgroup: chunk counts -> exclusive offsets (in place); the next iteration's state
-__global__ void __launch_bounds__(1024) k_ploc_offsets(int it, int32_t* __restrict__ state,
-                                                        uint32_t* __restrict__ part) {
-    const int32_t* cur = state + 4 * (it & 1);
-    int32_t* nxt = state + 4 * ((it + 1) & 1);
-    const int32_t m = cur[0], created = cur[1];
-    if (m <= kPlocTail) {
-        if (threadIdx.x == 0) {
-            nxt[0] = m;
-            nxt[1] = created;
-            nxt[2] = 0;
-            nxt[3] = cur[3];
-        }
-        return;
-    }
-    __shared__ uint64_t lds[1024];
-    __shared__ uint64_t carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    const int32_t nchunk = (m + kPlocChunk - 1) / kPlocChunk;
-    for (int32_t b = 0; b < nchunk; b += 1024) {
-        const int32_t c = b + (int32_t)threadIdx.x;
-        const uint64_t v = c < nchunk ? (uint64_t)part[2 * (uint64_t)c] | ((uint64_t)part[2 * (uint64_t)c + 1] << 32) : 0;
-        uint64_t total;
-        const uint64_t ex = block_exclusive_scan<1024>(v, lds, total) + carry;
-        if (c < nchunk) {
-            part[2 * (uint64_t)c] = (uint32_t)ex;
-            part[2 * (uint64_t)c + 1] = (uint32_t)(ex >> 32);
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) carry += total;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const uint32_t kept = (uint32_t)carry, merged = (uint32_t)(carry >> 32);
-        const bool forced = merged == 0;
-        nxt[0] = forced ? m - 1 : (int32_t)kept;
-        nxt[1] = created + (forced ? 1 : (int32_t)merged);
-        nxt[2] = forced ? 1 : 0;
-        nxt[3] = (it + 1) & 1;
-    }
-}
-
 // writes the merged node `id` from the clusters at positions i < j
-RT_DEV void ploc_merge(uint32_t n, int32_t id, int32_t ci, int32_t cj, float4 ilo, float4 ihi,
+RT_DEV void ploc_merge(uint32_t n, int32_t id, int32_t ci, int32_t cj, int32_t size, float4 ilo, float4 ihi,
                        float4 jlo, float4 jhi, int32_t* __restrict__ nleft, int32_t* __restrict__ nright,
                        int32_t* __restrict__ nsize, int32_t* __restrict__ parent, float4* __restrict__ nodes,
                        float* __restrict__ bounds, float4& ulo, float4& uhi) {
     const uint64_t ni = (uint64_t)n - 1;
     nleft[id] = ci;
     nright[id] = cj;
-    nsize[id] = ploc_size(nsize, ci) + ploc_size(nsize, cj);
+    nsize[id] = size;
     parent[ci >= 0 ? (uint64_t)ci : ni + (uint64_t)(~ci)] = id;
     parent[cj >= 0 ? (uint64_t)cj : ni + (uint64_t)(~cj)] = id;
     float4* nd = nodes + (uint64_t)id * 4;
@@ -998,65 +945,151 @@ RT_DEV void ploc_merge(uint32_t n, int32_t id, int32_t ci, int32_t cj, float4 il
     }
 }
 
-// compaction of one chunk: survivors to their new positions, merged pairs as new nodes
-__global__ void __launch_bounds__(256) k_ploc_compact(int it, uint32_t n, const int32_t* __restrict__ state,
-                                                       const int32_t* __restrict__ nn,
-                                                       const uint32_t* __restrict__ part,
-                                                       int32_t* __restrict__ cid0, int32_t* __restrict__ cid1,
-                                                       float4* __restrict__ cbox0, float4* __restrict__ cbox1,
-                                                       int32_t* __restrict__ nleft, int32_t* __restrict__ nright,
-                                                       int32_t* __restrict__ nsize, int32_t* __restrict__ parent,
-                                                       float4* __restrict__ nodes, float* __restrict__ bounds) {
+// Second kernel of an iteration: survivors to their new positions, merged pairs as new nodes. A workgroup
+// takes consecutive tiles and sums the counts of all tiles before its own itself (586 words at 150,000
+// positions), so the iteration needs no scan launch; one sum over all says whether any pair merged.
+__global__ void __launch_bounds__(kPlocTile) k_ploc_compact(int it, uint32_t n, int32_t* __restrict__ state,
+                                                            const int32_t* __restrict__ mate,
+                                                            const uint32_t* __restrict__ part,
+                                                            int32_t* __restrict__ cid0, int32_t* __restrict__ cid1,
+                                                            float4* __restrict__ cbox0, float4* __restrict__ cbox1,
+                                                            int32_t* __restrict__ nleft, int32_t* __restrict__ nright,
+                                                            int32_t* __restrict__ nsize, int32_t* __restrict__ parent,
+                                                            float4* __restrict__ nodes, float* __restrict__ bounds) {
+    constexpr int kWaves = kPlocTile / 64;
     const int32_t* cur = state + 4 * (it & 1);
+    int32_t* nxt = state + 4 * ((it + 1) & 1);
     const int32_t m = cur[0], created = cur[1];
-    if (m <= kPlocTail) return;
-    const bool forced = state[4 * ((it + 1) & 1) + 2] != 0;
+    const int32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const bool writer = blockIdx.x == 0 && t == 0;
+    if (m <= kPlocTail) {
+        if (writer) {
+            nxt[0] = m;
+            nxt[1] = created;
+            nxt[2] = cur[2];
+        }
+        return;
+    }
     const int32_t* __restrict__ C = (it & 1) ? cid1 : cid0;
     const float4* __restrict__ B = (it & 1) ? cbox1 : cbox0;
     int32_t* __restrict__ C2 = (it & 1) ? cid0 : cid1;
     float4* __restrict__ B2 = (it & 1) ? cbox0 : cbox1;
-    __shared__ uint64_t lds[256];
-    const int32_t nchunk = (m + kPlocChunk - 1) / kPlocChunk;
-    for (int32_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
-        uint32_t keep[4], merge[4];
-        uint64_t v = 0;
-        for (int q = 0; q < 4; ++q) {
-            const int32_t i = c * kPlocChunk + (int32_t)threadIdx.x * 4 + q;
-            keep[q] = merge[q] = 0;
-            if (i < m) ploc_flags(nn, i, forced, keep[q], merge[q]);
-            v += (uint64_t)keep[q] | ((uint64_t)merge[q] << 32);
-        }
-        uint64_t total;
-        uint64_t ex = block_exclusive_scan<256>(v, lds, total);
-        uint32_t dst = part[2 * (uint64_t)c] + (uint32_t)ex;
-        uint32_t rank = (forced ? 0u : part[2 * (uint64_t)c + 1]) + (uint32_t)(ex >> 32);
-        for (int q = 0; q < 4; ++q) {
-            const int32_t i = c * kPlocChunk + (int32_t)threadIdx.x * 4 + q;
-            if (!keep[q]) continue;
-            if (forced) dst = i == 0 ? 0u : (uint32_t)(i - 1);
-            const float4 ilo = B[2 * (uint64_t)i], ihi = B[2 * (uint64_t)i + 1];
-            if (merge[q]) {
-                const int32_t j = forced ? 1 : nn[i];
-                const int32_t id = (int32_t)n - 2 - (created + (int32_t)rank);
-                float4 ulo, uhi;
-                ploc_merge(n, id, C[i], C[j], ilo, ihi, B[2 * (uint64_t)j], B[2 * (uint64_t)j + 1], nleft,
-                           nright, nsize, parent, nodes, bounds, ulo, uhi);
-                C2[dst] = id;
-                B2[2 * (uint64_t)dst] = ulo;
-                B2[2 * (uint64_t)dst + 1] = uhi;
-                ++rank;
-            } else {
-                C2[dst] = C[i];
-                B2[2 * (uint64_t)dst] = ilo;
-                B2[2 * (uint64_t)dst + 1] = ihi;
+    __shared__ uint64_t wsum[2][kWaves];
+    __shared__ uint32_t wcount[2][kWaves];
+    const int32_t ntile = (m + kPlocTile - 1) / kPlocTile;
+    const int32_t per = (ntile + (int32_t)gridDim.x - 1) / (int32_t)gridDim.x;
+    const int32_t t0 = (int32_t)blockIdx.x * per, t1 = t0 + per < ntile ? t0 + per : ntile;
+    uint64_t before = 0, all = 0;  // kept | merged << 32
+#pragma unroll 4
+    for (int32_t k = t; k < ntile; k += kPlocTile) {
+        const uint64_t v = (uint64_t)(part[k] & 0xFFFFu) | ((uint64_t)(part[k] >> 16) << 32);
+        all += v;
+        before += k < t0 ? v : 0;
+    }
+    for (int x = 1; x < 64; x <<= 1) {
+        all += __shfl_xor((unsigned long long)all, x);
+        before += __shfl_xor((unsigned long long)before, x);
+    }
+    if (lane == 0) {
+        wsum[0][wave] = all;
+        wsum[1][wave] = before;
+    }
+    __syncthreads();
+    all = before = 0;
+    for (int w = 0; w < kWaves; ++w) {
+        all += wsum[0][w];
+        before += wsum[1][w];
+    }
+    const bool forced = (all >> 32) == 0;
+    if (writer) {
+        nxt[0] = forced ? m - 1 : (int32_t)(uint32_t)all;
+        nxt[1] = created + (forced ? 1 : (int32_t)(all >> 32));
+        nxt[2] = (it + 1) & 1;
+    }
+    uint32_t kept = (uint32_t)before, merged = (uint32_t)(before >> 32);
+    const uint64_t below = (1ull << lane) - 1;
+    for (int32_t tile = t0; tile < t1; ++tile) {
+        const int32_t i = tile * kPlocTile + t, j = forced ? 1 : i < m ? mate[i] : -1;
+        const bool keep = i < m && (forced ? i != 1 : j < 0 || i < j);
+        const bool merge = i < m && (forced ? i == 0 : j > i);
+        const uint64_t kb = __ballot(keep), mb = __ballot(merge);
+        uint32_t* wc = wcount[(tile - t0) & 1];
+        if (lane == 0) wc[wave] = (uint32_t)__popcll(kb) | ((uint32_t)__popcll(mb) << 16);
+        __syncthreads();
+        uint32_t dst = kept + (uint32_t)__popcll(kb & below), rank = merged + (uint32_t)__popcll(mb & below);
+        for (int w = 0; w < kWaves; ++w) {
+            const uint32_t c = wc[w];
+            if (w < wave) {
+                dst += c & 0xFFFFu;
+                rank += c >> 16;
             }
-            ++dst;
+            kept += c & 0xFFFFu;
+            merged += c >> 16;
         }
+        if (!keep) continue;
+        if (forced) {
+            dst = i == 0 ? 0u : (uint32_t)(i - 1);
+            rank = 0;
+        }
+        float4 lo = B[2 * (uint64_t)i], hi = B[2 * (uint64_t)i + 1];
+        int32_t c = C[i];
+        if (merge) {
+            const int32_t cj = C[j], id = (int32_t)n - 2 - (created + (int32_t)rank);
+            float4 ulo, uhi;
+            ploc_merge(n, id, c, cj, ploc_size(nsize, c) + ploc_size(nsize, cj), lo, hi, B[2 * (uint64_t)j],
+                       B[2 * (uint64_t)j + 1], nleft, nright, nsize, parent, nodes, bounds, ulo, uhi);
+            c = id;
+            lo = ulo;
+            hi = uhi;
+        }
+        C2[dst] = c;
+        B2[2 * (uint64_t)dst] = lo;
+        B2[2 * (uint64_t)dst + 1] = hi;
     }
 }
 
-// The remaining iterations (m <= kPlocTail normally; any m is handled) in one workgroup, from the
-// state left in state[4 * slot].
+// Nearest neighbour of position i among [i - R, i + R] by 2^lg consecutive lanes, lane q
+// taking a share of the candidates in order; valid in lane 0. The same as ploc_nn: only the first
+// candidate counts before it was compared, so a box of NaN keeps it, and a tie goes to the smaller position.
+template <typename AreaTo>
+RT_DEV int32_t ploc_nn_lanes(int32_t i, int32_t m, int lg, int q, AreaTo area) {
+    const int32_t lo = i - kPlocRadius < 0 ? 0 : i - kPlocRadius;
+    const int32_t hi = i + kPlocRadius > m - 1 ? m - 1 : i + kPlocRadius;
+    const int32_t count = hi - lo, share = (count + (1 << lg) - 1) >> lg;
+    int32_t k = q * share;
+    const int32_t end = k + share < count ? k + share : count;
+    float best = INFINITY;
+    int32_t bj = -1;
+    if (q == 0) {
+        bj = lo == i ? i + 1 : lo;
+        best = area(bj);
+        k = 1;
+    }
+#pragma unroll 4
+    for (; k < end; ++k) {
+        const int32_t j = lo + k + (lo + k >= i ? 1 : 0);
+        const float a = area(j);
+        if (a < best) {
+            best = a;
+            bj = j;
+        }
+    }
+    for (int x = 1; x < 1 << lg; x <<= 1) {
+        const float oa = __shfl_down(best, x);
+        const int32_t oj = __shfl_down(bj, x);
+        if (oa < best) {
+            best = oa;
+            bj = oj;
+        }
+    }
+    return bj;
+}
+
+// The remaining iterations in one workgroup, from the state left in state[4 * slot]: more than kPlocTail
+// clusters (only if the launched iterations merged less than expected) through memory, the rest in LDS,
+// where a search costs no L2 round trips, sizes need no loads and the compaction counts by ballots.
+// From 512 clusters down several lanes share a search. The 65 or so iterations from 4,096 clusters on
+// took 499 us through memory, 229 like this.
 __global__ void __launch_bounds__(1024) k_ploc_tail(int slot, uint32_t n, int32_t* __restrict__ state,
                                                      int32_t* __restrict__ nn, int32_t* __restrict__ cid0,
                                                      int32_t* __restrict__ cid1, float4* __restrict__ cbox0,
@@ -1072,11 +1105,11 @@ __global__ void __launch_bounds__(1024) k_ploc_tail(int slot, uint32_t n, int32_
         sm = state[4 * slot];
         screated = state[4 * slot + 1];
     }
-    int par = state[4 * slot + 3];
+    int par = state[4 * slot + 2];
     __syncthreads();
     for (;;) {
         const int32_t m = sm, created = screated;
-        if (m <= 1) break;
+        if (m <= kPlocTail) break;
         const int32_t* __restrict__ C = par ? cid1 : cid0;
         const float4* __restrict__ B = par ? cbox1 : cbox0;
         int32_t* __restrict__ C2 = par ? cid0 : cid1;
@@ -1120,8 +1153,8 @@ __global__ void __launch_bounds__(1024) k_ploc_tail(int slot, uint32_t n, int32_
                     const int32_t j = forced ? 1 : nn[i];
                     const int32_t id = (int32_t)n - 2 - (created + (int32_t)rank);
                     float4 ulo, uhi;
-                    ploc_merge(n, id, C[i], C[j], ilo, ihi, B[2 * (uint64_t)j], B[2 * (uint64_t)j + 1],
-                               nleft, nright, nsize, parent, nodes, bounds, ulo, uhi);
+                    ploc_merge(n, id, C[i], C[j], ploc_size(nsize, C[i]) + ploc_size(nsize, C[j]), ilo, ihi,
+                               B[2 * (uint64_t)j], B[2 * (uint64_t)j + 1], nleft, nright, nsize, parent, nodes, bounds, ulo, uhi);
                     C2[dst] = id;
                     B2[2 * (uint64_t)dst] = ulo;
                     B2[2 * (uint64_t)dst + 1] = uhi;
@@ -1142,6 +1175,121 @@ __global__ void __launch_bounds__(1024) k_ploc_tail(int slot, uint32_t n, int32_
             screated = created + (forced ? 1 : (int32_t)(carry >> 32));
         }
         par ^= 1;
+        __syncthreads();
+    }
+    constexpr int kPer = kPlocTail / 1024, kWaves = 16;
+    __shared__ float box[6][kPlocTail];
+    __shared__ int32_t cid[kPlocTail], csize[kPlocTail];
+    __shared__ uint16_t near[kPlocTail];
+    __shared__ uint32_t wcount[kPer * kWaves];  // per 64 positions: kept | merged << 16
+    int32_t m = sm, created = screated;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    {
+        const int32_t* __restrict__ C = par ? cid1 : cid0;
+        const float4* __restrict__ B = par ? cbox1 : cbox0;
+        for (int32_t i = tid; i < m; i += 1024) {
+            const Box b = load_box(B + 2 * (uint64_t)i);
+            for (int a = 0; a < 3; ++a) {
+                box[a][i] = b.lo[a];
+                box[3 + a][i] = b.hi[a];
+            }
+            cid[i] = C[i];
+            csize[i] = ploc_size(nsize, C[i]);
+        }
+    }
+    __syncthreads();
+    auto lo_of = [&](int32_t i) { return make_float4(box[0][i], box[1][i], box[2][i], 0.0f); };
+    auto hi_of = [&](int32_t i) { return make_float4(box[3][i], box[4][i], box[5][i], 0.0f); };
+    while (m > 1) {
+        const int lg = m > 512 ? 0 : m > 256 ? 1 : m > 128 ? 2 : m > 64 ? 3 : 4;  // 2^lg lanes per search
+        for (int32_t w = tid; w < m << lg; w += 1024) {  // one round where lg > 0
+            const int32_t i = w >> lg, q = w & ((1 << lg) - 1);
+            const float4 lo = lo_of(i), hi = hi_of(i);
+            const int32_t j = ploc_nn_lanes(i, m, lg, q, [&](int32_t j) { return union_area(lo, hi, lo_of(j), hi_of(j)); });
+            if (q == 0) near[i] = (uint16_t)j;
+        }
+        __syncthreads();
+        bool keep[kPer], merge[kPer];
+        int32_t mate[kPer];
+        uint64_t kb[kPer], mb[kPer];
+#pragma unroll
+        for (int c = 0; c < kPer; ++c) {
+            const int32_t i = tid + c * 1024;
+            keep[c] = merge[c] = false;
+            mate[c] = 0;
+            if (i < m) {
+                mate[c] = near[i];
+                const bool mutual = near[mate[c]] == i;
+                keep[c] = !mutual || i < mate[c];
+                merge[c] = mutual && i < mate[c];
+            }
+            kb[c] = __ballot(keep[c]);
+            mb[c] = __ballot(merge[c]);
+            if (lane == 0) wcount[c * kWaves + wave] = (uint32_t)__popcll(kb[c]) | ((uint32_t)__popcll(mb[c]) << 16);
+        }
+        __syncthreads();
+        const uint32_t own = wcount[lane];  // kPer * kWaves = 64 counts, scanned by every wave
+        uint32_t incl = own;
+        for (int x = 1; x < 64; x <<= 1) {
+            const uint32_t v = __shfl_up(incl, x);
+            if (lane >= x) incl += v;
+        }
+        const uint32_t total = __shfl(incl, 63);
+        const bool forced = (total >> 16) == 0;
+        const uint64_t below = (1ull << lane) - 1;
+        Box bi[kPer], bj[kPer];
+        int32_t ci[kPer], cj[kPer], si[kPer], sj[kPer];
+        uint32_t dst[kPer], rank[kPer];
+#pragma unroll
+        for (int c = 0; c < kPer; ++c) {
+            const int32_t i = tid + c * 1024;
+            const uint32_t at = __shfl(incl - own, c * kWaves + wave);
+            dst[c] = (at & 0xFFFFu) + (uint32_t)__popcll(kb[c] & below);
+            rank[c] = (at >> 16) + (uint32_t)__popcll(mb[c] & below);
+            if (forced) {
+                keep[c] = i < m && i != 1;
+                merge[c] = i == 0;
+                mate[c] = 1;
+                dst[c] = i == 0 ? 0u : (uint32_t)(i - 1);
+                rank[c] = 0;
+            }
+            if (keep[c]) {
+                const int32_t j = merge[c] ? mate[c] : i;
+                for (int a = 0; a < 3; ++a) {
+                    bi[c].lo[a] = box[a][i];
+                    bi[c].hi[a] = box[3 + a][i];
+                    bj[c].lo[a] = box[a][j];
+                    bj[c].hi[a] = box[3 + a][j];
+                }
+                ci[c] = cid[i];
+                cj[c] = cid[j];
+                si[c] = csize[i];
+                sj[c] = csize[j];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < kPer; ++c) {
+            if (!keep[c]) continue;
+            float4 ulo = make_float4(bi[c].lo[0], bi[c].lo[1], bi[c].lo[2], 0.0f);
+            float4 uhi = make_float4(bi[c].hi[0], bi[c].hi[1], bi[c].hi[2], 0.0f);
+            if (merge[c]) {
+                const float4 ilo = ulo, ihi = uhi;
+                const int32_t id = (int32_t)n - 2 - (created + (int32_t)rank[c]);
+                si[c] += sj[c];
+                ploc_merge(n, id, ci[c], cj[c], si[c], ilo, ihi,
+                           make_float4(bj[c].lo[0], bj[c].lo[1], bj[c].lo[2], 0.0f),
+                           make_float4(bj[c].hi[0], bj[c].hi[1], bj[c].hi[2], 0.0f), nleft, nright, nsize, parent,
+                           nodes, bounds, ulo, uhi);
+                ci[c] = id;
+            }
+            box[0][dst[c]] = ulo.x; box[1][dst[c]] = ulo.y; box[2][dst[c]] = ulo.z;
+            box[3][dst[c]] = uhi.x; box[4][dst[c]] = uhi.y; box[5][dst[c]] = uhi.z;
+            cid[dst[c]] = ci[c];
+            csize[dst[c]] = si[c];
+        }
+        m = forced ? m - 1 : (int32_t)(total & 0xFFFFu);
+        created += forced ? 1 : (int32_t)(total >> 16);
         __syncthreads();
     }
 }
@@ -1584,14 +1732,11 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
         hipLaunchKernelGGL(k_ploc_init, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, n, w.leafbox,
                            w.cid[0], w.cbox[0], w.pos_of, w.parent, w.state);
         const int iters = ploc_iterations(n);
-        const uint32_t gnn = std::min<uint32_t>(kPlocGrid, blocks_for(n, kPlocTile));
-        const uint32_t gch = std::min<uint32_t>(kPlocGrid, nchunk);
+        const uint32_t grid = std::min<uint32_t>(kPlocGrid, blocks_for(n, kPlocTile));
         for (int it = 0; it < iters; ++it) {
-            hipLaunchKernelGGL(k_ploc_nn, dim3(gnn), dim3(kPlocTile), 0, s, it, w.state, w.cbox[0],
-                               w.cbox[1], w.nn);
-            hipLaunchKernelGGL(k_ploc_count, dim3(gch), dim3(256), 0, s, it, w.state, w.nn, w.part);
-            hipLaunchKernelGGL(k_ploc_offsets, dim3(1), dim3(1024), 0, s, it, w.state, w.part);
-            hipLaunchKernelGGL(k_ploc_compact, dim3(gch), dim3(256), 0, s, it, n, w.state, w.nn, w.part,
+            hipLaunchKernelGGL(k_ploc_pairs, dim3(grid), dim3(kPlocLoad), 0, s, it, w.state, w.cbox[0],
+                               w.cbox[1], w.nn, w.part);
+            hipLaunchKernelGGL(k_ploc_compact, dim3(grid), dim3(kPlocTile), 0, s, it, n, w.state, w.nn, w.part,
                                w.cid[0], w.cid[1], w.cbox[0], w.cbox[1], w.nleft, w.nright, w.nsize,
                                w.parent, nodes, sc->bounds);
         }

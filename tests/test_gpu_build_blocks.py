@@ -3,7 +3,7 @@ equal codes (every split by slot number), and codes in a few crowded cells."""
 import numpy as np
 import pytest
 
-from helpers import gpu_from_meshes, twin_from_meshes
+from helpers import gpu_arrays, gpu_from_meshes, twin_from_meshes
 from test_gpu_parity import assert_build_equal
 
 pytestmark = pytest.mark.gpu
@@ -34,3 +34,30 @@ def test_small_order(ren, n, kind):
     """Order by chunks of 256 and merge by search (up to 32,768 triangles), and by radix passes from there."""
     meshes = [_mesh(n, kind)]
     assert_build_equal(gpu_from_meshes(meshes), twin_from_meshes(meshes))
+
+
+def _ploc(ren, mesh):
+    got = ren.Raycaster([ren.mesh_from_arrays(mesh["pos"], mesh["idx"])], tuning={"builder": "ploc"})
+    return got, twin_from_meshes([mesh], builder="ploc")
+
+
+@pytest.mark.parametrize("kind", ["spread", "equal", "crowded"])
+@pytest.mark.parametrize("n", [2, 3, 64, 65, 129, 257, 513, 1025, 4096, 4097, 4353, 9000])
+def test_ploc_sizes(ren, n, kind):
+    """PLOC at the widths of a search in its last workgroup, at the hand-over to it (4,096 clusters) and at
+    the tiles before it."""
+    assert_build_equal(*_ploc(ren, _mesh(n, kind)))
+
+
+@pytest.mark.parametrize("n", [40, 700])
+def test_ploc_nan(ren, n):
+    """Most boxes NaN: a search keeps its first candidate. A NaN's bits are not compared."""
+    mesh = _mesh(n, "spread")
+    mesh["pos"][np.random.default_rng(n).random(len(mesh["pos"])) < 0.9] = np.nan
+    rc, tw = _ploc(ren, mesh)
+    g = gpu_arrays(rc)
+    np.testing.assert_array_equal(g["order"].view(np.uint32), tw.order)
+    nodes, want = g["nodes"], np.asarray(tw.nodes).reshape(g["nodes"].shape)
+    np.testing.assert_array_equal(np.ascontiguousarray(nodes[:, 12:14]).view(np.uint32),
+                                  np.ascontiguousarray(want[:, 12:14]).view(np.uint32))
+    np.testing.assert_array_equal(nodes[:, :12], want[:, :12])
