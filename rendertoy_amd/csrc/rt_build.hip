@@ -2,16 +2,15 @@
 // (Raycaster.__init__ -> _build_ads, a stub in the reference that only counts triangles).
 //
 // Pipeline (one stream; no host synchronisation except the PLOC depth check):
-//   1. gather      per mesh: read MeshVertex P/N/C (rendering/_modeling.py:22-28) through the
-//                  optional int32 index list, write unsorted tri/shade records, padded leaf box,
-//                  AABB centroid.
+//   1. gather      per mesh: read MeshVertex P (rendering/_modeling.py:22-28) through the optional
+//                  int32 index list, write AABB centroids.
 //   2. bounds      min/max of the centroids per workgroup of the gather, folded by the next kernel.
 //   3. morton      30-bit Morton code of each centroid quantised to 1024^3 over those bounds.
 //   4. sort        stable LSD radix sort of (code, primitive) in 4 passes of 8 bits (rt_sort.h):
 //                  per-tile histogram -> per-digit row scan -> scatter, the scatter ranking keys
 //                  with wave64 ballot/mbcnt multi-split so equal digits keep input order and
 //                  writing each tile digit by digit from LDS.
-//   5. emit        permute tri/shade records into slot order.
+//   5. emit        tri/shade records and padded leaf boxes in slot order, from the meshes' P/N/C.
 //   6. tree        Karras 2012 binary radix tree over the extended keys (code, slot), with its boxes:
 //                  bottom-up in LDS inside blocks of 1024 slots, then one wave per node that spans
 //                  blocks (min/max are exact, so range unions equal the bottom-up boxes).
@@ -53,11 +52,17 @@ struct TopArrays {
     float4* block;     // 2 per block: box of all its slots
 };
 
+// A mesh with triangles as the kernels after the gather read it: its first primitive and its number
+// among all meshes.
+struct MeshSource {
+    rt_mesh_desc d;
+    uint32_t base, id;
+};
+
 struct Workspace {
     float4* cent;      // n
-    float4* leafbox;   // 2n
-    float4* tri_u;     // 3n
-    float4* shade_u;   // 4n
+    float4* leafbox;   // 2n: padded box of each slot (LBVH)
+    MeshSource* meshes;  // of the meshes that have triangles
     uint32_t* keys0;   // n
     uint32_t* vals0;
     uint32_t* keys1;
@@ -100,8 +105,7 @@ Workspace carve(char* base, uint64_t n) {
     };
     w.cent = (float4*)take(16 * n);
     w.leafbox = (float4*)take(32 * n);
-    w.tri_u = (float4*)take(48 * n);
-    w.shade_u = (float4*)take(64 * n);
+    w.meshes = (MeshSource*)take(sizeof(MeshSource) * n);
     w.keys0 = (uint32_t*)take(4 * n);
     w.vals0 = (uint32_t*)take(4 * n);
     w.keys1 = (uint32_t*)take(4 * n);
@@ -205,120 +209,83 @@ RT_DEV Box block_unite(const float4* __restrict__ parts, uint32_t count, float4*
     return b;
 }
 
-// Copies `per` float4s of each of the block's `rows` records from LDS (record r at
-// stage[r * pitch]) to out[0 .. rows*per), one float4 per thread and instruction.
-RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t rows, uint32_t per,
-                         uint32_t pitch) {
-    for (uint32_t q = threadIdx.x; q < rows * per; q += blockDim.x) {
-        const uint32_t r = q / per;
-        out[q] = stage[r * pitch + (q - r * per)];
+// Positions of triangle t of a mesh with canonical zeros, and its vertex indices; an index past the
+// vertices is clamped, so a malformed list cannot read past the buffer.
+RT_DEV void load_corners(const rt_mesh_desc& m, uint32_t t, uint32_t (&v)[3], float3 (&p)[3]) {
+    for (int k = 0; k < 3; ++k) v[k] = 3 * t + k;
+    if (m.indices) {
+        const uint32_t* ix = (const uint32_t*)m.indices + 3 * (uint64_t)t;
+        for (int k = 0; k < 3; ++k) v[k] = ix[k];
+        for (int k = 0; k < 3; ++k) v[k] = v[k] < m.n_vertices ? v[k] : m.n_vertices - 1;
+    }
+    for (int k = 0; k < 3; ++k) {
+        const float3 q = load_f3((const char*)m.vertices, v[k], m.vertex_stride, m.pos_offset);
+        p[k] = make_float3(canon(q.x), canon(q.y), canon(q.z));
     }
 }
 
-// One thread per triangle: positions (canonical zeros), the centroid, the padded leaf box, the
-// intersection record (p0, e1, e2, primitive id) and the shading record (three normals, three
-// uvs, mesh id). The block's records go out through LDS as consecutive float4s.
+RT_DEV Box corners_box(const float3 (&p)[3]) {
+    return {{fminf(fminf(p[0].x, p[1].x), p[2].x), fminf(fminf(p[0].y, p[1].y), p[2].y),
+             fminf(fminf(p[0].z, p[1].z), p[2].z)},
+            {fmaxf(fmaxf(p[0].x, p[1].x), p[2].x), fmaxf(fmaxf(p[0].y, p[1].y), p[2].y),
+             fmaxf(fmaxf(p[0].z, p[1].z), p[2].z)}};
+}
+
+RT_DEV Box padded(Box b) {
+    for (int c = 0; c < 3; ++c) {
+        const float pad = pad_of(b.lo[c], b.hi[c]);
+        b.lo[c] -= pad;
+        b.hi[c] += pad;
+    }
+    return b;
+}
+
+// The mesh of primitive p: the last one of `count` whose first primitive is not past it.
+RT_DEV const MeshSource& mesh_of(const MeshSource* __restrict__ meshes, uint32_t count, uint32_t p) {
+    uint32_t lo = 0, hi = count - 1;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1) / 2;
+        if (meshes[mid].base <= p)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return meshes[lo];
+}
+
+// One thread per triangle: the centroid of its box; the workgroup's union of centroids to `partial`, the
+// mesh's description to `source` (NULL for a mesh without triangles). Everything else a triangle needs is
+// read from its mesh again when its slot is known (k_emit).
 __global__ void __launch_bounds__(256) k_gather(rt_mesh_desc m, uint32_t mesh_id, uint32_t n_meshes,
-                                                 uint32_t prim_base, float4* __restrict__ cent,
-                                                 float4* __restrict__ leafbox,
-                                                 float4* __restrict__ tri_u,
-                                                 float4* __restrict__ shade_u,
-                                                 int32_t* __restrict__ mesh_offsets,
-                                                 float4* __restrict__ partial) {
-    constexpr uint32_t kPitch = 5;  // float4s per staged record (4 used)
-    __shared__ float4 stage[256 * kPitch];
+                                                uint32_t prim_base, float4* __restrict__ cent,
+                                                int32_t* __restrict__ mesh_offsets,
+                                                float4* __restrict__ partial, MeshSource* __restrict__ source) {
     __shared__ float4 wpart[4][2];
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) mesh_offsets[mesh_id] = (int32_t)prim_base;
-    if (t == 0 && mesh_id + 1 == n_meshes) mesh_offsets[n_meshes] = (int32_t)(prim_base + m.n_tris);
-    const uint32_t t0 = blockIdx.x * blockDim.x;
-    if (t0 >= m.n_tris) return;  // whole block (only the launch for an empty mesh)
-    const uint32_t rows = m.n_tris - t0 < blockDim.x ? m.n_tris - t0 : blockDim.x;
-    const uint64_t pb = (uint64_t)prim_base + t0;  // the block's first primitive
-    const bool mine = t < m.n_tris;
-    float4 box[2], tri[3], shd[4];
+    if (t == 0) {
+        mesh_offsets[mesh_id] = (int32_t)prim_base;
+        if (mesh_id + 1 == n_meshes) mesh_offsets[n_meshes] = (int32_t)(prim_base + m.n_tris);
+        if (m.n_tris) *source = {m, prim_base, mesh_id};
+    }
+    if (blockIdx.x * blockDim.x >= m.n_tris) return;  // whole block (only the launch for an empty mesh)
     Box cb = empty_box();
-    if (mine) {
-        const char* vb = (const char*)m.vertices;
-        uint32_t i0 = 3 * t, i1 = 3 * t + 1, i2 = 3 * t + 2;
-        if (m.indices) {
-            i0 = (uint32_t)m.indices[3 * (uint64_t)t];
-            i1 = (uint32_t)m.indices[3 * (uint64_t)t + 1];
-            i2 = (uint32_t)m.indices[3 * (uint64_t)t + 2];
-            // out-of-range indices are clamped so a malformed list cannot read past the buffer
-            i0 = i0 < m.n_vertices ? i0 : m.n_vertices - 1;
-            i1 = i1 < m.n_vertices ? i1 : m.n_vertices - 1;
-            i2 = i2 < m.n_vertices ? i2 : m.n_vertices - 1;
-        }
-        float3 p0 = load_f3(vb, i0, m.vertex_stride, m.pos_offset);
-        float3 p1 = load_f3(vb, i1, m.vertex_stride, m.pos_offset);
-        float3 p2 = load_f3(vb, i2, m.vertex_stride, m.pos_offset);
-        p0 = make_float3(canon(p0.x), canon(p0.y), canon(p0.z));
-        p1 = make_float3(canon(p1.x), canon(p1.y), canon(p1.z));
-        p2 = make_float3(canon(p2.x), canon(p2.y), canon(p2.z));
-        const uint32_t p = prim_base + t;
-
-        const float lox = fminf(fminf(p0.x, p1.x), p2.x), hix = fmaxf(fmaxf(p0.x, p1.x), p2.x);
-        const float loy = fminf(fminf(p0.y, p1.y), p2.y), hiy = fmaxf(fmaxf(p0.y, p1.y), p2.y);
-        const float loz = fminf(fminf(p0.z, p1.z), p2.z), hiz = fmaxf(fmaxf(p0.z, p1.z), p2.z);
-        const float cx = (lox + hix) * 0.5f, cy = (loy + hiy) * 0.5f, cz = (loz + hiz) * 0.5f;
-        cent[p] = make_float4(cx, cy, cz, 0.0f);
-        cb = unite(cb, {{cx, cy, cz}, {cx, cy, cz}});
-        const float px = pad_of(lox, hix), py = pad_of(loy, hiy), pz = pad_of(loz, hiz);
-        box[0] = make_float4(lox - px, loy - py, loz - pz, 0.0f);
-        box[1] = make_float4(hix + px, hiy + py, hiz + pz, 0.0f);
-
-        const float e1x = p1.x - p0.x, e1y = p1.y - p0.y, e1z = p1.z - p0.z;
-        const float e2x = p2.x - p0.x, e2y = p2.y - p0.y, e2z = p2.z - p0.z;
-        tri[0] = make_float4(p0.x, p0.y, p0.z, __int_as_float((int32_t)p));
-        tri[1] = make_float4(e1x, e1y, e1z, 0.0f);
-        tri[2] = make_float4(e2x, e2y, e2z, 0.0f);
-
-        float3 n0, n1, n2;
-        if (m.nrm_offset != RT_ABSENT) {
-            n0 = load_f3(vb, i0, m.vertex_stride, m.nrm_offset);
-            n1 = load_f3(vb, i1, m.vertex_stride, m.nrm_offset);
-            n2 = load_f3(vb, i2, m.vertex_stride, m.nrm_offset);
-        } else {
-            const float gx = fmaf(e1y, e2z, -(e1z * e2y));
-            const float gy = fmaf(e1z, e2x, -(e1x * e2z));
-            const float gz = fmaf(e1x, e2y, -(e1y * e2x));
-            const float l2 = fmaf(gx, gx, fmaf(gy, gy, gz * gz));
-            const float il = l2 > 0.0f ? 1.0f / sqrtf(l2) : 0.0f;
-            n0 = n1 = n2 = make_float3(gx * il, gy * il, gz * il);
-        }
-        float2 uv0 = make_float2(0.0f, 0.0f), uv1 = uv0, uv2 = uv0;
-        if (m.uv_offset != RT_ABSENT) {
-            const float* q0 = (const float*)(vb + (uint64_t)i0 * m.vertex_stride + m.uv_offset);
-            const float* q1 = (const float*)(vb + (uint64_t)i1 * m.vertex_stride + m.uv_offset);
-            const float* q2 = (const float*)(vb + (uint64_t)i2 * m.vertex_stride + m.uv_offset);
-            uv0 = make_float2(q0[0], q0[1]);
-            uv1 = make_float2(q1[0], q1[1]);
-            uv2 = make_float2(q2[0], q2[1]);
-        }
-        shd[0] = make_float4(n0.x, n0.y, n0.z, n1.x);
-        shd[1] = make_float4(n1.y, n1.z, n2.x, n2.y);
-        shd[2] = make_float4(n2.z, uv0.x, uv0.y, uv1.x);
-        shd[3] = make_float4(uv1.y, uv2.x, uv2.y, __int_as_float((int32_t)mesh_id));
+    if (t < m.n_tris) {
+        uint32_t v[3];
+        float3 p[3];
+        load_corners(m, t, v, p);
+        const Box b = corners_box(p);
+        float c[3];
+        for (int k = 0; k < 3; ++k) c[k] = (b.lo[k] + b.hi[k]) * 0.5f;
+        cent[prim_base + t] = make_float4(c[0], c[1], c[2], 0.0f);
+        cb = unite(cb, {{c[0], c[1], c[2]}, {c[0], c[1], c[2]}});
     }
     cb = wave_unite(cb);
     if ((threadIdx.x & 63) == 0) store_box(wpart[threadIdx.x >> 6], cb);
-    float4* st = stage + threadIdx.x * kPitch;
-    if (mine) { st[0] = shd[0]; st[1] = shd[1]; st[2] = shd[2]; st[3] = shd[3]; }
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < 4; ++w) cb = unite(cb, load_box(wpart[w]));
         store_box(partial + 2 * (uint64_t)blockIdx.x, cb);
     }
-    store_staged(shade_u + 4 * pb, stage, rows, 4, kPitch);
-    __syncthreads();
-    if (mine) { st[0] = tri[0]; st[1] = tri[1]; st[2] = tri[2]; }
-    __syncthreads();
-    store_staged(tri_u + 3 * pb, stage, rows, 3, kPitch);
-    __syncthreads();
-    if (mine) { st[0] = box[0]; st[1] = box[1]; }
-    __syncthreads();
-    store_staged(leafbox + 2 * pb, stage, rows, 2, kPitch);
 }
 
 __global__ void k_mesh_offsets_tail(int32_t* mesh_offsets, uint32_t n_meshes, uint32_t n) {
@@ -477,25 +444,81 @@ __global__ void __launch_bounds__(256) k_order_merge(const uint32_t* __restrict_
     }
 }
 
-// One thread per float4 of the outputs: thread x copies shade float4 x (record x/4) and, for
-// x < 3n, tris float4 x (record x/3), so each store instruction writes consecutive 16 B pieces
-// and each record's source is read as consecutive pieces by neighbouring lanes. Also the slot of each
-// primitive.
-__global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order, uint32_t n,
-                                              const float4* __restrict__ tri_u,
-                                              const float4* __restrict__ shade_u,
-                                              float4* __restrict__ tris,
-                                              float4* __restrict__ shade,
-                                              uint32_t* __restrict__ prim_slot) {
-    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= 4 * (uint64_t)n) return;
-    const uint64_t ps = order[x >> 2];
-    shade[x] = shade_u[4 * ps + (x & 3)];
-    if ((x & 3) == 0) prim_slot[ps] = (uint32_t)(x >> 2);
-    if (x < 3 * (uint64_t)n) {
-        const uint64_t s = x / 3;
-        tris[x] = tri_u[3 * (uint64_t)order[s] + (x - 3 * s)];
+// Copies `per` float4s of each of the block's `rows` records from LDS (record r at
+// stage[r * pitch]) to out[0 .. rows*per), one float4 per thread and instruction.
+RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t rows, uint32_t per,
+                         uint32_t pitch) {
+    for (uint32_t q = threadIdx.x; q < rows * per; q += blockDim.x) {
+        const uint32_t r = q / per;
+        out[q] = stage[r * pitch + (q - r * per)];
     }
+}
+
+// One thread per slot: the intersection record (p0, e1, e2, primitive id) and the shading record (three
+// normals, three uvs, mesh id) of its triangle, from the mesh's vertices; the padded leaf box of the slot if
+// `leafbox` is not NULL; the slot of the primitive. The block's records go out through LDS as consecutive
+// float4s. Bound by memory: 180 B of stores per triangle, and the vertices, which neighbours in Morton
+// order share in L2. At 1.31 M triangles 72 us and 32 for the gather; records written in
+// primitive order by the gather and permuted here took 81 and 71.
+__global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order, uint32_t n,
+                                              const MeshSource* __restrict__ meshes, uint32_t n_sources,
+                                              float4* __restrict__ leafbox, float4* __restrict__ tris,
+                                              float4* __restrict__ shade, uint32_t* __restrict__ prim_slot) {
+    constexpr uint32_t kPitch = 5;  // float4s per staged record (4 used)
+    __shared__ float4 stage[256 * kPitch];
+    const uint64_t s0 = (uint64_t)blockIdx.x * 256;
+    const uint32_t rows = n - s0 < 256 ? (uint32_t)(n - s0) : 256u;
+    const bool mine = threadIdx.x < rows;
+    float4 tri[3], shd[4];
+    Box box = empty_box();
+    if (mine) {
+        const uint32_t prim = order[s0 + threadIdx.x];
+        const MeshSource& src = mesh_of(meshes, n_sources, prim);
+        const rt_mesh_desc& m = src.d;
+        uint32_t v[3];
+        float3 p[3], nr[3];
+        load_corners(m, prim - src.base, v, p);
+        box = padded(corners_box(p));
+        prim_slot[prim] = (uint32_t)s0 + threadIdx.x;
+        const float e1x = p[1].x - p[0].x, e1y = p[1].y - p[0].y, e1z = p[1].z - p[0].z;
+        const float e2x = p[2].x - p[0].x, e2y = p[2].y - p[0].y, e2z = p[2].z - p[0].z;
+        tri[0] = make_float4(p[0].x, p[0].y, p[0].z, __int_as_float((int32_t)prim));
+        tri[1] = make_float4(e1x, e1y, e1z, 0.0f);
+        tri[2] = make_float4(e2x, e2y, e2z, 0.0f);
+        if (m.nrm_offset != RT_ABSENT) {
+            for (int k = 0; k < 3; ++k) nr[k] = load_f3((const char*)m.vertices, v[k], m.vertex_stride, m.nrm_offset);
+        } else {
+            const float gx = fmaf(e1y, e2z, -(e1z * e2y));
+            const float gy = fmaf(e1z, e2x, -(e1x * e2z));
+            const float gz = fmaf(e1x, e2y, -(e1y * e2x));
+            const float l2 = fmaf(gx, gx, fmaf(gy, gy, gz * gz));
+            const float il = l2 > 0.0f ? 1.0f / sqrtf(l2) : 0.0f;
+            nr[0] = nr[1] = nr[2] = make_float3(gx * il, gy * il, gz * il);
+        }
+        float2 uv[3] = {make_float2(0.0f, 0.0f), make_float2(0.0f, 0.0f), make_float2(0.0f, 0.0f)};
+        if (m.uv_offset != RT_ABSENT)
+            for (int k = 0; k < 3; ++k) {
+                const float* q = (const float*)((const char*)m.vertices + (uint64_t)v[k] * m.vertex_stride + m.uv_offset);
+                uv[k] = make_float2(q[0], q[1]);
+            }
+        shd[0] = make_float4(nr[0].x, nr[0].y, nr[0].z, nr[1].x);
+        shd[1] = make_float4(nr[1].y, nr[1].z, nr[2].x, nr[2].y);
+        shd[2] = make_float4(nr[2].z, uv[0].x, uv[0].y, uv[1].x);
+        shd[3] = make_float4(uv[1].y, uv[2].x, uv[2].y, __int_as_float((int32_t)src.id));
+    }
+    float4* st = stage + threadIdx.x * kPitch;
+    if (mine) { st[0] = shd[0]; st[1] = shd[1]; st[2] = shd[2]; st[3] = shd[3]; }
+    __syncthreads();
+    store_staged(shade + 4 * s0, stage, rows, 4, kPitch);
+    __syncthreads();
+    if (mine) { st[0] = tri[0]; st[1] = tri[1]; st[2] = tri[2]; }
+    __syncthreads();
+    store_staged(tris + 3 * s0, stage, rows, 3, kPitch);
+    if (!leafbox) return;
+    __syncthreads();
+    if (mine) store_box(st, box);
+    __syncthreads();
+    store_staged(leafbox + 2 * s0, stage, rows, 2, kPitch);
 }
 
 // ---- tree ----
@@ -554,8 +577,7 @@ RT_DEV void store_bounds(float* __restrict__ bounds, const Box& b) {
 }
 
 __global__ void __launch_bounds__(kTreeBlock) k_tree_local(const uint32_t* __restrict__ keys,
-                                                             const uint32_t* __restrict__ order, uint32_t n,
-                                                             const float4* __restrict__ leafbox,
+                                                             uint32_t n, const float4* __restrict__ leafbox,
                                                              float4* __restrict__ nodes,
                                                              float* __restrict__ bounds, TopArrays top) {
     __shared__ float box[6][kTreeBlock];  // by local node id: the box of a node whose parent is pending
@@ -571,10 +593,9 @@ __global__ void __launch_bounds__(kTreeBlock) k_tree_local(const uint32_t* __res
     const int tid = threadIdx.x;
     Box b = empty_box();
     if (tid < cnt) {
-        const uint32_t prim = order[blo + tid];
         diff[tid] = diff_at(keys, n, blo + tid);
         if (tid == 0) diff[cnt] = diff_at(keys, n, blo + cnt);
-        b = load_box(leafbox + 2 * (uint64_t)prim);
+        b = load_box(leafbox + 2 * (uint64_t)(blo + tid));
     }
     arrived[tid] = 0;
     __syncthreads();
@@ -799,7 +820,7 @@ RT_DEV float union_area(const float4& alo, const float4& ahi, const float4& blo,
 RT_DEV int32_t ploc_size(const int32_t* __restrict__ nsize, int32_t c) { return c >= 0 ? nsize[c] : 1; }
 
 __global__ void __launch_bounds__(256) k_ploc_init(const uint32_t* __restrict__ morder, uint32_t n,
-                                                    const float4* __restrict__ leafbox,
+                                                    const MeshSource* __restrict__ meshes, uint32_t n_sources,
                                                     int32_t* __restrict__ cid, float4* __restrict__ cbox,
                                                     uint32_t* __restrict__ pos_of,
                                                     int32_t* __restrict__ parent, int32_t* __restrict__ state) {
@@ -808,8 +829,11 @@ __global__ void __launch_bounds__(256) k_ploc_init(const uint32_t* __restrict__ 
     const uint32_t p = morder[i];
     pos_of[p] = i;
     cid[i] = ~(int32_t)p;
-    cbox[2 * (uint64_t)i] = leafbox[2 * (uint64_t)p];
-    cbox[2 * (uint64_t)i + 1] = leafbox[2 * (uint64_t)p + 1];
+    const MeshSource& src = mesh_of(meshes, n_sources, p);
+    uint32_t v[3];
+    float3 c[3];
+    load_corners(src.d, p - src.base, v, c);
+    store_box(cbox + 2 * (uint64_t)i, padded(corners_box(c)));
     if (i == 0) {
         parent[0] = -1;
         state[0] = (int32_t)n;
@@ -1699,12 +1723,13 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
     Workspace w = carve((char*)workspace, n);
 
     // 1. gather (one launch per mesh; the descriptor travels as a kernel argument)
-    uint32_t base = 0, nparts = 0;
+    uint32_t base = 0, nparts = 0, nsrc = 0;
     for (uint32_t m = 0; m < n_meshes; ++m) {
         const rt_mesh_desc& d = meshes[m];
         hipLaunchKernelGGL(k_gather, dim3(d.n_tris ? blocks_for(d.n_tris, 256) : 1), dim3(256), 0, s,
-                           d, m, n_meshes, base, w.cent, w.leafbox, w.tri_u, w.shade_u, sc->mesh_offsets,
-                           w.partial + 2 * (uint64_t)nparts);
+                           d, m, n_meshes, base, w.cent, sc->mesh_offsets, w.partial + 2 * (uint64_t)nparts,
+                           w.meshes + nsrc);
+        nsrc += d.n_tris ? 1 : 0;
         base += d.n_tris;
         nparts += blocks_for(d.n_tris, 256);
     }
@@ -1729,7 +1754,7 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
     if (ploc) {
         // 5. PLOC hierarchy (node boxes as it merges, scene bounds at the root), 6. leaf slots and
         // traversal refs, 7. leaf records in slot order, 8. 4-wide records
-        hipLaunchKernelGGL(k_ploc_init, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, n, w.leafbox,
+        hipLaunchKernelGGL(k_ploc_init, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, n, w.meshes, nsrc,
                            w.cid[0], w.cbox[0], w.pos_of, w.parent, w.state);
         const int iters = ploc_iterations(n);
         const uint32_t grid = std::min<uint32_t>(kPlocGrid, blocks_for(n, kPlocTile));
@@ -1766,18 +1791,18 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
                            w.nsize, w.nleft, w.nright, w.pos_of, w.scan, slot_order, w.slot_of, w.fslot);
         hipLaunchKernelGGL(k_ploc_refs, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n, w.nleft,
                            w.nright, w.nsize, w.slot_of, w.fslot, nodes);
-        hipLaunchKernelGGL(k_emit, dim3(blocks_for(4 * (uint64_t)n, 256)), dim3(256), 0, s, slot_order, n, w.tri_u,
-                           w.shade_u, (float4*)sc->tris, (float4*)sc->shade, (uint32_t*)sc->prim_slot);
+        hipLaunchKernelGGL(k_emit, dim3(blocks_for(n, 256)), dim3(256), 0, s, slot_order, n, w.meshes, nsrc,
+                           (float4*)nullptr, (float4*)sc->tris, (float4*)sc->shade, (uint32_t*)sc->prim_slot);
         hipLaunchKernelGGL(k_wide, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n,
                            (const float4*)nodes, (float4*)sc->nodes4);
         sc->root = n <= (uint32_t)kLeafMax ? leaf_ref(0, n) : 0;
     } else {
     // 5. emit, 6. tree (LBVH, or a PLOC tree found too deep)
-    hipLaunchKernelGGL(k_emit, dim3(blocks_for(4 * (uint64_t)n, 256)), dim3(256), 0, s, vi, n, w.tri_u, w.shade_u,
+    hipLaunchKernelGGL(k_emit, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, n, w.meshes, nsrc, w.leafbox,
                        (float4*)sc->tris, (float4*)sc->shade, (uint32_t*)sc->prim_slot);
     if (n > 1) {
         const uint32_t nb = blocks_for(n, kTreeBlock);
-        hipLaunchKernelGGL(k_tree_local, dim3(nb), dim3(kTreeBlock), 0, s, ki, vi, n, w.leafbox, nodes,
+        hipLaunchKernelGGL(k_tree_local, dim3(nb), dim3(kTreeBlock), 0, s, ki, n, w.leafbox, nodes,
                            sc->bounds, w.top);
         if (nb > 1) hipLaunchKernelGGL(k_tree_top, dim3(nb), dim3(kTopThreads), 0, s, ki, n, nodes, sc->bounds, w.top);
         hipLaunchKernelGGL(k_wide, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n,
