@@ -1,7 +1,7 @@
 // rt_build.hip — on-device LBVH construction for rendering/_raycaster.py:26-33
 // (Raycaster.__init__ -> _build_ads, a stub in the reference that only counts triangles).
 //
-// Pipeline (one stream; no host synchronisation except the PLOC depth check):
+// Pipeline (one stream; no host synchronisation):
 //   1. gather      per mesh: read MeshVertex P (rendering/_modeling.py:22-28) through the optional
 //                  int32 index list, write AABB centroids.
 //   2. bounds      min/max of the centroids per workgroup of the gather, folded by the next kernel.
@@ -444,6 +444,15 @@ __global__ void __launch_bounds__(256) k_order_merge(const uint32_t* __restrict_
     }
 }
 
+// Whether the LBVH kernels run: always (deep NULL), or where a PLOC tree turned out too deep (*deep set),
+// with `order` the Morton order instead of PLOC's slots. The device decides, so a PLOC build does not
+// wait for its stream.
+struct Fallback {
+    const uint32_t* deep;
+    const uint32_t* order;
+    RT_DEV bool taken() const { return !deep || *deep; }
+};
+
 // Copies `per` float4s of each of the block's `rows` records from LDS (record r at
 // stage[r * pitch]) to out[0 .. rows*per), one float4 per thread and instruction.
 RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t rows, uint32_t per,
@@ -455,12 +464,12 @@ RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t
 }
 
 // One thread per slot: the intersection record (p0, e1, e2, primitive id) and the shading record (three
-// normals, three uvs, mesh id) of its triangle, from the mesh's vertices; the padded leaf box of the slot if
-// `leafbox` is not NULL; the slot of the primitive. The block's records go out through LDS as consecutive
+// normals, three uvs, mesh id) of its triangle, from the mesh's vertices; the padded leaf box of the slot
+// for an LBVH; the slot of the primitive. The block's records go out through LDS as consecutive
 // float4s. Bound by memory: 180 B of stores per triangle, and the vertices, which neighbours in Morton
 // order share in L2. At 1.31 M triangles 72 us and 32 for the gather; records written in
 // primitive order by the gather and permuted here took 81 and 71.
-__global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order, uint32_t n,
+__global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ slots, Fallback fb, uint32_t n,
                                               const MeshSource* __restrict__ meshes, uint32_t n_sources,
                                               float4* __restrict__ leafbox, float4* __restrict__ tris,
                                               float4* __restrict__ shade, uint32_t* __restrict__ prim_slot) {
@@ -468,7 +477,8 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order
     __shared__ float4 stage[256 * kPitch];
     const uint64_t s0 = (uint64_t)blockIdx.x * 256;
     const uint32_t rows = n - s0 < 256 ? (uint32_t)(n - s0) : 256u;
-    const bool mine = threadIdx.x < rows;
+    const bool mine = threadIdx.x < rows, taken = fb.taken();
+    const uint32_t* __restrict__ order = fb.deep && taken ? fb.order : slots;
     float4 tri[3], shd[4];
     Box box = empty_box();
     if (mine) {
@@ -514,7 +524,7 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ order
     if (mine) { st[0] = tri[0]; st[1] = tri[1]; st[2] = tri[2]; }
     __syncthreads();
     store_staged(tris + 3 * s0, stage, rows, 3, kPitch);
-    if (!leafbox) return;
+    if (!taken) return;
     __syncthreads();
     if (mine) store_box(st, box);
     __syncthreads();
@@ -577,7 +587,7 @@ RT_DEV void store_bounds(float* __restrict__ bounds, const Box& b) {
 }
 
 __global__ void __launch_bounds__(kTreeBlock) k_tree_local(const uint32_t* __restrict__ keys,
-                                                             uint32_t n, const float4* __restrict__ leafbox,
+                                                             uint32_t n, Fallback fb, const float4* __restrict__ leafbox,
                                                              float4* __restrict__ nodes,
                                                              float* __restrict__ bounds, TopArrays top) {
     __shared__ float box[6][kTreeBlock];  // by local node id: the box of a node whose parent is pending
@@ -588,6 +598,7 @@ __global__ void __launch_bounds__(kTreeBlock) k_tree_local(const uint32_t* __res
     __shared__ int32_t sdiff[kTopMax + 2];  // diff there
     __shared__ float sbox[kTopMax + 2][6];
     __shared__ int32_t nseg;
+    if (!fb.taken()) return;
     const int64_t blo = (int64_t)blockIdx.x * kTreeBlock;
     const int cnt = (int)(n - blo < kTreeBlock ? n - blo : kTreeBlock);
     const int tid = threadIdx.x;
@@ -741,9 +752,10 @@ RT_DEV Box wave_range_box(const TopArrays& top, int64_t lo, int64_t hi1, uint32_
     return b;
 }
 
-__global__ void __launch_bounds__(kTopThreads) k_tree_top(const uint32_t* __restrict__ keys, uint32_t n,
+__global__ void __launch_bounds__(kTopThreads) k_tree_top(const uint32_t* __restrict__ keys, uint32_t n, Fallback fb,
                                                   float4* __restrict__ nodes, float* __restrict__ bounds,
                                                   TopArrays top) {
+    if (!fb.taken()) return;
     const int lane = threadIdx.x & 63;
     const uint32_t nb = gridDim.x, cnt = top.count[blockIdx.x];
     for (uint32_t i = threadIdx.x >> 6; i < cnt; i += blockDim.x >> 6) {
@@ -1350,7 +1362,8 @@ RT_DEV uint32_t ploc_minpos(int32_t x, const int32_t* __restrict__ nleft, const 
     return best;
 }
 
-__global__ void __launch_bounds__(256) k_ploc_leafroots(uint32_t n, const uint32_t* __restrict__ morder,
+__global__ void __launch_bounds__(256) k_ploc_leafroots(uint32_t n, const uint32_t* __restrict__ deep,
+                                                         const uint32_t* __restrict__ morder,
                                                          const int32_t* __restrict__ parent,
                                                          const int32_t* __restrict__ nsize,
                                                          const int32_t* __restrict__ nleft,
@@ -1358,7 +1371,7 @@ __global__ void __launch_bounds__(256) k_ploc_leafroots(uint32_t n, const uint32
                                                          const uint32_t* __restrict__ pos_of,
                                                          uint32_t* __restrict__ scan) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    if (i >= n || *deep) return;
     const int32_t x = ploc_leaf_root(n, parent, nsize, morder[i]);
     scan[i] = ploc_minpos(x, nleft, nright, pos_of) == i ? (uint32_t)ploc_size(nsize, x) : 0u;
 }
@@ -1417,7 +1430,8 @@ __global__ void __launch_bounds__(256) k_scan_apply(uint32_t n, uint32_t* __rest
 
 // slots of the leaf root whose smallest Morton position is i: its triangles left to right from
 // the root's first slot; first slots of its internal nodes
-__global__ void __launch_bounds__(256) k_ploc_slots(uint32_t n, const uint32_t* __restrict__ morder,
+__global__ void __launch_bounds__(256) k_ploc_slots(uint32_t n, const uint32_t* __restrict__ deep,
+                                                         const uint32_t* __restrict__ morder,
                                                      const int32_t* __restrict__ parent,
                                                      const int32_t* __restrict__ nsize,
                                                      const int32_t* __restrict__ nleft,
@@ -1428,7 +1442,7 @@ __global__ void __launch_bounds__(256) k_ploc_slots(uint32_t n, const uint32_t* 
                                                      uint32_t* __restrict__ slot_of,
                                                      uint32_t* __restrict__ fslot) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    if (i >= n || *deep) return;
     const int32_t x = ploc_leaf_root(n, parent, nsize, morder[i]);
     if (ploc_minpos(x, nleft, nright, pos_of) != i) return;
     uint32_t next = scan[i];
@@ -1451,14 +1465,15 @@ __global__ void __launch_bounds__(256) k_ploc_slots(uint32_t n, const uint32_t* 
 
 // traversal refs of every internal node: a child of more than kLeafMax triangles by id, else the
 // leaf of its slots
-__global__ void __launch_bounds__(256) k_ploc_refs(uint32_t n, const int32_t* __restrict__ nleft,
+__global__ void __launch_bounds__(256) k_ploc_refs(uint32_t n, const uint32_t* __restrict__ deep,
+                                                    const int32_t* __restrict__ nleft,
                                                     const int32_t* __restrict__ nright,
                                                     const int32_t* __restrict__ nsize,
                                                     const uint32_t* __restrict__ slot_of,
                                                     const uint32_t* __restrict__ fslot,
                                                     float4* __restrict__ nodes) {
     const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= n - 1) return;
+    if (x >= n - 1 || *deep) return;
     auto tref = [&](int32_t c) -> int32_t {
         if (c < 0) return leaf_ref(slot_of[~c], 1u);
         if (nsize[c] > kLeafMax) return c;
@@ -1559,10 +1574,11 @@ __global__ void k_empty_bounds(float* __restrict__ bounds) {
     bounds[3] = bounds[7] = 0.0f;
 }
 
-__global__ void __launch_bounds__(256) k_copy_u32(const uint32_t* __restrict__ a,
-                                                   uint32_t* __restrict__ b, uint32_t n) {
+__global__ void __launch_bounds__(256) k_copy_if(const uint32_t* __restrict__ deep,
+                                                  const uint32_t* __restrict__ a, uint32_t* __restrict__ b,
+                                                  uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = a[i];
+    if (i < n && *deep) b[i] = a[i];
 }
 
 inline uint32_t blocks_for(uint64_t n, uint32_t per) { return (uint32_t)((n + per - 1) / per); }
@@ -1735,7 +1751,7 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
     }
     // 2. - 4. centroid bounds, Morton codes and their sort, into the caller's arrays where it wants them
     // (PLOC writes the order of its own slots there)
-    bool ploc = n > 1 && tu.builder == RT_BUILD_PLOC;
+    const bool ploc = n > 1 && tu.builder == RT_BUILD_PLOC;
     uint32_t* ki = keys_out ? keys_out : w.keys0;
     uint32_t* vi = order_out && !ploc ? order_out : w.vals0;
     if (n <= kSmallMax) {
@@ -1751,9 +1767,10 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
     }
     float4* nodes = (float4*)sc->nodes;
     const uint32_t nchunk = blocks_for(n, kPlocChunk);
+    uint32_t* slots = vi;       // primitive of each slot
+    Fallback fb{nullptr, nullptr};
     if (ploc) {
-        // 5. PLOC hierarchy (node boxes as it merges, scene bounds at the root), 6. leaf slots and
-        // traversal refs, 7. leaf records in slot order, 8. 4-wide records
+        // 5. PLOC hierarchy (node boxes as it merges, scene bounds at the root)
         hipLaunchKernelGGL(k_ploc_init, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, n, w.meshes, nsrc,
                            w.cid[0], w.cbox[0], w.pos_of, w.parent, w.state);
         const int iters = ploc_iterations(n);
@@ -1768,50 +1785,39 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
         hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(1024), 0, s, iters & 1, n, w.state, w.nn, w.cid[0],
                            w.cid[1], w.cbox[0], w.cbox[1], w.nleft, w.nright, w.nsize, w.parent, nodes,
                            sc->bounds);
-        // a tree deeper than the traversal stacks allow is replaced by the LBVH of the same keys;
-        // this reads one word back, so a PLOC build waits for its stream here
+        // a tree deeper than the traversal stacks allow is replaced by the LBVH of the same keys
         hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, s, w.depth);
         hipLaunchKernelGGL(k_ploc_depth, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, w.parent, w.depth);
-        uint32_t deep = 0;
-        int e = check_hip(hipMemcpyAsync(&deep, w.depth, 4, hipMemcpyDeviceToHost, s), "rt_scene_build(PLOC depth)");
-        if (!e) e = check_hip(hipStreamSynchronize(s), "rt_scene_build(PLOC depth)");
-        if (e) return e;
-        ploc = deep == 0;
-        if (!ploc && order_out)
-            hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, order_out, n);
-    }
-    if (ploc) {
-        uint32_t* slot_order = order_out ? order_out : w.slot_order;
-        hipLaunchKernelGGL(k_ploc_leafroots, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, vi, w.parent,
+        // 6. leaf slots and traversal refs
+        slots = order_out ? order_out : w.slot_order;
+        fb = {w.depth, vi};
+        hipLaunchKernelGGL(k_ploc_leafroots, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, w.depth, vi, w.parent,
                            w.nsize, w.nleft, w.nright, w.pos_of, w.scan);
         hipLaunchKernelGGL(k_scan_chunks, dim3(nchunk), dim3(256), 0, s, n, w.scan, w.part);
         hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, nchunk, w.part);
         hipLaunchKernelGGL(k_scan_apply, dim3(nchunk), dim3(256), 0, s, n, w.scan, w.part);
-        hipLaunchKernelGGL(k_ploc_slots, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, vi, w.parent,
-                           w.nsize, w.nleft, w.nright, w.pos_of, w.scan, slot_order, w.slot_of, w.fslot);
-        hipLaunchKernelGGL(k_ploc_refs, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n, w.nleft,
+        hipLaunchKernelGGL(k_ploc_slots, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, w.depth, vi, w.parent,
+                           w.nsize, w.nleft, w.nright, w.pos_of, w.scan, slots, w.slot_of, w.fslot);
+        hipLaunchKernelGGL(k_ploc_refs, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n, w.depth, w.nleft,
                            w.nright, w.nsize, w.slot_of, w.fslot, nodes);
-        hipLaunchKernelGGL(k_emit, dim3(blocks_for(n, 256)), dim3(256), 0, s, slot_order, n, w.meshes, nsrc,
-                           (float4*)nullptr, (float4*)sc->tris, (float4*)sc->shade, (uint32_t*)sc->prim_slot);
-        hipLaunchKernelGGL(k_wide, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n,
-                           (const float4*)nodes, (float4*)sc->nodes4);
-        sc->root = n <= (uint32_t)kLeafMax ? leaf_ref(0, n) : 0;
-    } else {
-    // 5. emit, 6. tree (LBVH, or a PLOC tree found too deep)
-    hipLaunchKernelGGL(k_emit, dim3(blocks_for(n, 256)), dim3(256), 0, s, vi, n, w.meshes, nsrc, w.leafbox,
+    }
+    // leaf records; the LBVH tree, or the one in place of a PLOC tree found too deep; 4-wide records
+    hipLaunchKernelGGL(k_emit, dim3(blocks_for(n, 256)), dim3(256), 0, s, slots, fb, n, w.meshes, nsrc, w.leafbox,
                        (float4*)sc->tris, (float4*)sc->shade, (uint32_t*)sc->prim_slot);
+    if (ploc && order_out)
+        hipLaunchKernelGGL(k_copy_if, dim3(blocks_for(n, 256)), dim3(256), 0, s, w.depth, vi, order_out, n);
     if (n > 1) {
         const uint32_t nb = blocks_for(n, kTreeBlock);
-        hipLaunchKernelGGL(k_tree_local, dim3(nb), dim3(kTreeBlock), 0, s, ki, n, w.leafbox, nodes,
+        hipLaunchKernelGGL(k_tree_local, dim3(nb), dim3(kTreeBlock), 0, s, ki, n, fb, w.leafbox, nodes,
                            sc->bounds, w.top);
-        if (nb > 1) hipLaunchKernelGGL(k_tree_top, dim3(nb), dim3(kTopThreads), 0, s, ki, n, nodes, sc->bounds, w.top);
+        if (nb > 1)
+            hipLaunchKernelGGL(k_tree_top, dim3(nb), dim3(kTopThreads), 0, s, ki, n, fb, nodes, sc->bounds, w.top);
         hipLaunchKernelGGL(k_wide, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n,
                            (const float4*)nodes, (float4*)sc->nodes4);
         sc->root = n <= (uint32_t)kLeafMax ? leaf_ref(0, n) : 0;
     } else {
         hipLaunchKernelGGL(k_single_leaf_bounds, dim3(1), dim3(1), 0, s, w.leafbox, sc->bounds);
         sc->root = ~0;
-    }
     }
     return check_launch("rt_scene_build");
 }
