@@ -389,10 +389,12 @@ class Raycaster:
     def _on_stream(self):
         """Runs the block with this scene's stream current (allocations, copies and kernels all on
         it), after the work already queued on the caller's stream."""
-        ts = self._torch_stream()
         cur = torch.cuda.current_stream()
-        if ts != cur:
-            ts.wait_stream(cur)
+        ts = self._stream if self._stream is not None else cur
+        if ts == cur:
+            yield ts
+            return
+        ts.wait_stream(cur)
         with torch.cuda.stream(ts):
             yield ts
 
@@ -418,46 +420,62 @@ class Raycaster:
             sizes = N.rt_scene_sizes()
             N.check(lib.rt_scene_sizes_for(n_tris, ctypes.byref(sizes)), "rt_scene_sizes_for")
             dev = torch.device("cuda")
-            # the scene's arrays are 256-byte-aligned slices of one allocation (one allocator
-            # call); allocated on the build's stream, so torch orders reuse of the freed workspace
-            # after the build kernels
-            parts = [("_nodes", sizes.nodes_bytes, torch.uint8), ("_nodes4", sizes.nodes4_bytes, torch.uint8),
-                     ("_tris", sizes.tris_bytes, torch.uint8), ("_shade", sizes.shade_bytes, torch.uint8),
-                     ("_bounds", 32, torch.float32), ("_mesh_offsets", 4 * (len(self.models) + 1), torch.int32),
-                     ("_prim_slot", sizes.prim_slot_bytes, torch.int32),
-                     ("keys", 4 * max(1, n_tris), torch.int32), ("order", 4 * max(1, n_tris), torch.int32)]
-            offsets, total = [], 0
-            for _, nbytes, _ in parts:
-                offsets.append(total)
-                total += (int(nbytes) + 255) // 256 * 256
-            arena = torch.empty(total, dtype=torch.uint8, device=dev)
+            # the scene's arrays are 256-byte-aligned parts of one allocation (one allocator call);
+            # allocated on the build's stream, so torch orders reuse of the freed workspace after the
+            # build kernels. The kernels get addresses; tensors over the parts are made when asked for
+            # (_part): as slices made here they cost half of a small scene's build.
+            n4 = 4 * max(1, n_tris)
+            sizes_of = {"nodes": sizes.nodes_bytes, "nodes4": sizes.nodes4_bytes, "tris": sizes.tris_bytes,
+                        "shade": sizes.shade_bytes, "bounds": 32, "mesh_offsets": 4 * (len(self.models) + 1),
+                        "prim_slot": sizes.prim_slot_bytes, "keys": n4, "order": n4}
+            total, self._parts = 0, {}
+            for name, nbytes in sizes_of.items():
+                self._parts[name] = (total, nbytes)
+                total += (nbytes + 255) // 256 * 256
+            self._arena = torch.empty(total // 4, dtype=torch.int32, device=dev)
             ws = torch.empty(sizes.workspace_bytes, dtype=torch.uint8, device=dev)
-            for (name, nbytes, dtype), off in zip(parts, offsets):
-                setattr(self, name, arena[off:off + int(nbytes)].view(dtype))
+            at = self._arena.data_ptr()
             sc = N.rt_scene()
             sc.n_tris = n_tris
             sc.n_meshes = len(self.models)
-            sc.nodes = self._nodes.data_ptr()
-            sc.nodes4 = self._nodes4.data_ptr()
-            sc.tris = self._tris.data_ptr()
-            sc.shade = self._shade.data_ptr()
-            sc.mesh_offsets = self._mesh_offsets.data_ptr()
-            sc.bounds = self._bounds.data_ptr()
-            sc.prim_slot = self._prim_slot.data_ptr()
+            for name in ("nodes", "nodes4", "tris", "shade", "mesh_offsets", "bounds", "prim_slot"):
+                setattr(sc, name, at + self._parts[name][0])
             code = lib.rt_scene_build(descs, len(self.models), ctypes.byref(sc), ws.data_ptr(),
-                                      sizes.workspace_bytes, self.keys.data_ptr(),
-                                      self.order.data_ptr(), tuning_arg(self._tuning),
+                                      sizes.workspace_bytes, at + self._parts["keys"][0],
+                                      at + self._parts["order"][0], tuning_arg(self._tuning),
                                       N.stream_handle(ts))
             N.check(code, "rt_scene_build")
             del ws
         self._scene = sc
         self._keep = keep
 
+    def _part(self, name, shape, dtype=torch.int32):
+        """Tensor of one of the scene's arrays, a view of its allocation."""
+        a = self._arena if dtype == torch.int32 else self._arena.view(dtype)
+        return a.as_strided(shape, (shape[1], 1) if len(shape) == 2 else (1,), self._parts[name][0] // 4)
+
+    def _bytes(self, name):
+        off, nbytes = self._parts[name]
+        return self._arena.view(torch.uint8)[off:off + nbytes]
+
+    _nodes = property(lambda self: self._bytes("nodes"))
+    _nodes4 = property(lambda self: self._bytes("nodes4"))
+    _tris = property(lambda self: self._bytes("tris"))
+    _shade = property(lambda self: self._bytes("shade"))
+
+    @property
+    def keys(self):
+        """Sorted Morton keys, int32 [max(n_tris, 1)]."""
+        return self._part("keys", (max(1, self.n_tris),))
+
+    @property
+    def order(self):
+        """Primitive of each slot, int32 [max(n_tris, 1)]."""
+        return self._part("order", (max(1, self.n_tris),))
+
     def device_bytes(self) -> int:
         """Device memory held by the built scene (BVH, triangle and shading records, keys)."""
-        ts = [self._nodes, self._nodes4, self._tris, self._shade, self._bounds, self._mesh_offsets,
-              self._prim_slot, self.keys, self.order]
-        return int(sum(t.numel() * t.element_size() for t in ts))
+        return int(sum(nbytes for _, nbytes in self._parts.values()))
 
     def release_inputs(self):
         """Drops the references to the input meshes' device buffers; queries and renders only read
@@ -474,17 +492,18 @@ class Raycaster:
         """Raw device arrays of the built scene: nodes [n-1,16] f32, tris [n,12] f32,
         shade [n,16] f32, bounds [8], sorted Morton keys and primitive order."""
         n = self.n_tris
-        ni = max(n - 1, 1)
+        m = max(n - 1, 0)
+        f32 = torch.float32
         return {
-            "nodes": self._nodes.view(torch.float32).view(ni, 16)[: max(n - 1, 0)],
-            "nodes4": self._nodes4.view(torch.float32).view(ni, 32)[: max(n - 1, 0)],
-            "tris": self._tris.view(torch.float32).view(max(n, 1), 12)[:n],
-            "shade": self._shade.view(torch.float32).view(max(n, 1), 16)[:n],
-            "bounds": self._bounds,
-            "keys": self.keys[:n],
-            "order": self.order[:n],
-            "prim_slot": self._prim_slot[:n],
-            "mesh_offsets": self._mesh_offsets,
+            "nodes": self._part("nodes", (m, 16), f32),
+            "nodes4": self._part("nodes4", (m, 32), f32),
+            "tris": self._part("tris", (n, 12), f32),
+            "shade": self._part("shade", (n, 16), f32),
+            "bounds": self._part("bounds", (8,), f32),
+            "keys": self._part("keys", (n,)),
+            "order": self._part("order", (n,)),
+            "prim_slot": self._part("prim_slot", (n,)),
+            "mesh_offsets": self._part("mesh_offsets", (len(self.mesh_tri_counts) + 1,)),
         }
 
     def export_ads(self):
