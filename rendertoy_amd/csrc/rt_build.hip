@@ -809,8 +809,8 @@ __global__ void __launch_bounds__(256) k_ploc_depth(uint32_t n, const int32_t* _
 // order. An iteration with no mutual pair (possible only with NaN boxes) merges positions 0 and 1.
 // The k-th node created (over iterations, in position order) gets id n-2-k: the root is 0 and
 // children have larger ids than their parents. Large iterations run as two grid launches
-// (the pairs and their counts per tile; compaction), which took 297 us of a build of 151,380 triangles
-// where four (neighbours, counts, offsets, compaction) took 598; once at most kPlocTail clusters remain,
+// (the pairs and their counts per tile; compaction), which take 9 us an iteration of a build of 151,380 triangles
+// where four (neighbours, counts, offsets, compaction) took 18; once at most kPlocTail clusters remain,
 // one workgroup finishes in a single launch. Subtrees of at most
 // kLeafMax triangles whose parent is larger become leaves: leaf roots take consecutive slot ranges
 // in the order of their smallest Morton position, their triangles left to right.
@@ -818,7 +818,9 @@ constexpr int kPlocRadius = 16;
 constexpr int kPlocTile = 256;        // clusters per neighbour-search tile (one per thread)
 constexpr int kPlocChunk = 1024;      // values per chunk of the slot scan (4 per thread)
 constexpr int kPlocGrid = 1024;       // blocks of the grid-stride iteration kernels
-constexpr int32_t kPlocTail = 4096;   // cluster count handed to the one-workgroup tail
+// cluster count handed to the one-workgroup tail: above 2,048 an iteration there (15 to 20 us) costs more than
+// two launches (9 us); from 4,096 on a build of 151,380 triangles took 650 us, from 2,048 on 590
+constexpr int32_t kPlocTail = 2048;
 
 // state[4 * parity]: clusters m, nodes created, buffer parity of the clusters
 
@@ -1125,7 +1127,7 @@ RT_DEV int32_t ploc_nn_lanes(int32_t i, int32_t m, int lg, int q, AreaTo area) {
 // clusters (only if the launched iterations merged less than expected) through memory, the rest in LDS,
 // where a search costs no L2 round trips, sizes need no loads and the compaction counts by ballots.
 // From 512 clusters down several lanes share a search. The 65 or so iterations from 4,096 clusters on
-// took 499 us through memory, 229 like this.
+// took 499 us through memory, 229 like this; those from 2,048 on take 120.
 __global__ void __launch_bounds__(1024) k_ploc_tail(int slot, uint32_t n, int32_t* __restrict__ state,
                                                      int32_t* __restrict__ nn, int32_t* __restrict__ cid0,
                                                      int32_t* __restrict__ cid1, float4* __restrict__ cbox0,
@@ -1264,7 +1266,7 @@ __global__ void __launch_bounds__(1024) k_ploc_tail(int slot, uint32_t n, int32_
             if (lane == 0) wcount[c * kWaves + wave] = (uint32_t)__popcll(kb[c]) | ((uint32_t)__popcll(mb[c]) << 16);
         }
         __syncthreads();
-        const uint32_t own = wcount[lane];  // kPer * kWaves = 64 counts, scanned by every wave
+        const uint32_t own = lane < kPer * kWaves ? wcount[lane] : 0u;  // every wave scans the counts
         uint32_t incl = own;
         for (int x = 1; x < 64; x <<= 1) {
             const uint32_t v = __shfl_up(incl, x);

@@ -42,9 +42,9 @@ def _ploc(ren, mesh):
 
 
 @pytest.mark.parametrize("kind", ["spread", "equal", "crowded"])
-@pytest.mark.parametrize("n", [2, 3, 64, 65, 129, 257, 513, 1025, 4096, 4097, 4353, 9000])
+@pytest.mark.parametrize("n", [2, 3, 64, 65, 129, 257, 513, 1025, 2048, 2049, 2305, 4097, 9000])
 def test_ploc_sizes(ren, n, kind):
-    """PLOC at the widths of a search in its last workgroup, at the hand-over to it (4,096 clusters) and at
+    """PLOC at the widths of a search in its last workgroup, at the hand-over to it (2,048 clusters) and at
     the tiles before it."""
     assert_build_equal(*_ploc(ren, _mesh(n, kind)))
 
