@@ -453,13 +453,21 @@ struct Fallback {
     RT_DEV bool taken() const { return !deep || *deep; }
 };
 
+// Store of arrays that no kernel of the build reads again (leaf records, 4-wide nodes): past the caches, which
+// then keep what the next kernels read. At 1.31 M triangles the emit went from 72 to 63 us, the 4-wide nodes
+// from 45 to 39 and the next build's gather, which finds the vertices, from 32 to 21.
+RT_DEV void store_last(float4* p, const float4& v) {
+    typedef float vec4 __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store((vec4){v.x, v.y, v.z, v.w}, (vec4*)p);
+}
+
 // Copies `per` float4s of each of the block's `rows` records from LDS (record r at
 // stage[r * pitch]) to out[0 .. rows*per), one float4 per thread and instruction.
 RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t rows, uint32_t per,
                          uint32_t pitch) {
     for (uint32_t q = threadIdx.x; q < rows * per; q += blockDim.x) {
         const uint32_t r = q / per;
-        out[q] = stage[r * pitch + (q - r * per)];
+        store_last(out + q, stage[r * pitch + (q - r * per)]);
     }
 }
 
@@ -467,7 +475,7 @@ RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t
 // normals, three uvs, mesh id) of its triangle, from the mesh's vertices; the padded leaf box of the slot
 // for an LBVH; the slot of the primitive. The block's records go out through LDS as consecutive
 // float4s. Bound by memory: 180 B of stores per triangle, and the vertices, which neighbours in Morton
-// order share in L2. At 1.31 M triangles 72 us and 32 for the gather; records written in
+// order share in L2. At 1.31 M triangles 63 us and 21 for the gather; records written in
 // primitive order by the gather and permuted here took 81 and 71.
 __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ slots, Fallback fb, uint32_t n,
                                               const MeshSource* __restrict__ meshes, uint32_t n_sources,
@@ -528,7 +536,7 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ slots
     __syncthreads();
     if (mine) store_box(st, box);
     __syncthreads();
-    store_staged(leafbox + 2 * s0, stage, rows, 2, kPitch);
+    for (uint32_t q = threadIdx.x; q < rows * 2; q += 256) leafbox[2 * s0 + q] = stage[(q >> 1) * kPitch + (q & 1)];
 }
 
 // ---- tree ----
@@ -1557,7 +1565,7 @@ __global__ void __launch_bounds__(256) k_wide(uint32_t n, const float4* __restri
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const uint32_t q = j * 256 + threadIdx.x;  // float4 q of the block's output
-        if (q < rows * 8) out[q] = stage[(q >> 3) * kPitch + (q & 7)];
+        if (q < rows * 8) store_last(out + q, stage[(q >> 3) * kPitch + (q & 7)]);
     }
 }
 
