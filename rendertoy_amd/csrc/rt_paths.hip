@@ -10,6 +10,7 @@
 //   k_paths_primary  camera rays (QUAD: a 4x4 tile per one-wave workgroup; else an 8x8 tile per
 //                    wave, AUTO coherence rule), hits append a bounce ray
 //                    to queue 0 (wave ballot + one atomic per wave = compaction)
+//                    (small frames: k_paths_primary_group, k_paths_bounce_group, 16 or 64 lanes a ray)
 //   k_paths_bounce   per depth: the waves share the queue's 64-ray groups (count read on the
 //                    device), per-lane walks with refill; each ray records the slot it hit
 //   k_paths_emit     per depth, in queue order: misses write their sample, hits append their
@@ -157,6 +158,27 @@ __global__ void k_paths_init(PathArgs a) {
     if (threadIdx.x <= a.bounces) a.counts[threadIdx.x] = threadIdx.x == 0 ? a.W * a.H * a.spp : 0u;
 }
 
+// Camera ray of sample s of a pixel.
+RT_DEV Ray sample_ray(const rt_camera& cam, const PathArgs& a, uint32_t col, uint32_t row, uint32_t pixel, uint32_t s) {
+    const uint4 rnd = philox4x32_10(make_uint4(pixel, s, 0u, 0u), a.key0, a.key1);
+    const float fx = (float)col + unit_float(rnd.x), fy = (float)row + unit_float(rnd.y);
+    const float nx = fx / (float)a.W * 2.0f - 1.0f, ny = 1.0f - fy / (float)a.H * 2.0f;
+    const float x = fmaf(nx, cam.right[0], fmaf(ny, cam.up[0], cam.forward[0]));
+    const float y = fmaf(nx, cam.right[1], fmaf(ny, cam.up[1], cam.forward[1]));
+    const float z = fmaf(nx, cam.right[2], fmaf(ny, cam.up[2], cam.forward[2]));
+    const float il = 1.0f / sqrtf(fmaf(x, x, fmaf(y, y, z * z)));
+    Ray r;
+    r.ox = cam.eye[0];
+    r.oy = cam.eye[1];
+    r.oz = cam.eye[2];
+    r.dx = x * il;
+    r.dy = y * il;
+    r.dz = z * il;
+    r.tmin = 0.0f;
+    r.tmax = INFINITY;
+    return r;
+}
+
 // Camera rays, for every sample in turn (sample s of pixel p jittered by the first two Philox
 // words of counter (p, s, 0, 0)); the pixel layout per traversal is below.
 template <int PM>
@@ -202,22 +224,7 @@ __global__ void __launch_bounds__(256) k_paths_primary(SceneArgs sc, rt_camera c
             __syncthreads();
         }
         const bool live = valid && s < a.spp;
-        const uint4 rnd = philox4x32_10(make_uint4(pixel, s, 0u, 0u), a.key0, a.key1);
-        const float fx = (float)col + unit_float(rnd.x), fy = (float)row + unit_float(rnd.y);
-        const float nx = fx / (float)a.W * 2.0f - 1.0f, ny = 1.0f - fy / (float)a.H * 2.0f;
-        const float x = fmaf(nx, cam.right[0], fmaf(ny, cam.up[0], cam.forward[0]));
-        const float y = fmaf(nx, cam.right[1], fmaf(ny, cam.up[1], cam.forward[1]));
-        const float z = fmaf(nx, cam.right[2], fmaf(ny, cam.up[2], cam.forward[2]));
-        const float il = 1.0f / sqrtf(fmaf(x, x, fmaf(y, y, z * z)));
-        Ray r;
-        r.ox = cam.eye[0];
-        r.oy = cam.eye[1];
-        r.oz = cam.eye[2];
-        r.dx = x * il;
-        r.dy = y * il;
-        r.dz = z * il;
-        r.tmin = 0.0f;
-        r.tmax = INFINITY;
+        const Ray r = sample_ray(cam, a, col, row, pixel, s);
         Hit h;
         if constexpr (QL) {
             // leaf records in pairs: 94 VGPRs and 5 waves per SIMD instead of 111 and 4; the 4-spp
@@ -261,6 +268,76 @@ __global__ void __launch_bounds__(256) k_paths_primary(SceneArgs sc, rt_camera c
     }
 }
 
+// Camera rays of a small frame, G lanes per sample (group_walk): samples of a pixel consecutive, pixels in
+// rows of 8x8 blocks, 1024 / G samples per workgroup, whose bounces go to queue 0 with one reservation.
+template <int G>
+__global__ void __launch_bounds__(1024) k_paths_primary_group(SceneArgs sc, rt_camera cam, PathArgs a, uint32_t tiles_x8) {
+    constexpr uint32_t kSamples = 1024 / G;
+    __shared__ int32_t stk[16][kGroupWords];
+    __shared__ float4 stage[kSamples * 3];
+    __shared__ uint32_t s_count, s_base;
+    const uint32_t item = blockIdx.x * kSamples + threadIdx.x / G, p = item / a.spp, s = item - p * a.spp;
+    const uint32_t blk = p >> 6, col = (blk % tiles_x8) * 8 + (p & 7), row = (blk / tiles_x8) * 8 + ((p >> 3) & 7);
+    const bool live = col < a.W && row < a.H;
+    const uint32_t pixel = live ? row * a.W + col : 0u, id = pixel * a.spp + s;
+    if (threadIdx.x == 0) s_count = 0;
+    __syncthreads();
+    const Ray r = sample_ray(cam, a, col, row, pixel, s);
+    Hit h;
+    group_walk<false, G>(sc.nodes4, sc.tris, sc.root, r, live, -1, h, stk[threadIdx.x >> 6]);
+    const bool lead = (threadIdx.x & (G - 1)) == 0, hit = live && h.prim >= 0, go = hit && lead && a.bounces > 0;
+    if (live && lead) a.samples[id] = hit ? 0.0f : a.sky;
+    if (go) {
+        refine_hit(sc.tris, r, h);
+        float4 e0, e1, e2;
+        bounce_entry(sc, a, r, h, true, id, 1u, 1.0f, e0, e1, e2);
+        float4* e = stage + atomicAdd(&s_count, 1u) * 3u;  // LDS; the queue's order enters no result
+        e[0] = e0;
+        e[1] = e1;
+        e[2] = e2;
+    }
+    __syncthreads();
+    const uint32_t staged = s_count;
+    if (threadIdx.x == 0 && staged) s_base = atomicAdd(&a.counts[1], staged);
+    __syncthreads();
+    for (uint32_t x = threadIdx.x; x < staged * 3u; x += 1024) a.q[0][(size_t)s_base * 3 + x] = stage[x];
+}
+
+RT_DEV int32_t load_bounce(const PathArgs& a, const float4* qi, uint32_t i, Ray& r) {
+    const float4 e0 = qi[(size_t)i * 3], e1 = qi[(size_t)i * 3 + 1], e2 = qi[(size_t)i * 3 + 2];
+    r.ox = e0.x;
+    r.oy = e0.y;
+    r.oz = e0.z;
+    r.dx = e1.x;
+    r.dy = e1.y;
+    r.dz = e1.z;
+    r.tmin = a.tmin;
+    r.tmax = INFINITY;
+    return __float_as_int(e2.x);
+}
+
+// Rays of depth k of a small frame, G lanes per ray (group_walk), the entries as k_paths_bounce writes them.
+template <int G>
+__global__ void __launch_bounds__(64) k_paths_bounce_group(SceneArgs sc, PathArgs a, uint32_t k) {
+    __shared__ int32_t stk[kGroupWords];
+    constexpr uint32_t kRays = 64 / G;
+    const uint32_t n = a.counts[k];
+    float4* qi = a.q[(k - 1) & 1];
+    for (uint32_t base = blockIdx.x * kRays; base < n; base += gridDim.x * kRays) {
+        const uint32_t i = base + threadIdx.x / G;
+        const bool want = i < n;
+        Ray r;
+        const int32_t skip = load_bounce(a, qi, want ? i : 0u, r);
+        Hit h;
+        group_walk<false, G>(sc.nodes4, sc.tris, sc.root, r, want, skip, h, stk);
+        if (want && (threadIdx.x & (G - 1)) == 0) {
+            float* e2 = (float*)(qi + (size_t)i * 3 + 2);
+            e2[1] = __int_as_float(h.slot);
+            e2[2] = h.t;
+        }
+    }
+}
+
 // Rays of depth k, queue (k-1)&1 (its count written by the previous kernel on the stream): per-lane
 // walks of the 4-wide nodes with refill (refill_walks), the grid's waves sharing the queue's 64-ray
 // groups. Each finished ray records the triangle slot it hit (-1: none) and its FP32 t in its own
@@ -277,18 +354,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
     // 128 (4 waves per SIMD) without scratch
     refill_walks<false, RT_TRAVERSAL_LANE, RT_PARK_PATHS, true, false>(
         sc, n, gridDim.x, refill_slot(blockIdx.x, 0, 1, gridDim.x), stk + threadIdx.x, 64, lane_stack, ovf, pk,
-        [&](uint32_t i, Ray& r) -> int32_t {
-            const float4 e0 = qi[(size_t)i * 3], e1 = qi[(size_t)i * 3 + 1], e2 = qi[(size_t)i * 3 + 2];
-            r.ox = e0.x;
-            r.oy = e0.y;
-            r.oz = e0.z;
-            r.dx = e1.x;
-            r.dy = e1.y;
-            r.dz = e1.z;
-            r.tmin = a.tmin;
-            r.tmax = INFINITY;
-            return __float_as_int(e2.x);
-        },
+        [&](uint32_t i, Ray& r) -> int32_t { return load_bounce(a, qi, i, r); },
         [&](bool fin, uint32_t i, const Ray&, Hit& h) {
             if (fin) {
                 float* e2 = (float*)(qi + (size_t)i * 3 + 2);
@@ -379,6 +445,21 @@ __global__ void __launch_bounds__(256) k_paths_resolve(PathArgs a, float* __rest
     if (counts_out && p <= a.bounces) counts_out[p] = a.counts[p];
 }
 
+// Frames of n samples whose camera rays and bounces are walked by groups of lanes (group_walk): a small
+// frame takes as long as its slowest rays' chains, which a group shortens, a large one pays a group's
+// greater cost per ray. us per frame of 2 bounces (all old : camera rays by 16 lanes : bounces by 16):
+//   triangles   4,096 samples      32,768            65,536             131,072            256,000
+//   1.5 k       136 : 130 : 61     160 : 160 : 80    170 : 187 : 106    223 : 267 : 179    289 : 376 : 318
+//   19 k        203 : 171 : 113    262 : 247 : 121   254 : 260 : 156    307 : 369 : 235    374 : 508 : 414
+//   150 k       466 : 320 : 264    573 : 442 : 298   533 : 479 : 312    570 : 627 : 390    652 : 782 : 644
+//   753 k       1137 : 741 : 741   1320 : 921 : 747  1335 : 1050 : 738  1276 : 1250 : 754  1397 : 1469 : 1245
+// Whole waves per ray gain a little more on the fewest samples (753 k, 12,288: bounces 708 against 757).
+int path_group(uint64_t n, uint32_t n_tris) {
+    return n <= std::max(4096u, std::min(n_tris / 16u, 16384u)) ? 64 : 16;
+}
+uint64_t primary_group_most(uint32_t n_tris) { return n_tris >= 100000u ? 65536 : 32768; }
+uint64_t bounce_group_most(uint32_t n_tris) { return n_tris >= 250000u ? 262144 : 131072; }
+
 }  // namespace
 }  // namespace rt
 
@@ -432,7 +513,15 @@ extern "C" int rt_trace_paths(const rt_scene* scene, const rt_camera* cam, const
     using K = decltype(&k_paths_primary<0>);
     static const K prim[4] = {k_paths_primary<0>, k_paths_primary<1>, k_paths_primary<2>,
                               k_paths_primary<3>};
-    if (tu.primary == RT_TRAVERSAL_QUAD) {
+    const int g = path_group(n, scene->n_tris);
+    const int gp = tu.primary == RT_TRAVERSAL_QUAD && n <= primary_group_most(scene->n_tris) ? g : 0;
+    const int gb = tu.lane_stack == RT_LANE_STACK_MAX && n <= bounce_group_most(scene->n_tris) ? g : 0;
+    if (gp) {
+        const uint32_t tx8 = (p->width + 7) / 8, ty8 = (p->height + 7) / 8;
+        const uint64_t items = 64ull * tx8 * ty8 * p->spp;
+        hipLaunchKernelGGL(gp == 64 ? k_paths_primary_group<64> : k_paths_primary_group<16>,
+                           dim3((uint32_t)((items * gp + 1023) / 1024)), dim3(1024), 0, s, sc, *cam, a, tx8);
+    } else if (tu.primary == RT_TRAVERSAL_QUAD) {
         const uint32_t tx8 = (p->width + 7) / 8, ty8 = (p->height + 7) / 8;
         hipLaunchKernelGGL(k_paths_primary<RT_TRAVERSAL_QUAD>, dim3(32u * ((tx8 * ty8 + 7u) / 8u)),
                            dim3(64u * std::min(p->spp, 4u)), 0, s, sc, *cam, a, tx8, (int)tu.lane_stack, (int)tu.packet_budget, coherent);
@@ -444,7 +533,12 @@ extern "C" int rt_trace_paths(const rt_scene* scene, const rt_camera* cam, const
     // emit 1 M bounces in 86 us, 16 per CU in 200
     const uint32_t grid = (uint32_t)device_cu_count() * 16u;
     for (uint32_t k = 1; k <= p->bounces; ++k) {
-        hipLaunchKernelGGL(k_paths_bounce, dim3(grid), dim3(64), 0, s, sc, a, k, (int)tu.lane_stack);
+        if (gb) {
+            hipLaunchKernelGGL(gb == 64 ? k_paths_bounce_group<64> : k_paths_bounce_group<16>,
+                               dim3((uint32_t)std::min<uint64_t>((n * gb + 63) / 64, 2ull * grid)), dim3(64), 0, s, sc, a, k);
+        } else {
+            hipLaunchKernelGGL(k_paths_bounce, dim3(grid), dim3(64), 0, s, sc, a, k, (int)tu.lane_stack);
+        }
         hipLaunchKernelGGL(k_paths_emit, dim3(grid / 4u), dim3(256), 0, s, sc, a, k);
     }
     const uint64_t px = (uint64_t)p->width * p->height;
