@@ -362,7 +362,7 @@ RT_DEV void group_walk(const float4* __restrict__ nodes4, const float4* __restri
     h.slot = __shfl(h.slot, wl);
 }
 
-template <bool ANY, int MODE, int PARK, bool NF = false, bool COOP = true, typename Load, typename Finish>
+template <bool ANY, int MODE, int PARK, bool NF = false, bool COOP = true, bool MASK = true, typename Load, typename Finish>
 RT_DEV void refill_walks(const SceneArgs& sc, uint64_t n, uint32_t n_waves, uint32_t wid, int32_t* stk,
                          int stk_stride, int lane_stack, uint32_t* list, float4* pk, Load&& load,
                          Finish&& finish) {
@@ -415,7 +415,7 @@ RT_DEV void refill_walks(const SceneArgs& sc, uint64_t n, uint32_t n_waves, uint
                 else if (MODE == RT_TRAVERSAL_BINARY)
                     st = bin_steps<ANY, true>(sc.nodes, sc.tris, r, skip, h, w, stk, stk_stride, lane_stack, kRefillSteps);
                 else
-                    st = lane4_steps<ANY, PARK, NF, true>(sc.nodes4, sc.tris, r, skip, h, w, stk, stk_stride, lane_stack,
+                    st = lane4_steps<ANY, PARK, NF, MASK>(sc.nodes4, sc.tris, r, skip, h, w, stk, stk_stride, lane_stack,
                                           kRefillSteps);
             }
             finish(st == kWalkDone, ri, r, h);
