@@ -559,9 +559,9 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ slots
 // What bounds it: LDS round trips per level of a walk (10 to 17 levels), and 64 B per node of stores
 // in pieces of 16 B; 37 KB of LDS and one slot per thread put two
 // workgroups on a CU.
-// At 1.31 M triangles 67 us for the local pass and 25 for the top; separate kernels for the hierarchy
+// At 1.31 M triangles 56 us for the local pass and 25 for the top; separate kernels for the hierarchy
 // (binary searches in memory, 93 us), a refit over its arrays (142), a sparse table of block unions
-// (17) and the top refit (10) took 262. At 11,560 triangles 25 us against 61.
+// (17) and the top refit (10) took 262. At 11,560 triangles 24 us against 61.
 // length of the common prefix of the extended keys (a, i) and (b, j)
 RT_DEV int key_prefix(uint32_t a, uint32_t b, int64_t i, int64_t j) {
     return a != b ? __clz(a ^ b) : 32 + __clz((uint32_t)i ^ (uint32_t)j);
