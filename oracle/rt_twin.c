@@ -534,6 +534,11 @@ static inline float safe_inv(float d) {
 /* 1 + 2*gamma(3), gamma(n) = n*eps/(1-n*eps), eps = 2^-24, rounded up (Ize 2013). */
 #define TW_TFAR_SCALE 1.0000004f
 
+/* A closest-hit walk whose best hit is t skips the boxes entered past this: 2^-18 beyond t, more than the
+ * rounding of an entry distance, which the boxes' padding covers only where coordinates are not much
+ * smaller than t. */
+static inline float cull_past(float t) { return fmaf(fabsf(t), 0x1p-18f, t); }
+
 /* Two-sided Moller-Trumbore; the barycentric tests compare the numerators with the determinant
  * after multiplying both by sign(det) (exact), the division happens only for a hit. */
 static inline int mt32(const float* tr, const ray32* r, float* t, float* u, float* v) {
@@ -593,8 +598,9 @@ static void traverse32(const float* nodes, const float* tris, int32_t root, cons
             float tf0 = fminf(fminf(fmaxf(a0, a1), fmaxf(a2, a3)), fmaxf(a4, a5)) * TW_TFAR_SCALE;
             float tn1 = fmaxf(fmaxf(fminf(b0, b1), fminf(b2, b3)), fmaxf(fminf(b4, b5), r->tmin));
             float tf1 = fminf(fminf(fmaxf(b0, b1), fmaxf(b2, b3)), fmaxf(b4, b5)) * TW_TFAR_SCALE;
-            int hit0 = tn0 <= fminf(tf0, h->t);
-            int hit1 = tn1 <= fminf(tf1, h->t);
+            float cull = any ? h->t : cull_past(h->t);
+            int hit0 = tn0 <= fminf(tf0, cull);
+            int hit1 = tn1 <= fminf(tf1, cull);
             int32_t r0 = (int32_t)fbits(nd[12]), r1 = (int32_t)fbits(nd[13]);
             if (hit0 && hit1) {
                 int32_t nearc = r0, farc = r1;
@@ -861,13 +867,14 @@ static void packet32(const float* nodes4, const float* tris, int32_t root, const
         for (int l = 0; l < 64; ++l) {
             if (!((m >> l) & 1)) continue;
             h[l].node_visits++;
+            float cull = any ? h[l].t : cull_past(h[l].t);
             for (int k = 0; k < 4; ++k) {
                 float x0 = fmaf(nd[k], idx[l], -oxx[l]), x1 = fmaf(nd[4 + k], idx[l], -oxx[l]);
                 float y0 = fmaf(nd[8 + k], idy[l], -oyy[l]), y1 = fmaf(nd[12 + k], idy[l], -oyy[l]);
                 float z0 = fmaf(nd[16 + k], idz[l], -ozz[l]), z1 = fmaf(nd[20 + k], idz[l], -ozz[l]);
                 float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), r[l].tmin));
                 float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fmaxf(z0, z1)) * TW_TFAR_SCALE;
-                int hk = ref[k] != 0x7FFFFFFF && tn <= fminf(tf, h[l].t);
+                int hk = ref[k] != 0x7FFFFFFF && tn <= fminf(tf, cull);
                 if (hk) mk[k] |= 1ull << l;
                 if (l == rep) key[k] = hk ? tn : INFINITY;
             }

@@ -14,6 +14,7 @@
 //   ray toward the light per lit hit (wave-coherent any-hit over the tile's hit points, skipping
 //   each hit's own triangle), RGBA8 texture fetch, RGB float32 store.
 #include <algorithm>
+#include <cfloat>
 #include <mutex>
 
 #include "rt_trace_shared.h"
@@ -53,7 +54,8 @@ RT_DEV Ray load_ray(const rt_rays& rays, uint64_t i) {
     r.dy = ld_f(rays.dy, i, rays.stride);
     r.dz = ld_f(rays.dz, i, rays.stride);
     r.tmin = rays.tmin ? ld_f(rays.tmin, i, rays.stride) : rays.tmin_default;
-    r.tmax = rays.tmax ? ld_f(rays.tmax, i, rays.stride) : rays.tmax_default;
+    // (-FLT_MAX for -inf, which would make cull_past's bound NaN: neither leaves room for a hit)
+    r.tmax = fmaxf(rays.tmax ? ld_f(rays.tmax, i, rays.stride) : rays.tmax_default, -FLT_MAX);
     return r;
 }
 

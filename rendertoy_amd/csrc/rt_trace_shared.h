@@ -210,7 +210,7 @@ RT_DEV bool wave_walk(const float4* __restrict__ nodes4, const float4* __restric
             const float z0 = fmaf(clz, idz, -ozz), z1 = fmaf(chz, idz, -ozz);
             const float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), r.tmin));
             const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fmaxf(z0, z1)) * kTfarScale;
-            const bool hk = (cref != RT_EMPTY_ROOT) & (tn <= fminf(tf, h.t));
+            const bool hk = (cref != RT_EMPTY_ROOT) & (tn <= fminf(tf, ANY ? h.t : cull_past(h.t)));
             push = hk & (cref >= 0);
             leaf = hk & (cref < 0);
         }
@@ -235,11 +235,9 @@ RT_DEV bool wave_walk(const float4* __restrict__ nodes4, const float4* __restric
 // ray's best t, the entered internal children are pushed (ballot compaction within the group; for
 // closest hits an entry's nearer children above its farther ones, which halves the time) and each
 // entered leaf is tested by its lane; the group's closest candidate (t, then the smaller primitive)
-// is reduced after a step that found one. The closest hit does not depend on the visiting order, so
-// h is the one-lane walk's hit: a box is skipped only where it is entered 2^-18 past the best hit,
-// more than the rounding of an entry distance, which the boxes' padding covers only where the
-// coordinates are not much smaller than the distance. The stack never overflows: above kSwitch entries a step takes one
-// entry, so the walk goes on depth first, whose at most 31 levels push at most 3 each.
+// is reduced after a step that found one. The closest hit does not depend on the visiting order
+// (cull_past), so h is the one-lane walk's hit. The stack never overflows: above kSwitch entries a step takes
+// one entry, so the walk goes on depth first, whose at most 31 levels push at most 3 each.
 // What bounds a walk of few rays is the chain of dependent steps of its slowest ray (up to 600
 // nodes of one lane): a step costs about the same with 1 entry as with 16, so a group shortens the
 // chain to the depth of the tree plus the nodes / entries left over.
@@ -281,7 +279,7 @@ RT_DEV void group_walk(const float4* __restrict__ nodes4, const float4* __restri
     if (root == RT_EMPTY_ROOT) return;
     float bt = r.tmax;  // the group's best; h is this lane's own until the end
     int32_t bp = -1;
-    float cull = r.tmax;  // boxes entered past this are skipped
+    float cull = ANY ? r.tmax : cull_past(r.tmax);  // boxes entered past this are skipped
     if (root < 0) {  // the whole tree is one leaf
         test_leaf(tris, root, r, want && gl == 0, skip_slot, h);
     } else {
@@ -344,7 +342,7 @@ RT_DEV void group_walk(const float4* __restrict__ nodes4, const float4* __restri
                     bp = h.prim;
                     group_closest<G>(bt, bp);
                     if (ANY && bp >= 0) sp = 0;
-                    if (bp >= 0) cull = fmaf(fabsf(bt), 0x1p-18f, bt);
+                    if (!ANY && bp >= 0) cull = cull_past(bt);
                 }
             }
         }
