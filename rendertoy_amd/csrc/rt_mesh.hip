@@ -11,22 +11,27 @@
 // as the scene build does.
 //
 // Pipeline (one stream): a counting placement of the pairs by vertex, whose runs are in arrival
-// order, each put in order where it is summed. (Before, a stable radix sort of the pairs by vertex
-// fixed the order: 133 of 219 us at 1.31 M triangles, 0.66 M vertices; now 82 us: face 34,
+// order, each put in order where it is summed or before. (A stable radix sort of the pairs by vertex
+// fixed the order before: 133 of 219 us at 1.31 M triangles, 0.66 M vertices; now 83 us: face 34,
 // scan 11, place 15, vertex 16.)
 //   1. k_nrm_face   per triangle: FP64 face normal (32 B record); per pair its arrival number among
 //                   its vertex's pairs (an integer atomic on the vertex's count).
 //   2. k_nrm_sums, k_nrm_offsets   exclusive scan of the counts: each vertex's run in `run`; vertices
-//                   of more than kSmallRun pairs are listed.
+//                   of more than kNetRun pairs are listed.
 //   3. k_nrm_place  run[offset of its vertex + arrival] = p for every pair.
-//   4. k_nrm_big    sorts the listed runs (none in most meshes).
+//   4. k_nrm_order  puts the listed runs in order (none in a mesh of 5 or 6 triangles a vertex).
 //   5. k_nrm_vertex per vertex: its run in ascending p (up to 8 pairs by a sorting network in
 //                   registers), the FP64 sum, float3 N at out + v * out_stride.
+// Triangles gathered on few vertices, us for 600,000 of random vertices of 6 : 12 : 48 : 80 : 200 : 1,000
+// triangles each, and 300 hubs of 4,500: 194 : 210 : 205 : 222 : 325 : 826, 1,380. With the radix sort
+// 208 : 205 : 181 : 215 : 338 : 1,158, 2,047. The pairs of one vertex are same-address atomics in k_nrm_face
+// (about 14 ns each) and one lane's sum in k_nrm_vertex (140 ns each, the larger part of a hub's time).
 // A non-indexed mesh (vertices 3t, 3t+1, 3t+2) has one pair per vertex: k_nrm_direct computes it
 // with no sort and no workspace.
 //
 // Also here: MeshVertex records <-> dense float arrays (k_mesh_pack / k_mesh_unpack), the device-side
 // ingest and export of the 80-byte vertex layout of rendering/_modeling.py:22-28.
+#include <algorithm>
 #include <cmath>
 
 #include "rt_common.h"
@@ -34,18 +39,20 @@
 namespace rt {
 namespace {
 
-constexpr uint32_t kSmallRun = 64;     // longest run k_nrm_vertex puts in order by itself
-constexpr uint32_t kLdsRun = 4096;     // longest run k_nrm_big sorts in LDS
+constexpr uint32_t kNetRun = 8;        // longest run k_nrm_vertex puts in order in registers
+constexpr uint32_t kWaveRun = 256;     // longest run a wave of k_nrm_order ranks
+constexpr uint32_t kLdsRun = 4096;     // longest run, or piece of one, k_nrm_order sorts in LDS
 constexpr uint32_t kScanChunk = 2048;  // counts per workgroup of the scan
 
 struct NrmWorkspace {
     double4* face;    // n_tris
-    uint32_t* rank;   // 3 n_tris: arrival number of pair p
+    uint32_t* rank;   // 3 n_tris: arrival number of pair p, then k_nrm_order's merges
     uint32_t* run;    // 3 n_tris: the pairs by vertex
-    uint32_t* count;  // n_vertices, then the number of listed vertices
+    uint32_t* count;  // n_vertices, then the numbers of listed vertices (mid, big)
     uint32_t* off;    // n_vertices
     uint32_t* sums;   // per scan chunk
-    uint32_t* big;    // listed vertices
+    uint32_t* mid;    // vertices of kNetRun + 1 .. kWaveRun pairs
+    uint32_t* big;    // vertices of more
     uint64_t bytes;
 };
 
@@ -63,10 +70,11 @@ NrmWorkspace carve_nrm(char* base, uint64_t n_vertices, uint64_t n_tris) {
     w.face = (double4*)take(32 * n_tris);
     w.rank = (uint32_t*)take(4 * np);
     w.run = (uint32_t*)take(4 * np);
-    w.count = (uint32_t*)take(4 * (n_vertices + 1));
+    w.count = (uint32_t*)take(4 * (n_vertices + 2));
     w.off = (uint32_t*)take(4 * n_vertices);
     w.sums = (uint32_t*)take(4 * ((n_vertices + kScanChunk - 1) / kScanChunk));
-    w.big = (uint32_t*)take(4 * (np / kSmallRun + 1));
+    w.mid = (uint32_t*)take(4 * (np / (kNetRun + 1) + 1));
+    w.big = (uint32_t*)take(4 * (np / (kWaveRun + 1) + 1));
     w.bytes = off;
     return w;
 }
@@ -167,13 +175,15 @@ __global__ void __launch_bounds__(1024) k_nrm_scan_sums(uint32_t* __restrict__ s
 }
 
 // off[i] = the counts before i (the chunks before from their sums, or, `scanned`, from their scan);
-// vertices of long runs are listed
+// vertices of runs that k_nrm_order puts in order are listed, listed[0] of them in `mid` and listed[1] in
+// `big`, with one atomic per workgroup and list: one per vertex took 0.3 ms for 20,000 of them.
 __global__ void __launch_bounds__(256) k_nrm_offsets(const uint32_t* __restrict__ count, uint32_t n,
                                                       const uint32_t* __restrict__ sums, bool scanned,
-                                                      uint32_t* __restrict__ off, uint32_t* __restrict__ n_big,
-                                                      uint32_t* __restrict__ big) {
+                                                      uint32_t* __restrict__ off, uint32_t* __restrict__ listed,
+                                                      uint32_t* __restrict__ mid, uint32_t* __restrict__ big) {
     constexpr uint32_t kPer = kScanChunk / 256;
-    __shared__ uint32_t lds[4], scan[256];
+    __shared__ uint32_t lds[4], scan[256], s_count[2], s_base[2];
+    if (threadIdx.x < 2) s_count[threadIdx.x] = 0;
     uint32_t before = 0;
     if (scanned) {
         before = sums[blockIdx.x];
@@ -182,11 +192,13 @@ __global__ void __launch_bounds__(256) k_nrm_offsets(const uint32_t* __restrict_
         before = block_sum(before, lds);
     }
     const uint64_t base = (uint64_t)blockIdx.x * kScanChunk + threadIdx.x * kPer;
-    uint32_t c[kPer], sum = 0;
+    uint32_t c[kPer], sum = 0, n_mid = 0, n_big = 0;
 #pragma unroll
     for (uint32_t k = 0; k < kPer; ++k) {
         c[k] = base + k < n ? count[base + k] : 0u;
         sum += c[k];
+        n_mid += c[k] > kNetRun && c[k] <= kWaveRun;
+        n_big += c[k] > kWaveRun;
     }
     scan[threadIdx.x] = sum;
     __syncthreads();
@@ -197,11 +209,19 @@ __global__ void __launch_bounds__(256) k_nrm_offsets(const uint32_t* __restrict_
         __syncthreads();
     }
     uint32_t at = before + scan[threadIdx.x] - sum;
+    uint32_t at_mid = n_mid ? atomicAdd(&s_count[0], n_mid) : 0u, at_big = n_big ? atomicAdd(&s_count[1], n_big) : 0u;
+    __syncthreads();
+    if (threadIdx.x < 2 && s_count[threadIdx.x])
+        s_base[threadIdx.x] = atomicAdd(&listed[threadIdx.x], s_count[threadIdx.x]);
+    __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < kPer; ++k) {
         if (base + k < n) {
             off[base + k] = at;
-            if (c[k] > kSmallRun) big[atomicAdd(n_big, 1u)] = (uint32_t)(base + k);
+            if (c[k] > kWaveRun)
+                big[s_base[1] + at_big++] = (uint32_t)(base + k);
+            else if (c[k] > kNetRun)
+                mid[s_base[0] + at_mid++] = (uint32_t)(base + k);
         }
         at += c[k];
     }
@@ -220,61 +240,126 @@ __global__ void __launch_bounds__(256) k_nrm_place(rt_mesh_desc m, const uint32_
     }
 }
 
-// Sorts the runs of the listed vertices, one workgroup each: a bitonic sort in LDS, or, past its size,
-// the vertex's pairs collected again in order from the index list.
-__global__ void __launch_bounds__(1024) k_nrm_big(rt_mesh_desc m, const uint32_t* __restrict__ n_big,
-                                                   const uint32_t* __restrict__ big,
-                                                   const uint32_t* __restrict__ count,
-                                                   const uint32_t* __restrict__ off, uint32_t* __restrict__ run) {
-    __shared__ uint32_t key[kLdsRun];
-    __shared__ uint32_t waves[16];
-    const uint32_t n = *n_big, tid = threadIdx.x;
-    for (uint32_t b = blockIdx.x; b < n; b += gridDim.x) {
-        const uint32_t v = big[b], len = count[v];
-        uint32_t* out = run + off[v];
-        __syncthreads();  // before the last vertex's LDS is written again
-        if (len <= kLdsRun) {
-            uint32_t pow2 = 1;
-            while (pow2 < len) pow2 <<= 1;
-            for (uint32_t i = tid; i < pow2; i += 1024u) key[i] = i < len ? out[i] : 0xFFFFFFFFu;
-            for (uint32_t k = 2; k <= pow2; k <<= 1) {
-                for (uint32_t d = k >> 1; d > 0; d >>= 1) {
-                    __syncthreads();
-                    for (uint32_t i = tid; i < pow2; i += 1024u) {
-                        const uint32_t x = i ^ d;
-                        if (x <= i) continue;
-                        const uint32_t lo = key[i], hi = key[x];
-                        if ((lo > hi) == ((i & k) == 0)) {
-                            key[i] = hi;
-                            key[x] = lo;
-                        }
+// One pass of a merge sort by a workgroup of 256: src[0, n), sorted in pieces of w (a multiple of 16), to dst
+// in pieces of 2 w. A thread finds where its 16 outputs begin in their two pieces and merges them.
+RT_DEV void merge_pieces(const uint32_t* src, uint32_t* dst, uint64_t n, uint64_t w) {
+    for (uint64_t o = 16ull * threadIdx.x; o < n; o += 16ull * 256) {
+        const uint64_t a0 = o / (2 * w) * (2 * w), a1 = a0 + w < n ? a0 + w : n, b1 = a1 + w < n ? a1 + w : n;
+        const uint64_t d = o - a0;  // outputs of the two pieces before these
+        uint64_t lo = d > b1 - a1 ? d - (b1 - a1) : 0, hi = d < a1 - a0 ? d : a1 - a0;
+        while (lo < hi) {
+            const uint64_t m = (lo + hi) / 2;
+            if (src[a0 + m] < src[a1 + d - 1 - m])
+                lo = m + 1;
+            else
+                hi = m;
+        }
+        uint64_t i = a0 + lo, j = a1 + (d - lo);
+        for (int k = 0; k < 16 && o + k < n; ++k) {
+            const bool left = j >= b1 || (i < a1 && src[i] < src[j]);
+            dst[o + k] = left ? src[i] : src[j];
+            i += left;
+            j += !left;
+        }
+    }
+}
+
+// Sorts run[0, n) by a workgroup of 256: pieces of kLdsRun by a bitonic sort in LDS, then merges, through
+// tmp[0, n). The work grows with the run's own length; called with the same arguments by all threads.
+RT_DEV void sort_run(uint32_t* run, uint32_t* tmp, uint32_t n, uint32_t* key) {
+    const uint32_t tid = threadIdx.x;
+    for (uint64_t base = 0; base < n; base += kLdsRun) {
+        const uint32_t len = (uint32_t)(n - base < kLdsRun ? n - base : kLdsRun);
+        uint32_t pow2 = 2;
+        while (pow2 < len) pow2 <<= 1;
+        __syncthreads();  // before the last piece's LDS is written again
+        for (uint32_t i = tid; i < pow2; i += 256u) key[i] = i < len ? run[base + i] : 0xFFFFFFFFu;
+        for (uint32_t k = 2; k <= pow2; k <<= 1) {
+            for (uint32_t d = k >> 1; d > 0; d >>= 1) {
+                __syncthreads();
+                for (uint32_t q = tid; q < pow2 / 2; q += 256u) {
+                    const uint32_t i = ((q & ~(d - 1)) << 1) | (q & (d - 1)), x = i + d;
+                    const uint32_t lo = key[i], hi = key[x];
+                    if ((lo > hi) == ((i & k) == 0)) {
+                        key[i] = hi;
+                        key[x] = lo;
                     }
                 }
             }
-            __syncthreads();
-            for (uint32_t i = tid; i < len; i += 1024u) out[i] = key[i];
-            continue;
         }
-        uint32_t done = 0;  // the same in every thread
-        for (uint32_t k = 0; k < 3; ++k) {
-            for (uint32_t t0 = 0; t0 < m.n_tris; t0 += 1024u) {
-                const uint32_t t = t0 + tid;
-                const bool mine = t < m.n_tris && clamp_index(m.indices[3 * (uint64_t)t + k], m.n_vertices) == v;
-                const uint64_t mask = __ballot(mine);
-                if ((tid & 63u) == 0) waves[tid >> 6] = (uint32_t)__popcll(mask);
-                __syncthreads();
-                uint32_t at = done, all = 0;
-                for (uint32_t w = 0; w < 16u; ++w) {
-                    at += w < (tid >> 6) ? waves[w] : 0u;
-                    all += waves[w];
-                }
-                at += __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-                if (mine) out[at] = k * m.n_tris + t;
-                done += all;
-                __syncthreads();
-            }
+        __syncthreads();
+        for (uint32_t i = tid; i < len; i += 256u) run[base + i] = key[i];
+    }
+    uint32_t *src = run, *dst = tmp;
+    for (uint64_t w = kLdsRun; w < n; w *= 2) {
+        __syncthreads();
+        merge_pieces(src, dst, n, w);
+        uint32_t* t = src;
+        src = dst;
+        dst = t;
+    }
+    if (src != run) {
+        __syncthreads();
+        for (uint64_t i = tid; i < n; i += 256u) run[i] = src[i];
+    }
+}
+
+// Puts run[0, n) in order by one wave, K pairs in each lane (n <= 64 K): a pair's place is the number of
+// smaller ones.
+template <int K>
+RT_DEV void rank_run(uint32_t* run, uint32_t n, uint32_t lane) {
+    uint32_t p[K], rank[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        p[k] = 64u * k + lane < n ? run[64 * k + lane] : 0xFFFFFFFFu;
+        rank[k] = 0;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const uint32_t here = n > 64u * k ? (n - 64u * k < 64u ? n - 64u * k : 64u) : 0u;
+        for (uint32_t j = 0; j < here; ++j) {
+            const uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)p[k], (int)j);
+#pragma unroll
+            for (int i = 0; i < K; ++i) rank[i] += q < p[i];
         }
     }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if (64u * k + lane < n) run[rank[k]] = p[k];
+}
+
+// Puts the listed runs in order, a workgroup each for the big ones, a wave each for the others. Bound by the
+// latency of three dependent loads per run; where no run is listed it ends at once. Random vertices of 80
+// triangles, 600,000 in all: 22,500 runs in 26 us by waves, 73 by workgroups. One workgroup per run of more
+// than 64 over 64 workgroups took the mesh 2,473 us in all, the index list read again for each of 300 hubs
+// of 4,500 14,476.
+__global__ void __launch_bounds__(256) k_nrm_order(const uint32_t* __restrict__ listed,
+                                                    const uint32_t* __restrict__ mid,
+                                                    const uint32_t* __restrict__ big,
+                                                    const uint32_t* __restrict__ count,
+                                                    const uint32_t* __restrict__ off, uint32_t* run, uint32_t* tmp) {
+    __shared__ uint32_t key[kLdsRun];
+    const uint32_t n_mid = listed[0], n_big = listed[1], lane = threadIdx.x & 63u;
+    for (uint32_t b = blockIdx.x; b < n_big; b += gridDim.x) {
+        const uint32_t v = big[b];
+        sort_run(run + off[v], tmp + off[v], count[v], key);
+    }
+    for (uint32_t w = blockIdx.x * 4u + (threadIdx.x >> 6); w < n_mid; w += gridDim.x * 4u) {
+        const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int)mid[w]);
+        const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)count[v]);
+        uint32_t* r = run + off[v];
+        if (n <= 64)
+            rank_run<1>(r, n, lane);
+        else if (n <= 128)
+            rank_run<2>(r, n, lane);
+        else
+            rank_run<4>(r, n, lane);
+    }
+}
+
+// Triangle of pair p.
+RT_DEV uint32_t pair_tri(uint32_t p, uint32_t n_tris) {
+    return p >= 2 * n_tris ? p - 2 * n_tris : (p >= n_tris ? p - n_tris : p);
 }
 
 // Bound by the gathers of the face records (32 B a pair, from all over the list): the 8 of a small run
@@ -296,9 +381,8 @@ __global__ void __launch_bounds__(256) k_nrm_vertex(const uint32_t* __restrict__
         return;
     }
     const uint32_t* r = run + off[v];
-    auto tri = [&](uint32_t p) { return p >= 2 * n_tris ? p - 2 * n_tris : (p >= n_tris ? p - n_tris : p); };
     double x = 0.0, y = 0.0, z = 0.0;
-    if (n <= 8) {
+    if (n <= kNetRun) {
         uint32_t p[8];
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) p[j] = j < n ? r[j] : 0xFFFFFFFFu;
@@ -317,7 +401,7 @@ __global__ void __launch_bounds__(256) k_nrm_vertex(const uint32_t* __restrict__
         double4 f[8];
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j)
-            if (j < n) f[j] = face[tri(p[j])];
+            if (j < n) f[j] = face[pair_tri(p[j], n_tris)];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) {
@@ -328,18 +412,9 @@ __global__ void __launch_bounds__(256) k_nrm_vertex(const uint32_t* __restrict__
             }
         }
     } else {
-        uint32_t last = 0;
+#pragma unroll 4
         for (uint32_t j = 0; j < n; ++j) {
-            uint32_t p = r[j];
-            if (n <= kSmallRun) {  // the smallest pair past the last one
-                p = 0xFFFFFFFFu;
-                for (uint32_t i = 0; i < n; ++i) {
-                    const uint32_t q = r[i];
-                    p = (j == 0 || q > last) && q < p ? q : p;
-                }
-                last = p;
-            }
-            const double4 f = face[tri(p)];
+            const double4 f = face[pair_tri(r[j], n_tris)];
             x = x + f.x;
             y = y + f.y;
             z = z + f.z;
@@ -472,20 +547,22 @@ extern "C" int rt_mesh_compute_normals(const rt_mesh_desc* mesh, float* normals_
         return set_error(RT_EINVAL, "rt_mesh_compute_normals: workspace must be 256-byte aligned");
     NrmWorkspace w = carve_nrm((char*)workspace, m.n_vertices, m.n_tris);
     const uint32_t chunks = nblocks(m.n_vertices, kScanChunk);
-    uint32_t* n_big = w.count + m.n_vertices;
-    hipLaunchKernelGGL(k_nrm_clear, dim3(nblocks((uint64_t)m.n_vertices + 1, 256)), dim3(256), 0, s, w.count,
-                       (uint64_t)m.n_vertices + 1);
+    uint32_t* listed = w.count + m.n_vertices;
+    hipLaunchKernelGGL(k_nrm_clear, dim3(nblocks((uint64_t)m.n_vertices + 2, 256)), dim3(256), 0, s, w.count,
+                       (uint64_t)m.n_vertices + 2);
     if (m.n_tris)
         hipLaunchKernelGGL(k_nrm_face, dim3(nblocks(m.n_tris, 256)), dim3(256), 0, s, m, w.face, w.count, w.rank);
     hipLaunchKernelGGL(k_nrm_sums, dim3(chunks), dim3(256), 0, s, w.count, m.n_vertices, w.sums);
     const bool scanned = chunks > kSumChunks;
     if (scanned) hipLaunchKernelGGL(k_nrm_scan_sums, dim3(1), dim3(1024), 0, s, w.sums, chunks);
     hipLaunchKernelGGL(k_nrm_offsets, dim3(chunks), dim3(256), 0, s, w.count, m.n_vertices, w.sums, scanned, w.off,
-                       n_big, w.big);
+                       listed, w.mid, w.big);
     if (m.n_tris) {
         hipLaunchKernelGGL(k_nrm_place, dim3(nblocks(m.n_tris, 256)), dim3(256), 0, s, m, w.off, w.rank, w.run);
-        if (3 * (uint64_t)m.n_tris > kSmallRun)
-            hipLaunchKernelGGL(k_nrm_big, dim3(64), dim3(1024), 0, s, m, n_big, w.big, w.count, w.off, w.run);
+        const uint64_t np = 3 * (uint64_t)m.n_tris;
+        if (np > kNetRun)  // a wave for each of the most mid runs, up to 8 workgroups per CU
+            hipLaunchKernelGGL(k_nrm_order, dim3((uint32_t)std::min<uint64_t>(np / (4 * kNetRun) + 1, 2048)), dim3(256), 0,
+                               s, listed, w.mid, w.big, w.count, w.off, w.run, w.rank);
     }
     hipLaunchKernelGGL(k_nrm_vertex, dim3(nblocks(m.n_vertices, 256)), dim3(256), 0, s, w.count, w.off, w.run,
                        m.n_tris, w.face, m.n_vertices, out, out_stride);
