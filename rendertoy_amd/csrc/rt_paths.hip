@@ -454,6 +454,9 @@ __global__ void __launch_bounds__(256) k_paths_resolve(PathArgs a, float* __rest
 //   150 k       466 : 320 : 264    573 : 442 : 298   533 : 479 : 312    570 : 627 : 390    652 : 782 : 644
 //   753 k       1137 : 741 : 741   1320 : 921 : 747  1335 : 1050 : 738  1276 : 1250 : 754  1397 : 1469 : 1245
 // Whole waves per ray gain a little more on the fewest samples (753 k, 12,288: bounces 708 against 757).
+// Over scenes of eight shapes (image_group's), 16 lanes take whole frames to 0.97 of their time on average and
+// 1.13 at worst for camera rays of 32,768 samples, bounces to 0.70 and 1.44 at 131,072 and, from 250,000
+// triangles on, to 0.96 and 1.50 at 256,000 (a room from inside).
 int path_group(uint64_t n, uint32_t n_tris) {
     return n <= std::max(4096u, std::min(n_tris / 16u, 16384u)) ? 64 : 16;
 }

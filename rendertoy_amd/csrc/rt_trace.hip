@@ -15,6 +15,7 @@
 //   each hit's own triangle), RGBA8 texture fetch, RGB float32 store.
 #include <algorithm>
 #include <cfloat>
+#include <cmath>
 #include <mutex>
 
 #include "rt_trace_shared.h"
@@ -281,22 +282,44 @@ uint32_t group_blocks(int g, uint32_t W, uint32_t H) {
     return 8u * ((blocks8 + 7u) / 8u) * (uint32_t)g;
 }
 
+// The lines below were set over scenes of eight shapes (a smooth sphere, a rough one on a plane, one from near, a
+// terrain, a room from inside, boxes, random triangles, long thin ones) of 1,300 to 1.3 M triangles, since how
+// much longer the slowest walk is than the average one depends on the shape as much as on the triangles.
+double fourth_root(uint32_t n) { return std::sqrt(std::sqrt((double)n)); }
+
+// Lanes per ray where groups walk n rays: 64 for few, 16 for more. Whole waves shorten a ray's chain more the
+// deeper its tree, and cost 3 to 4 times as much per ray: camera time of 16 : 64 lanes over quad-lane packets,
+// geometric mean over the shapes, 0.59 : 0.54 at 4,096 pixels with 1,300 triangles, 0.31 : 0.23 at 8,192 with
+// 80,000, 0.35 : 0.39 at 24,576 with 320,000, 0.32 : 0.34 at 36,864 with 1.3 M (176 : 118 us on the rough sphere).
+int group_lanes(uint64_t n, uint32_t n_tris) {
+    return (double)n <= std::max(4096.0, std::min(n_tris / 6.0, 1200.0 * fourth_root(n_tris))) ? 64 : 16;
+}
+
 // Lanes per pixel of an image of n pixels: 64 or 16 (group_walk), or 0 for the quad-lane packets.
 // Packets share their node fetches, but a frame takes at least as long as its slowest packet's chain
 // of steps, the longer the denser the scene and the fewer the pixels; groups shorten the chain and
-// cost more per pixel (us, mean of three views, quads : 16 : 64 lanes, camera / render):
+// cost more per pixel (us, mean of three views of a rough sphere on a plane, quads : 16 : 64 lanes, camera /
+// render):
 //   triangles  64x64                          256x256                       768x512
 //   1.3 k      26/39 : 12/16 : 11/16          20/33 : 26/37 : 74/106        31/54 : 114/163 : 398/575
 //   11.5 k     77/105 : 19/24 : 13/18         42/64 : 32/44 : 76/107        49/80 : 119/167 : 400/559
 //   50 k       197/236 : 32/38 : 18/22        103/129 : 49/60 : 84/119      92/132 : 138/201 : 435/615
 //   251 k      546/627 : 59/70 : 26/32        265/332 : 82/100 : 97/141     221/295 : 175/280 : 472/678
 //   1.3 M      2160/2483 : 168/198 : 64/71    928/1225 : 202/243 : 132/191  720/951 : 340/480 : 556/811
-// The 16-lane groups are faster up to about 900 sqrt(triangles) pixels (1.3 M at 1024x768: 558
-// against 688 us, at 1600x900 831 against 735), whole waves up to 4,096 pixels or, where the tree is
-// deeper, a sixth of the triangles.
+// There 16 lanes are faster up to about 900 sqrt(triangles) pixels. Over the eight shapes (camera time of 16
+// lanes over the packets', best, geometric mean, worst):
+//   triangles   16,384 pixels        65,536               147,456              262,144              786,432
+//   1.3 k       0.50  0.72  0.86     0.98  1.36  1.63     1.04  1.76  2.35     2.00  2.46  2.93
+//   20 k        0.29  0.51  0.85     0.64  1.02  1.70     0.76  1.38  2.19     1.46  2.05  2.92
+//   320 k       0.15  0.31  0.55     0.27  0.69  1.31     0.37  0.95  1.83     0.76  1.54  2.73     1.43  2.25  3.75
+//   1.3 M       0.13  0.26  0.40     0.22  0.51  1.12     0.22  0.73  1.71     0.43  1.22  2.32     0.83  1.83  3.44
+// so a second line, 12,000 fourth roots of the triangles, ends the groups where hardly a shape gains. Below it a
+// frame can still take up to 2.8 times as long as by packets where all its rays' walks are alike (a sphere from
+// near), against up to 9 times as long by packets where few are long (a wide frame of a small object: 1281x143
+// pixels, 155,000 triangles, 93 us against 410).
 int image_group(uint64_t n, uint32_t n_tris) {
-    if (n * n > 810000ull * n_tris) return 0;
-    return n <= std::max(4096u, std::min(n_tris / 6u, 65536u)) ? 64 : 16;
+    if ((double)n > std::min(900.0 * std::sqrt((double)n_tris), 12000.0 * fourth_root(n_tris))) return 0;
+    return group_lanes(n, n_tris);
 }
 
 // Camera closest hit of a small image, G lanes per pixel (image_group).
@@ -1124,13 +1147,13 @@ int query_variant(const rt_tuning& tu, uint32_t n, uint32_t n_tris, bool any) {
 //   50 k        107/83 : 26/17 : 18/9      121/89 : 35/23 : 40/28     123/91 : 84/60 : 128/90     132/106 : 142/107 : 244/172
 //   251 k       194/159 : 48/27 : 23/12    238/194 : 70/53 : 58/43    249/220 : 156/105 : 168/116 262/222 : 254/179 : 314/219
 //   1.3 M       573/355 : 99/53 : 42/21    664/469 : 192/116 : 98/68  639/459 : 347/249 : 264/183 649/463 : 533/444 : 477/348
-// so groups serve up to 65,536 rays, twice that in scenes of 250,000 triangles, and whole waves the
-// fewer rays the smaller (shallower) the scene. A caller that bounds the lane stacks, or asks for
-// the binary nodes, gets the walk that has them.
-int query_group(const rt_tuning& tu, uint32_t n, uint32_t n_tris) {
+// Over the eight shapes, random and coherent rays, 16 lanes take 0.72 of the one-lane walks' time for closest hits
+// of 65,536 rays on average and 1.17 at worst, 1.12 and 1.94 for 131,072 (a near view of a sphere of 320,000
+// triangles); any hits 0.56 and 0.83, 0.83 and 1.36.
+// A caller that bounds the lane stacks, or asks for the binary nodes, gets the walk that has them.
+int query_group(const rt_tuning& tu, uint32_t n, uint32_t n_tris, bool any) {
     if (tu.query != RT_TRAVERSAL_LANE || tu.lane_stack != RT_LANE_STACK_MAX) return 0;
-    if (n > (n_tris >= 250000u ? 131072u : 65536u)) return 0;
-    return n <= std::max(4096u, n_tris / 8u) ? 64 : 16;
+    return n <= (any && n_tris >= 250000u ? 131072u : 65536u) ? group_lanes(n, n_tris) : 0;
 }
 
 template <bool ANY>
@@ -1156,7 +1179,7 @@ extern "C" int rt_trace_closest(const rt_scene* scene, const rt_rays* rays, uint
     rt_tuning tu;
     if ((e = resolve_tuning(tuning, tu, "rt_trace_closest"))) return e;
     if (n == 0) return RT_OK;
-    if (const int g = query_group(tu, n, scene->n_tris)) {
+    if (const int g = query_group(tu, n, scene->n_tris, false)) {
         launch_query_group<false>(g, scene, *rays, n, *hits, nullptr, (hipStream_t)stream);
         return check_launch("rt_trace_closest");
     }
@@ -1179,7 +1202,7 @@ extern "C" int rt_trace_any(const rt_scene* scene, const rt_rays* rays, uint32_t
     rt_tuning tu;
     if ((e = resolve_tuning(tuning, tu, "rt_trace_any"))) return e;
     if (n == 0) return RT_OK;
-    if (const int g = query_group(tu, n, scene->n_tris)) {
+    if (const int g = query_group(tu, n, scene->n_tris, true)) {
         launch_query_group<true>(g, scene, *rays, n, rt_hits{}, occluded, (hipStream_t)stream);
         return check_launch("rt_trace_any");
     }
