@@ -613,8 +613,10 @@ RT_DEV uint32_t job_tiles(const rt_render_job& j, uint32_t unit, uint32_t& statu
 
 // The tile queue of k_render_batch_refill in the workspace bytes past the prefix, where the caller
 // gives them: kQueues counters, each on a 256-byte line of its own, then the order of the jobs.
-// Waves of one queue take every kQueues-th grab of tiles. One counter for all waves is the kernel's
-// bound once most tiles miss everything: it is read and written about 70 times a microsecond at
+// The x-th grab of queue q is grab x kQueues + (q + 8 x) mod kQueues of the launch: without the turn a queue
+// would keep to the same columns of an image whose rows are a multiple of kQueues grabs (8 images of 1024x1024
+// pixels, 1,300 triangles, 1.21 ms instead of 0.95); turned by 8 it stays on its XCD's stripes. One counter for
+// all waves is the kernel's bound once most tiles miss everything: it is read and written about 70 times a microsecond at
 // most, and 48 images of 128..768 pixels a side are 30,000 grabs of 4 tiles.
 constexpr uint32_t kQueues = 64, kQueueStride = 64;  // words
 
@@ -623,11 +625,21 @@ struct BatchQueue {
     uint32_t* order;     // job of the p-th prefix entry
 };
 
-// A grab is the launch's unit of work at its end: a wave can hold one of its densest tiles (256 pixels
-// of 4 tiles take up to 1.5 ms). Smaller grabs cost more job changes, whose drains leave lanes idle:
-// with 1 : 2 : 4 tiles, 122,000 tiles in all take 1.44 : 1.24 : 1.55 ms, 30,000 tiles 0.64 : 0.84 :
-// 1.38 (0.55 : 0.76 : 1.14 over 3 scenes instead of 12).
-constexpr uint32_t kGrabsPerWave = 16;
+RT_DEV uint32_t queue_grab(uint32_t x, uint32_t q) { return x * kQueues + (q + 8u * x) % kQueues; }
+
+// Tiles per grab. A grab is the launch's unit of work at its end: a wave can hold one of its densest tiles (256
+// pixels of 4 tiles take up to 1.5 ms), so a wave should have 16 grabs, or 6 where each is one tile. But a wave
+// finishes all its rays before it changes jobs, and with small jobs each grab is another job: two tiles at
+// least then, and the caller's number for jobs of less than 64 tiles. (Time over the single counter's of 4 tiles
+// per grab, for 1 : 2 : 4 tiles: 48 images of 128 to 768 pixels, 2,540 tiles a job, 0.59 : 0.59 : 0.82 [12 images
+// 0.55 : 0.69 : 0.97]; 64 of 256 pixels of 50,000 random triangles, 1,024 a job, 1.24 : 1.02 : 0.97; 2,000 of 16 to
+// 40 pixels 1.41 : 1.11 : 0.98, on a rough sphere 1.13 : 1.03 : 1.00.)
+RT_DEV uint32_t tiles_per_grab(uint32_t most, uint32_t total, uint32_t n_jobs, uint32_t waves) {
+    const uint32_t least = total <= 6u * waves || total > 1024u * n_jobs ? 1u : total >= 64u * n_jobs ? 2u : most;
+    const uint32_t even = (total + 16u * waves - 1u) / (16u * waves);
+    const uint32_t want = even > least ? even : least;
+    return want < most ? want : most;
+}
 
 inline uint64_t batch_queue_offset(uint32_t n_jobs) { return (4ull * (kBatchPrefixWord + (uint64_t)n_jobs + 1) + 255) & ~255ull; }
 inline uint64_t batch_queue_bytes(uint32_t n_jobs) { return 4ull * (kQueues * kQueueStride + n_jobs); }
@@ -828,10 +840,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
     for (uint32_t j = lane; j <= n_jobs; j += 64) pref[j] = ws[kBatchPrefixWord + j];
     __syncthreads();
     const uint32_t total = pref[n_jobs];
-    if (queue.counters) {  // at least kGrabsPerWave grabs per wave where the caller's grab allows it
-        const uint32_t most = (total + gridDim.x * kGrabsPerWave - 1u) / (gridDim.x * kGrabsPerWave);
-        grab = grab < most ? grab : most;
-    }
+    if (queue.counters) grab = tiles_per_grab(grab, total, n_jobs, gridDim.x);
 
     // wave-uniform: the tile being handed out, its next pixel, the end of the grabbed tiles, and
     // the job the lanes work on (with its scene, camera, parameters and counts)
@@ -890,11 +899,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
                         // is not (the counters only grow, so every wave finds all of them empty)
                         for (;;) {
                             if (lane == 0) u0 = atomicAdd(&queue.counters[q * kQueueStride], 1u);
-                            u0 = ((uint32_t)__builtin_amdgcn_readfirstlane((int)u0) * kQueues + q) * grab;
+                            u0 = queue_grab((uint32_t)__builtin_amdgcn_readfirstlane((int)u0), q) * grab;
                             if (u0 < total) break;
                             const uint32_t at = __hip_atomic_load(&queue.counters[lane * kQueueStride],
                                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            const uint64_t open = __ballot((at * kQueues + lane) * grab < total);
+                            const uint64_t open = __ballot(queue_grab(at, lane) * grab < total);
                             if (open == 0) break;
                             const uint64_t after = open & ~((2ull << q) - 1ull);
                             q = (uint32_t)__ffsll((unsigned long long)(after ? after : open)) - 1u;
