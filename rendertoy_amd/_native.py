@@ -224,6 +224,7 @@ SIGNATURES = [
      [ctypes.POINTER(rt_scene), ctypes.POINTER(rt_camera), ctypes.POINTER(rt_render_params),
       ctypes.POINTER(rt_render_out), ctypes.c_void_p, ctypes.c_uint64, ctypes.POINTER(rt_tuning), ctypes.c_void_p]),
     ("rt_render_batch_workspace_bytes", ctypes.c_uint64, [ctypes.c_uint32]),
+    ("rt_render_batch_queue_bytes", ctypes.c_uint64, [ctypes.c_uint32]),
     ("rt_render_batch", ctypes.c_int,
      [ctypes.c_void_p, ctypes.c_uint32, ctypes.POINTER(rt_batch_config), ctypes.c_void_p,
       ctypes.c_uint64, ctypes.c_void_p]),

@@ -47,10 +47,6 @@ _ALG = {"packet": N.RT_TRAVERSAL_PACKET, "lane": N.RT_TRAVERSAL_LANE, "hybrid": 
         "auto": N.RT_TRAVERSAL_AUTO, "quad": N.RT_TRAVERSAL_QUAD}
 
 
-# room in the workspace for the tile queues and the order of the jobs (rt_render_batch_workspace_bytes)
-_QUEUE_BYTES = 16640 + 4 * N.RT_BATCH_MAX_JOBS
-
-
 @dataclasses.dataclass
 class BatchConfig:
     """Launch shape of rt_render_batch (rt_batch_config)."""
@@ -122,7 +118,7 @@ class BatchRender:
             # queued on the stream, and a serving loop enqueues the next batch behind a running one
             self._jobs_host = torch.frombuffer(bytearray(bytes(jobs)), dtype=torch.uint8).pin_memory()
             self.jobs_dev = self._jobs_host.to(dev, non_blocking=True)
-            wsb = lib.rt_render_batch_workspace_bytes(n) + _QUEUE_BYTES
+            wsb = lib.rt_render_batch_queue_bytes(n)
             self.workspace = torch.zeros(wsb, dtype=torch.uint8, device=dev)
         self._graph = None
 
@@ -181,7 +177,7 @@ class BatchSlot:
         self.host = torch.empty(nbytes, dtype=torch.uint8).pin_memory()
         with torch.cuda.stream(self.stream):
             self.dev = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
-            self.workspace = torch.empty(lib.rt_render_batch_workspace_bytes(self.max_jobs) + _QUEUE_BYTES,
+            self.workspace = torch.empty(lib.rt_render_batch_queue_bytes(self.max_jobs),
                                          dtype=torch.uint8, device="cuda")
         self._copied = None
         self._keep = []

@@ -615,7 +615,7 @@ RT_DEV uint32_t job_tiles(const rt_render_job& j, uint32_t unit, uint32_t& statu
 // gives them: kQueues counters, each on a 256-byte line of its own, then the order of the jobs.
 // The x-th grab of queue q is grab x kQueues + (q + 8 x) mod kQueues of the launch: without the turn a queue
 // would keep to the same columns of an image whose rows are a multiple of kQueues grabs (8 images of 1024x1024
-// pixels, 1,300 triangles, 1.21 ms instead of 0.95); turned by 8 it stays on its XCD's stripes. One counter for
+// pixels, 1,300 triangles, 1.14 ms instead of 0.92); turned by 8 it stays on its XCD's stripes. One counter for
 // all waves is the kernel's bound once most tiles miss everything: it is read and written about 70 times a microsecond at
 // most, and 48 images of 128..768 pixels a side are 30,000 grabs of 4 tiles.
 constexpr uint32_t kQueues = 64, kQueueStride = 64;  // words
@@ -1341,6 +1341,10 @@ extern "C" uint64_t rt_render_batch_workspace_bytes(uint32_t n_jobs) {
     return 4ull * (kBatchPrefixWord + (uint64_t)n_jobs + 1);
 }
 
+extern "C" uint64_t rt_render_batch_queue_bytes(uint32_t n_jobs) {
+    return batch_queue_offset(n_jobs) + batch_queue_bytes(n_jobs);
+}
+
 extern "C" const uint32_t* rt_render_batch_status(const void* workspace_dev) {
     return workspace_dev ? (const uint32_t*)workspace_dev + 1 : nullptr;
 }
@@ -1365,14 +1369,14 @@ int check_batch_args(const rt_render_job* jobs_dev, uint32_t n_jobs, const rt_ba
 }
 
 // The two launches of a batch (prepare + persistent kernel) on `ws`, a workspace of
-// rt_render_batch_workspace_bytes(n_jobs) bytes whose every word the prepare kernel rewrites.
+// at least rt_render_batch_workspace_bytes(n_jobs) bytes whose every word in use the prepare kernel rewrites.
 int launch_batch(const rt_render_job* jobs_dev, uint32_t n_jobs, const rt_batch_config* cfg,
                  uint32_t* ws, uint64_t ws_bytes, hipStream_t s, const char* what) {
     const bool quad = cfg->primary == RT_TRAVERSAL_QUAD;
     const bool refill = cfg->primary == RT_TRAVERSAL_LANE && cfg->shadow == RT_TRAVERSAL_LANE;
     BatchQueue queue{nullptr, nullptr};
     const uint64_t at = batch_queue_offset(n_jobs);
-    if (refill && ws_bytes >= at + batch_queue_bytes(n_jobs)) {
+    if (refill && ws_bytes >= rt_render_batch_queue_bytes(n_jobs)) {
         queue.counters = ws + at / 4;
         queue.order = queue.counters + kQueues * kQueueStride;
     }

@@ -54,3 +54,23 @@ def test_queues_take_no_longer(ren, scene, jobs, lo, hi):
     counter = _time(batch.launch)
     assert all(torch.equal(a, b) for a, b in zip(images, batch.images))
     assert queues < 1.15 * counter, (queues, counter)
+
+
+@pytest.mark.parametrize("jobs", [1, 5, 63])
+def test_reported_size_reaches_the_queues(ren, jobs):
+    """A workspace of rt_render_batch_queue_bytes is handed out from the queues, one byte less is not."""
+    import ctypes
+    from rendertoy_amd import _native as N
+    from rendertoy_amd.batch import BatchRender, RenderRequest
+    lib, rc = N.load(), gpu_from_meshes(_sphere())
+    cam = ren.Camera((0.6, 0.8, 2.2), (0, 0, 0), (0, 1, 0), 0.785, 1.0)
+    batch = BatchRender([RenderRequest(rc, cam, 40, 40)] * jobs)
+    size, cfg = lib.rt_render_batch_queue_bytes(jobs), batch.config.to_c()
+    assert batch.workspace.numel() >= size > lib.rt_render_batch_workspace_bytes(jobs)
+    for given in (size, size - 1):
+        ws = torch.full((size + 256,), 0x5A, dtype=torch.uint8, device="cuda")
+        N.check(lib.rt_render_batch(batch.jobs_dev.data_ptr(), jobs, ctypes.byref(cfg), ws.data_ptr(), given,
+                                    N.stream_handle()), "rt_render_batch")
+        past = ws[lib.rt_render_batch_workspace_bytes(jobs):size]
+        assert bool((past != 0x5A).any()) == (given == size)
+        assert bool((ws[size:] == 0x5A).all())
