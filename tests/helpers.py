@@ -87,3 +87,49 @@ def cull_scenes():
     f[..., 2] = 0.0
     out["flat"] = (soup(f), *aimed(4000, 3.0, 0.9))
     return out
+
+
+def deep_wide_scene():
+    """Meshes whose 4-wide tree is a spine of full nodes, each sibling with 16 inner grandchildren, every box of
+    which holds the unit cube: a ray from inside enters them all and walks that take several entries of their
+    stack a step pile the siblings up. One triangle in the plane x - y = const per Morton code, several per
+    code at the siblings' leaves."""
+    rng = np.random.default_rng(7)
+    codes = []
+    for level in range(15):  # 2 bits of the 30 per 4-wide level; the spine is 11 11 11 ...
+        spine = ((1 << (2 * level)) - 1) << (30 - 2 * level)
+        for sib in range(3):
+            base = spine | sib << (28 - 2 * level)
+            free = 28 - 2 * level  # bits below the sibling's
+            for k in range(16):
+                code = base | (k << (free - 4) if free >= 4 else k >> (4 - free))
+                codes += [code] * 8
+    codes += [(1 << 30) - 1] * 40960  # the spine's end: codes alike, split by slot
+    codes = np.array(sorted(codes), np.int64)
+
+    def compact(c):  # every third bit
+        return sum(((c >> np.int64(3 * b)) & 1) << np.int64(b) for b in range(10))
+    q = np.stack([compact(codes >> 2), compact(codes >> 1), compact(codes)], 1)
+    centre = (q + 0.5) / 1024.0
+    tri = centre[:, None, :] + 4.0 * np.array([[-1, -1, -1], [1, 1, 1], [1, 1, -1]])[None]
+    pos = tri[rng.permutation(len(tri))].reshape(-1, 3).astype(np.float32)
+    idx = np.arange(len(pos), dtype=np.int32).reshape(-1, 3)
+    return [{"pos": pos, "idx": idx, "nrm": None, "uv": None}]
+
+
+def group_walk_peak(nodes4, lanes, words=1024):
+    """(highest number of stack entries, steps of one entry) of a walk of `lanes` lanes per ray that enters every
+    box, by the rules of the device's group_walk."""
+    entries, cap = lanes // 4, words * lanes // 64
+    switch = cap - 3 * entries - 93
+    refs = np.asarray(nodes4, np.float32).reshape(-1, 32)[:, 24:28].copy().view(np.int32)
+    stack, peak, single = [0], 1, 0
+    while stack:
+        k = 1 if len(stack) > switch else min(len(stack), entries)
+        single += len(stack) > switch
+        taken, stack = stack[-k:], stack[:-k]
+        for node in taken:
+            stack += [int(r) for r in refs[node] if 0 <= r < 0x7FFFFFFF]
+        peak = max(peak, len(stack))
+        assert peak <= cap, "a group's stack would run into its neighbour's"
+    return peak, single, switch, cap
