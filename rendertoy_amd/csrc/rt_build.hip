@@ -95,7 +95,6 @@ inline uint64_t align256(uint64_t x) { return (x + 255) & ~uint64_t(255); }
 
 Workspace carve(char* base, uint64_t n) {
     Workspace w{};
-    const uint64_t nblk = (n + kSortTile - 1) / kSortTile;
     const uint64_t ni = n > 1 ? n - 1 : 1;
     uint64_t off = 0;
     auto take = [&](uint64_t bytes) {
@@ -110,7 +109,7 @@ Workspace carve(char* base, uint64_t n) {
     w.vals0 = (uint32_t*)take(4 * n);
     w.keys1 = (uint32_t*)take(4 * n);
     w.vals1 = (uint32_t*)take(4 * n);
-    w.hist = (uint32_t*)take(4 * kRadix * (nblk ? nblk : 1));
+    w.hist = (uint32_t*)take(sort_hist_bytes(n));
     w.totals = (uint32_t*)take(4 * kRadix);
     w.cbounds = (float*)take(4 * 8);
     w.parent = (int32_t*)take(4 * (ni + n));
@@ -453,30 +452,41 @@ struct Fallback {
     RT_DEV bool taken() const { return !deep || *deep; }
 };
 
-// Store of arrays that no kernel of the build reads again (leaf records, 4-wide nodes): past the caches, which
-// then keep what the next kernels read. At 1.31 M triangles the emit went from 72 to 63 us, the 4-wide nodes
-// from 45 to 39 and the next build's gather, which finds the vertices, from 32 to 21.
+// Store of arrays that no kernel of the build reads again (leaf records, 4-wide nodes). PAST: past the caches, which
+// then keep what the next kernels read. That pays where the scene does not fit them: at 1.31 M triangles the emit went
+// from 72 to 63 us, the 4-wide nodes from 45 to 39, a build with its first frame from 466 to 434 (256x144) and from
+// 1,506 to 1,474 (1280x720). A smaller scene's first calls find these arrays in the caches: build and first frame
+// of 256x144 at 450,000 triangles 292 us, past the caches 302, at 251,000 225 and 229, at 648,000 365 and 366.
+constexpr uint32_t kPastCaches = 500000;  // triangles
+
+template <bool PAST>
 RT_DEV void store_last(float4* p, const float4& v) {
     typedef float vec4 __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store((vec4){v.x, v.y, v.z, v.w}, (vec4*)p);
+    const vec4 q = {v.x, v.y, v.z, v.w};
+    if constexpr (PAST)
+        __builtin_nontemporal_store(q, (vec4*)p);
+    else
+        *(vec4*)p = q;
 }
 
 // Copies `per` float4s of each of the block's `rows` records from LDS (record r at
 // stage[r * pitch]) to out[0 .. rows*per), one float4 per thread and instruction.
+template <bool PAST>
 RT_DEV void store_staged(float4* __restrict__ out, const float4* stage, uint32_t rows, uint32_t per,
                          uint32_t pitch) {
     for (uint32_t q = threadIdx.x; q < rows * per; q += blockDim.x) {
         const uint32_t r = q / per;
-        store_last(out + q, stage[r * pitch + (q - r * per)]);
+        store_last<PAST>(out + q, stage[r * pitch + (q - r * per)]);
     }
 }
 
 // One thread per slot: the intersection record (p0, e1, e2, primitive id) and the shading record (three
 // normals, three uvs, mesh id) of its triangle, from the mesh's vertices; the padded leaf box of the slot
 // for an LBVH; the slot of the primitive. The block's records go out through LDS as consecutive
-// float4s. Bound by memory: 180 B of stores per triangle, and the vertices, which neighbours in Morton
+// float4s. Bound by memory: 148 B of stores per triangle, and the vertices, which neighbours in Morton
 // order share in L2. At 1.31 M triangles 63 us and 21 for the gather; records written in
-// primitive order by the gather and permuted here took 81 and 71.
+// primitive order by the gather and permuted here took 71 and 81.
+template <bool PAST>
 __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ slots, Fallback fb, uint32_t n,
                                               const MeshSource* __restrict__ meshes, uint32_t n_sources,
                                               float4* __restrict__ leafbox, float4* __restrict__ tris,
@@ -527,11 +537,11 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ slots
     float4* st = stage + threadIdx.x * kPitch;
     if (mine) { st[0] = shd[0]; st[1] = shd[1]; st[2] = shd[2]; st[3] = shd[3]; }
     __syncthreads();
-    store_staged(shade + 4 * s0, stage, rows, 4, kPitch);
+    store_staged<PAST>(shade + 4 * s0, stage, rows, 4, kPitch);
     __syncthreads();
     if (mine) { st[0] = tri[0]; st[1] = tri[1]; st[2] = tri[2]; }
     __syncthreads();
-    store_staged(tris + 3 * s0, stage, rows, 3, kPitch);
+    store_staged<PAST>(tris + 3 * s0, stage, rows, 3, kPitch);
     if (!taken) return;
     __syncthreads();
     if (mine) store_box(st, box);
@@ -557,8 +567,7 @@ __global__ void __launch_bounds__(256) k_emit(const uint32_t* __restrict__ slots
 // blocks. No node waits on another workgroup.
 //
 // What bounds it: LDS round trips per level of a walk (10 to 17 levels), and 64 B per node of stores
-// in pieces of 16 B; 37 KB of LDS and one slot per thread put two
-// workgroups on a CU.
+// in pieces of 16 B; one slot per thread puts two workgroups on a CU (41 KB of LDS would let in three).
 // At 1.31 M triangles 56 us for the local pass and 25 for the top; separate kernels for the hierarchy
 // (binary searches in memory, 93 us), a refit over its arrays (142), a sparse table of block unions
 // (17) and the top refit (10) took 262. At 11,560 triangles 24 us against 61.
@@ -1513,6 +1522,7 @@ inline int ploc_iterations(uint32_t n) {
 // 144-byte stride keeps the per-lane writes off one bank) and stored as consecutive float4s, so
 // every store instruction writes 4 KB of the output contiguously. (Loading the block's binary
 // records through LDS as well measured slower: they are read once and the child reads hit L2.)
+template <bool PAST>
 __global__ void __launch_bounds__(256) k_wide(uint32_t n, const float4* __restrict__ nodes,
                                               float4* __restrict__ nodes4) {
     constexpr int kPitch = 9;  // float4s per staged record
@@ -1566,7 +1576,7 @@ __global__ void __launch_bounds__(256) k_wide(uint32_t n, const float4* __restri
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const uint32_t q = j * 256 + threadIdx.x;  // float4 q of the block's output
-        if (q < rows * 8) store_last(out + q, stage[(q >> 3) * kPitch + (q & 7)]);
+        if (q < rows * 8) store_last<PAST>(out + q, stage[(q >> 3) * kPitch + (q & 7)]);
     }
 }
 
@@ -1813,7 +1823,8 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
                            w.nright, w.nsize, w.slot_of, w.fslot, nodes);
     }
     // leaf records; the LBVH tree, or the one in place of a PLOC tree found too deep; 4-wide records
-    hipLaunchKernelGGL(k_emit, dim3(blocks_for(n, 256)), dim3(256), 0, s, slots, fb, n, w.meshes, nsrc, w.leafbox,
+    const bool past = n >= kPastCaches;
+    hipLaunchKernelGGL(past ? k_emit<true> : k_emit<false>, dim3(blocks_for(n, 256)), dim3(256), 0, s, slots, fb, n, w.meshes, nsrc, w.leafbox,
                        (float4*)sc->tris, (float4*)sc->shade, (uint32_t*)sc->prim_slot);
     if (ploc && order_out)
         hipLaunchKernelGGL(k_copy_if, dim3(blocks_for(n, 256)), dim3(256), 0, s, w.depth, vi, order_out, n);
@@ -1823,7 +1834,7 @@ extern "C" int rt_scene_build(const rt_mesh_desc* meshes, uint32_t n_meshes, rt_
                            sc->bounds, w.top);
         if (nb > 1)
             hipLaunchKernelGGL(k_tree_top, dim3(nb), dim3(kTopThreads), 0, s, ki, n, fb, nodes, sc->bounds, w.top);
-        hipLaunchKernelGGL(k_wide, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n,
+        hipLaunchKernelGGL(past ? k_wide<true> : k_wide<false>, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n,
                            (const float4*)nodes, (float4*)sc->nodes4);
         sc->root = n <= (uint32_t)kLeafMax ? leaf_ref(0, n) : 0;
     } else {
