@@ -285,15 +285,16 @@ uint32_t group_blocks(int g, uint32_t W, uint32_t H) {
 // The lines below were set over scenes of eight shapes (a smooth sphere, a rough one on a plane, one from near, a
 // terrain, a room from inside, boxes, random triangles, long thin ones) of 1,300 to 1.3 M triangles, since how
 // much longer the slowest walk is than the average one depends on the shape as much as on the triangles.
-double fourth_root(uint32_t n) { return std::sqrt(std::sqrt((double)n)); }
 
-// Lanes per ray where groups walk n rays: 64 for few, 16 for more. Whole waves shorten a ray's chain more the
-// deeper its tree, and cost 3 to 4 times as much per ray: camera time of 16 : 64 lanes over quad-lane packets,
-// geometric mean over the shapes, 0.59 : 0.54 at 4,096 pixels with 1,300 triangles, 0.31 : 0.23 at 8,192 with
-// 80,000, 0.35 : 0.39 at 24,576 with 320,000, 0.32 : 0.34 at 36,864 with 1.3 M (176 : 118 us on the rough sphere).
-int group_lanes(uint64_t n, uint32_t n_tris) {
-    return (double)n <= std::max(4096.0, std::min(n_tris / 6.0, 1200.0 * fourth_root(n_tris))) ? 64 : 16;
-}
+// Lanes per ray where groups walk n rays: 64 for few (up to `some`, at most `most`), 16 for more. Whole waves shorten
+// a ray's chain more the deeper its tree, and cost 3 to 4 times as much per ray: camera time of 16 : 64 lanes over
+// quad-lane packets, geometric mean over the shapes, 0.59 : 0.54 at 4,096 pixels with 1,300 triangles, 0.31 : 0.23 at
+// 8,192 with 80,000, 0.42 : 0.53 at 36,864 with 320,000, 0.32 : 0.34 with 1.3 M. Images change over at a sixth of the
+// triangles (a rough sphere of 650,000 at 256x180 takes 77 us with 64 lanes and 144 with 16, one of 251,000 at 256x144
+// 54 and 72; a room of 250,000 from inside 120 and 47), ray buffers at an eighth and at 40,960 rays (at 65,536 with
+// 1.3 M triangles 16 lanes take 0.76 of the one-lane walks' time on average, 64 1.06; random rays at a rough sphere
+// 390 us and 330).
+int group_lanes(uint64_t n, uint32_t some, uint32_t most) { return n <= std::max(4096u, std::min(some, most)) ? 64 : 16; }
 
 // Lanes per pixel of an image of n pixels: 64 or 16 (group_walk), or 0 for the quad-lane packets.
 // Packets share their node fetches, but a frame takes at least as long as its slowest packet's chain
@@ -313,13 +314,14 @@ int group_lanes(uint64_t n, uint32_t n_tris) {
 //   20 k        0.29  0.51  0.85     0.64  1.02  1.70     0.76  1.38  2.19     1.46  2.05  2.92
 //   320 k       0.15  0.31  0.55     0.27  0.69  1.31     0.37  0.95  1.83     0.76  1.54  2.73     1.43  2.25  3.75
 //   1.3 M       0.13  0.26  0.40     0.22  0.51  1.12     0.22  0.73  1.71     0.43  1.22  2.32     0.83  1.83  3.44
-// so a second line, 12,000 fourth roots of the triangles, ends the groups where hardly a shape gains. Below it a
-// frame can still take up to 2.8 times as long as by packets where all its rays' walks are alike (a sphere from
-// near), against up to 9 times as long by packets where few are long (a wide frame of a small object: 1281x143
-// pixels, 155,000 triangles, 93 us against 410).
+// so a second line, 16,000 fourth roots of the triangles (from 100,000 triangles on it is the lower one), ends the
+// groups where hardly a shape gains (1024x768 of 1.3 M triangles: the rough sphere 558 us by groups, 688 by packets, a
+// sphere from near 1,321 and 389). Below it a frame can still take up to 3 times as long as by packets where
+// all its rays' walks are alike, against up to 4 times as long by packets where few are long (a wide frame of a
+// small object: 1281x143 pixels, 155,000 triangles, 93 us against 410).
 int image_group(uint64_t n, uint32_t n_tris) {
-    if ((double)n > std::min(900.0 * std::sqrt((double)n_tris), 12000.0 * fourth_root(n_tris))) return 0;
-    return group_lanes(n, n_tris);
+    const double root = std::sqrt((double)n_tris);
+    return (double)n <= std::min(900.0 * root, 16000.0 * std::sqrt(root)) ? group_lanes(n, n_tris / 6u, 65536u) : 0;
 }
 
 // Camera closest hit of a small image, G lanes per pixel (image_group).
@@ -1162,7 +1164,7 @@ int query_variant(const rt_tuning& tu, uint32_t n, uint32_t n_tris, bool any) {
 // A caller that bounds the lane stacks, or asks for the binary nodes, gets the walk that has them.
 int query_group(const rt_tuning& tu, uint32_t n, uint32_t n_tris, bool any) {
     if (tu.query != RT_TRAVERSAL_LANE || tu.lane_stack != RT_LANE_STACK_MAX) return 0;
-    return n <= (any && n_tris >= 250000u ? 131072u : 65536u) ? group_lanes(n, n_tris) : 0;
+    return n <= (any && n_tris >= 250000u ? 131072u : 65536u) ? group_lanes(n, n_tris / 8u, 40960u) : 0;
 }
 
 template <bool ANY>

@@ -15,10 +15,10 @@ def _u32(a):
     return np.ascontiguousarray(a).view(np.uint32)
 
 
-# 722 triangles: 64 lanes to 4,096 rays, images to 24,183 pixels; 317,522: 28,485 and 284,858
+# 722 triangles: 64 lanes to 4,096 rays, images to 24,183 pixels; 317,522: 52,920 pixels and 39,690 rays, 379,807
 @pytest.mark.parametrize("freq,images,rays", [
     (6, ((64, 64), (4097, 1), (155, 156), (24184, 1)), (4096, 4097, 65536, 65537)),
-    (126, ((211, 135), (28486, 1), (533, 534), (538, 530)), (28485, 28486, 65536, 65537, 131072, 131073))])
+    (126, ((210, 252), (52921, 1), (612, 620), (613, 620)), (39690, 39691, 65536, 65537, 131072, 131073))])
 def test_same_hits_on_both_sides(ren, freq, images, rays):
     from rendertoy_amd import scenes
     meshes = [scenes.icosphere(freq, 17), scenes.ground_plane()]
@@ -77,7 +77,7 @@ def near_view(ren):
     return out
 
 
-@pytest.mark.parametrize("w,h", [(600, 500), (768, 512)])
+@pytest.mark.parametrize("w,h", [(640, 620), (768, 512)])
 def test_time_of_images(ren, near_view, w, h):
     cam = ren.Camera((0.1, 0.2, 0.8), (0, 0, 0), (0, 1, 0), math.pi / 4, w / h)
     for rc in near_view:
