@@ -146,8 +146,10 @@ typedef struct rt_render_out {
     uint32_t* stats;
 } rt_render_out;
 
-/* Traversal algorithms of the camera and render kernels. Both return the same hits (the closest
- * hit does not depend on the visiting order); they differ in speed only. */
+/* Traversal algorithms. All return the same hits (the closest hit does not depend on the visiting
+ * order: boxes are skipped only where they are entered 2^-18 of the best hit's distance past it); they differ
+ * in speed only. QUAD and LANE name the walks of calls that fill the device: calls of few rays are walked by
+ * groups of 16 or 64 lanes per ray instead (see rt_tuning). */
 enum {
     RT_TRAVERSAL_PACKET = 0, /* a wave's 64 rays walk one node sequence (scalar node fetches) */
     RT_TRAVERSAL_LANE = 1,   /* each lane walks its own ray (per-lane stack in LDS) */
@@ -160,7 +162,7 @@ enum {
                                 lane testing one child box / one leaf triangle (the default) */
     RT_TRAVERSAL_BINARY = 5  /* ray buffers (rt_trace_closest / rt_trace_any): each lane walks its
                                 own ray over the binary nodes, nearer child first, per-lane stack in
-                                LDS (the default for ray buffers) */
+                                LDS (the default for ray buffers is LANE) */
 };
 #define RT_LANE_STACK_MAX 32
 
@@ -169,20 +171,26 @@ enum {
  * a `const rt_tuning*`: the caller's choices for that call, or NULL for the process default set by
  * rt_set_tuning (so two callers on two streams never share mutable state). */
 typedef struct rt_tuning {
-    int32_t primary;          /* RT_TRAVERSAL_* for camera rays (default QUAD) */
+    int32_t primary;          /* RT_TRAVERSAL_* for camera rays (default QUAD). With QUAD, images of few
+                                 pixels (up to min(900 n^(1/2), 16000 n^(1/4)) for n triangles) and path
+                                 frames of few samples are walked by 16 or 64 lanes per ray */
     int32_t shadow;           /* RT_TRAVERSAL_* for rt_render's shadow rays (default LANE; not used
                                  with a QUAD primary); not QUAD, which is for camera rays */
     uint32_t super_tile;      /* blocks are mapped to XCDs in super-tiles of this many 16x16-pixel
-                                 blocks per side; 0 = row-major block order (default) */
+                                 blocks per side; 0 = row-major block order (default). Not 0:
+                                 rt_trace_camera with QUAD keeps to packets at every size */
     uint32_t lane_stack;      /* per-lane stack entries, 1..RT_LANE_STACK_MAX (default 32); a ray
-                                 needing more is traced again by its wave with the packet traversal */
+                                 needing more is traced again by its wave with the packet traversal.
+                                 Less than the default: ray buffers with LANE, and rt_trace_paths'
+                                 bounces, are walked by one lane per ray at every size */
     uint32_t packet_budget;   /* RT_TRAVERSAL_HYBRID: packet steps before the per-lane walk (256) */
     uint32_t builder;         /* RT_BUILD_* hierarchy of rt_scene_build (default LBVH) */
     int32_t query;            /* RT_TRAVERSAL_LANE (per-lane walk of the 4-wide nodes, default) or
                                  RT_TRAVERSAL_BINARY (of the binary nodes) for rt_trace_closest /
                                  rt_trace_any; both keep their stacks in LDS (lane_stack entries per
                                  lane) and trace a ray that needs more again with the packet
-                                 traversal */
+                                 traversal. With LANE, calls of up to 65,536 rays (any hits in scenes of
+                                 250,000 triangles: 131,072) are walked by 16 or 64 lanes per ray */
     uint32_t handoff_steps;   /* must be 0: reserved for a hand-off of the slowest camera packets' walks
                                  to other waves, which is switched off (its first runs did not finish) */
     uint32_t item_steps;      /* reserved with handoff_steps: 1..2^20, default 32 */
@@ -190,11 +198,12 @@ typedef struct rt_tuning {
 
 /* Hierarchy builders of rt_scene_build; both start from the same Morton order and give the same
  * hits. The PLOC tree (locally ordered clustering by surface area) needs ~30% fewer traversal
- * steps per packet and ~17% fewer instructions than the LBVH radix tree, and takes ~3.7x longer
- * to build; frames whose time is set by their slowest tiles gain little from it. A PLOC tree with
+ * steps per packet and ~17% fewer instructions than the LBVH radix tree, and takes 4 to 6 times as
+ * long to build; frames whose time is set by their slowest tiles gain little from it. A PLOC tree with
  * a triangle more than 62 internal levels deep (the depth the traversal stacks are sized for, and
- * the bound of the radix tree) is replaced by the LBVH; checking this makes a PLOC build wait for
- * its stream once. */
+ * the bound of the radix tree) is replaced by the LBVH; the device decides this, so a PLOC build, like an
+ * LBVH one, is kernels on its stream and does not wait for it. Of triangles whose boxes are alike
+ * an iteration merges one pair, so a PLOC build of n of them takes n iterations. */
 enum {
     RT_BUILD_LBVH = 0, /* Karras radix tree over the Morton order, leaves of <= 4 consecutive slots */
     RT_BUILD_PLOC = 1  /* PLOC (Meister & Bittner 2018), search radius 16, leaves of <= 4 triangles */
@@ -272,8 +281,8 @@ int rt_trace_camera(const rt_scene* scene, const rt_camera* cam, uint32_t width,
  * counts there; NULL (or fewer bytes) is accepted, the counts are then summed per 4-wave workgroup
  * (slower). Two calls in flight must not share a workspace. With the QUAD camera-ray traversal (the default) the
  * primary and the shadow rays both take the quad-lane traversal (16-ray packets over 4x4 pixels, 4
- * lanes per ray) and `tuning->shadow` is not used; with the others the primary rays take the
- * chosen traversal and the shadow rays `tuning->shadow`. */
+ * lanes per ray; for few pixels 16 or 64 lanes per ray, as rt_tuning.primary says) and `tuning->shadow` is not
+ * used; with the others the primary rays take the chosen traversal and the shadow rays `tuning->shadow`. */
 uint64_t rt_render_workspace_bytes(uint32_t n_pixels);
 int rt_render(const rt_scene* scene, const rt_camera* cam, const rt_render_params* params,
               const rt_render_out* out, void* workspace_dev, uint64_t workspace_bytes,
@@ -329,7 +338,8 @@ const uint32_t* rt_render_batch_status(const void* workspace_dev);
  * reference; for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc). The batch workspace is a file-scope device array
  * of the library sized for RT_BATCH_MAX_JOBS jobs (16,644 bytes, one copy per device, held until
- * the process ends); more jobs return RT_ECAPACITY. Output is bit-identical to rt_render_batch.
+ * the process ends; it has no room for the tile queues, so tiles come from one counter); more jobs return
+ * RT_ECAPACITY. Output is bit-identical to rt_render_batch.
  * Every call on one device shares that array: calls whose launches overlap on one device (e.g. on
  * two streams) race; issue them on one stream or wait between them. The status word is not
  * readable (a skipped job leaves its outputs unwritten). */

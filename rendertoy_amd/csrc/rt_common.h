@@ -130,13 +130,14 @@ RT_DEV void refine_hit(const float4* __restrict__ tris, const Ray& r, Hit& h) {
 // smaller primitive id). Every record of the leaf is fetched before the first test, so a leaf costs
 // one memory round trip instead of one per triangle. `active` = this lane takes part; `skip_slot` =
 // a slot never reported (a shadow ray's own triangle). Returns whether h changed.
-// MASK: slots past the leaf's count are not fetched; else they re-read its first record. A load
-// costs the CU's address and tag units one access per lane that takes part, wherever it points, and
-// in the ray-buffer walks those units are the busiest (74% of a 2 M segment query's cycles, against
-// 56% for the vector ALUs): leaves hold 2.9 triangles on average, so a third of the accesses of a
-// full fetch are for nothing. Masked, 2 M segments through 251 k triangles take 1.05 ms instead of
-// 1.18, 1.5 M random rays through 1.3 M 2.49 instead of 2.59, a 3-sphere path frame 3.90 instead of
-// 4.03. The batch refill kernel, bound by its slowest walks, loses 3% to the extra branches.
+// MASK: slots past the leaf's count are not fetched; else they re-read its first record. Leaves hold 2.9
+// triangles on average, so a third of the accesses of a full fetch are for nothing. Masked, 2 M segments through
+// 251 k triangles take 1.05 ms instead of 1.18, 1.5 M random rays through 1.3 M 2.49 instead of 2.59, a 3-sphere
+// path frame 3.90 instead of 4.03. (A load costs the CU's address and tag units one access per lane that takes
+// part, and in the ray-buffer walks they are the busiest units, 74% of a 2 M segment query's cycles against 56%
+// for the vector ALUs. But node records of half the loads gained nothing, so it is where leaves come from
+// memory, and not by the count of accesses alone, that the masks pay: query_variant's table.) The batch refill
+// kernel, bound by its slowest walks, loses 3% to the extra branches.
 template <bool MASK = false>
 RT_DEV bool test_leaf(const float4* __restrict__ tris, int32_t ref, const Ray& r, bool active,
                       int32_t skip_slot, Hit& h) {
