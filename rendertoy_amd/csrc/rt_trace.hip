@@ -615,19 +615,20 @@ RT_DEV uint32_t job_tiles(const rt_render_job& j, uint32_t unit, uint32_t& statu
 
 // The tile queue of k_render_batch_refill in the workspace bytes past the prefix, where the caller
 // gives them: kQueues counters, each on a 256-byte line of its own, then the order of the jobs.
-// The x-th grab of queue q is grab x kQueues + (q + 8 x) mod kQueues of the launch: without the turn a queue
-// would keep to the same columns of an image whose rows are a multiple of kQueues grabs (8 images of 1024x1024
-// pixels, 1,300 triangles, 1.14 ms instead of 0.92); turned by 8 it stays on its XCD's stripes. One counter for
+// The x-th grab of queue q is grab x kQueues + (q + turn x) mod kQueues of the launch. Without a turn a queue keeps to
+// the same columns of an image whose rows are a multiple of kQueues grabs (8 images of 1024x1024 pixels, 1,300
+// triangles, 1.14 ms instead of 0.92 with a turn of 8, which stays on an XCD's stripes); where no image's row is a
+// multiple of 32 tiles there is none, which other rows are 1 to 4% faster with. One counter for
 // all waves is the kernel's bound once most tiles miss everything: it is read and written about 70 times a microsecond at
 // most, and 48 images of 128..768 pixels a side are 30,000 grabs of 4 tiles.
 constexpr uint32_t kQueues = 64, kQueueStride = 64;  // words
 
 struct BatchQueue {
-    uint32_t* counters;  // NULL: the one counter ws[0], jobs in table order
+    uint32_t* counters;  // NULL: the one counter ws[0], jobs in table order; counters[1]: the turn
     uint32_t* order;     // job of the p-th prefix entry
 };
 
-RT_DEV uint32_t queue_grab(uint32_t x, uint32_t q) { return x * kQueues + (q + 8u * x) % kQueues; }
+RT_DEV uint32_t queue_grab(uint32_t x, uint32_t q, uint32_t turn) { return x * kQueues + (q + turn * x) % kQueues; }
 
 // Tiles per grab. A grab is the launch's unit of work at its end: a wave can hold one of its densest tiles (256
 // pixels of 4 tiles take up to 1.5 ms), so a wave should have 16 grabs, or 6 where each is one tile. But a wave
@@ -654,10 +655,10 @@ __global__ void __launch_bounds__(1024) k_batch_prepare(const rt_render_job* __r
                                                          uint32_t n_jobs, uint32_t unit,
                                                          uint32_t* __restrict__ ws, BatchQueue q) {
     __shared__ uint32_t part[1024];
-    __shared__ uint32_t status;
+    __shared__ uint32_t status, rows;
     __shared__ uint64_t keys[RT_BATCH_MAX_JOBS];
     const uint32_t t = threadIdx.x;
-    if (t == 0) status = 0;
+    if (t == 0) status = rows = 0;
     if (q.counters) {
         uint32_t m = 1;
         while (m < n_jobs) m <<= 1;
@@ -689,6 +690,7 @@ __global__ void __launch_bounds__(1024) k_batch_prepare(const rt_render_job* __r
             const uint32_t j = q.counters ? (uint32_t)keys[p] : p;
             if (q.counters) q.order[p] = j;
             cnt[k] = job_tiles(jobs[j], unit, bad);
+            if (cnt[k] && (jobs[j].params.width + unit - 1u) / unit % 32u == 0) rows = 1;
             uint32_t* st = as_global(jobs[j].out.stats);
             if (st) {
                 st[0] = 0;
@@ -722,6 +724,7 @@ __global__ void __launch_bounds__(1024) k_batch_prepare(const rt_render_job* __r
     if (t == 0) {
         ws[0] = 0;
         ws[1] = status;
+        if (q.counters) q.counters[1] = rows ? 8u : 0u;
     }
 }
 
@@ -842,7 +845,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
     for (uint32_t j = lane; j <= n_jobs; j += 64) pref[j] = ws[kBatchPrefixWord + j];
     __syncthreads();
     const uint32_t total = pref[n_jobs];
-    if (queue.counters) grab = tiles_per_grab(grab, total, n_jobs, gridDim.x);
+    uint32_t turn = 0;
+    if (queue.counters) {
+        grab = tiles_per_grab(grab, total, n_jobs, gridDim.x);
+        turn = queue.counters[1];
+    }
 
     // wave-uniform: the tile being handed out, its next pixel, the end of the grabbed tiles, and
     // the job the lanes work on (with its scene, camera, parameters and counts)
@@ -901,11 +908,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
                         // is not (the counters only grow, so every wave finds all of them empty)
                         for (;;) {
                             if (lane == 0) u0 = atomicAdd(&queue.counters[q * kQueueStride], 1u);
-                            u0 = queue_grab((uint32_t)__builtin_amdgcn_readfirstlane((int)u0), q) * grab;
+                            u0 = queue_grab((uint32_t)__builtin_amdgcn_readfirstlane((int)u0), q, turn) * grab;
                             if (u0 < total) break;
                             const uint32_t at = __hip_atomic_load(&queue.counters[lane * kQueueStride],
                                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            const uint64_t open = __ballot(queue_grab(at, lane) * grab < total);
+                            const uint64_t open = __ballot(queue_grab(at, lane, turn) * grab < total);
                             if (open == 0) break;
                             const uint64_t after = open & ~((2ull << q) - 1ull);
                             q = (uint32_t)__ffsll((unsigned long long)(after ? after : open)) - 1u;
